@@ -398,27 +398,65 @@ __device__ __forceinline__ float tex_weight(float c, int *i0) {
 }
 
 // check_point_d (tracking_helpers.cu:63-73): linear filter of the stop map,
-// border colour -1, texture x = array z (cu_tractography.py:237-241).
-__device__ int check_point(const DevParams &P, const float *__restrict__ stop, float px, float py,
-                           float pz) {
+// border colour -1, texture x = array z (cu_tractography.py:237-241).  In two
+// halves, so that a caller can put other loads between the 8 texel reads and
+// their use; texels outside the map read a clamped one and are replaced.
+struct StopTap {
+    float a, b, g;
+    float t[8];
+    uint32_t in;  // bit k: texel k lies in the map
+};
+
+__device__ __forceinline__ StopTap stop_begin(const DevParams &P, const float *__restrict__ stop, float px, float py,
+                                              float pz) {
+    StopTap s;
     int iz, iy, ix;
-    const float a = tex_weight(pz, &iz), b = tex_weight(py, &iy), g = tex_weight(px, &ix);
-    const float a0 = 1.0f - a, b0 = 1.0f - b, g0 = 1.0f - g;
+    s.a = tex_weight(pz, &iz);
+    s.b = tex_weight(py, &iy);
+    s.g = tex_weight(px, &ix);
     const int DX = P.dimx, DY = P.dimy, DZ = P.dimz;
-    auto fetch = [&](int z, int y, int x) -> float {
-        if (z < 0 || z >= DZ || y < 0 || y >= DY || x < 0 || x >= DX) return -1.0f;
-        return stop[((size_t)x * DY + y) * DZ + z];
-    };
-    float acc = ((a0 * b0) * g0) * fetch(iz, iy, ix);
-    acc = __builtin_fmaf((a * b0) * g0, fetch(iz + 1, iy, ix), acc);
-    acc = __builtin_fmaf((a0 * b) * g0, fetch(iz, iy + 1, ix), acc);
-    acc = __builtin_fmaf((a * b) * g0, fetch(iz + 1, iy + 1, ix), acc);
-    acc = __builtin_fmaf((a0 * b0) * g, fetch(iz, iy, ix + 1), acc);
-    acc = __builtin_fmaf((a * b0) * g, fetch(iz + 1, iy, ix + 1), acc);
-    acc = __builtin_fmaf((a0 * b) * g, fetch(iz, iy + 1, ix + 1), acc);
-    acc = __builtin_fmaf((a * b) * g, fetch(iz + 1, iy + 1, ix + 1), acc);
+    uint32_t xo[2], yo[2], zo[2];
+    bool xi[2], yi[2], zi[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        // k + clamp(i) would overflow for a position far outside, so the
+        // second texel is clamped from the first's range
+        xi[k] = ix >= -k && ix < DX - k;
+        yi[k] = iy >= -k && iy < DY - k;
+        zi[k] = iz >= -k && iz < DZ - k;
+        xo[k] = (uint32_t)min(max(ix, -k), DX - 1 - k) + k;
+        yo[k] = (uint32_t)min(max(iy, -k), DY - 1 - k) + k;
+        zo[k] = (uint32_t)min(max(iz, -k), DZ - 1 - k) + k;
+    }
+    s.in = 0u;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int kz = k & 1, ky = (k >> 1) & 1, kx = k >> 2;
+        s.t[k] = stop[(size_t)((xo[kx] * (uint32_t)DY + yo[ky]) * (uint32_t)DZ + zo[kz])];
+        if (xi[kx] && yi[ky] && zi[kz]) s.in |= 1u << k;
+    }
+    return s;
+}
+
+__device__ __forceinline__ int stop_end(const DevParams &P, const StopTap &s) {
+    const float a = s.a, b = s.b, g = s.g;
+    const float a0 = 1.0f - a, b0 = 1.0f - b, g0 = 1.0f - g;
+    auto t = [&](int k) { return ((s.in >> k) & 1u) ? s.t[k] : -1.0f; };
+    float acc = ((a0 * b0) * g0) * t(0);
+    acc = __builtin_fmaf((a * b0) * g0, t(1), acc);
+    acc = __builtin_fmaf((a0 * b) * g0, t(2), acc);
+    acc = __builtin_fmaf((a * b) * g0, t(3), acc);
+    acc = __builtin_fmaf((a0 * b0) * g, t(4), acc);
+    acc = __builtin_fmaf((a * b0) * g, t(5), acc);
+    acc = __builtin_fmaf((a0 * b) * g, t(6), acc);
+    acc = __builtin_fmaf((a * b) * g, t(7), acc);
     if (acc == -1.0f) return CUSLINES_OUTSIDEIMAGE;
     return (acc > P.tc_threshold) ? CUSLINES_TRACKPOINT : CUSLINES_ENDPOINT;
+}
+
+__device__ __forceinline__ int check_point(const DevParams &P, const float *__restrict__ stop, float px, float py,
+                                           float pz) {
+    return stop_end(P, stop_begin(P, stop, px, py, pz));
 }
 
 // Texel index I of one axis of the vertex-tiled PTT texture -> (tile, local),
@@ -691,40 +729,31 @@ struct ProbLds {
     uint16_t *cand;
 };
 
-template <bool IS_START>
-__device__ int get_direction_prob(const DevParams &P, const DevBufs &B, const float *sv, ProbLds &S,
-                                  Philox &rng, float dx, float dy, float dz, float px, float py,
-                                  float pz, float *ndx, float *ndy, float *ndz) {
+// Threshold, cone test and running sum of the interpolated pmf (LDS, nverts
+// values); returns its last element.
+__device__ float prob_sum(int nv, int symm, float cos_max_angle, const float *sv, float *pmf, float dx, float dy,
+                          float dz) {
     const int l = lane32();
-    const int nv = P.nverts;
-    float *pmf = S.pmf;
-    if (trilinear<3>(P, B.data, P.t32, P.dimt, px, py, pz, pmf) != 0) return 0;
-    WAVE_SYNC();
     float mx = REAL_MIN;
     for (int i = l; i < nv; i += 32) mx = (mx > pmf[i]) ? mx : pmf[i];
     mx = max32(mx);
     const float thr = (float)(PMF_THRESHOLD_P * (double)mx);
-    if (IS_START) {
-        for (int i = l; i < nv; i += 32)
-            if (pmf[i] < thr) pmf[i] = 0.0f;
-        WAVE_SYNC();
-        return peak_directions(P, B, pmf, S.marks, S.cand, sv);
-    }
     for (int i = l; i < nv; i += 32) {
         float v = pmf[i];
         if (v < thr) v = 0.0f;
         float d = dot3(dx, dy, dz, sv[3 * i], sv[3 * i + 1], sv[3 * i + 2]);
-        if (P.sphere_symm) d = fabsf(d);
-        if (d < P.cos_max_angle) v = 0.0f;
+        if (symm) d = fabsf(d);
+        if (d < cos_max_angle) v = 0.0f;
         pmf[i] = v;
     }
     WAVE_SYNC();
     prefix_sum(pmf, nv);
-    const float last = pmf[nv - 1];
-    if (last == 0.0f) return 0;
-    float sel = 0.0f;
-    if (l == 0) sel = rng.uniform() * last;
-    sel = shfl32(sel, 0);
+    return pmf[nv - 1];
+}
+
+// Index of the direction that `sel` falls on in the running sum `pmf`.
+__device__ int prob_pick(const float *pmf, int nv, float sel) {
+    const int l = lane32();
     int low = 0, high = nv - 1;
     while ((high - low) >= 32) {
         const int mid = (low + high) / 2;
@@ -734,12 +763,84 @@ __device__ int get_direction_prob(const DevParams &P, const DevBufs &B, const fl
     const uint32_t msk = half_ballot(pr);
     int ind = low + __ffs(msk) - 1;
     if (ind < 0) ind = 0;
-    const float vx = sv[3 * ind], vy = sv[3 * ind + 1], vz = sv[3 * ind + 2];
-    if (dot3(dx, dy, dz, vx, vy, vz) > 0.0f) { *ndx = vx; *ndy = vy; *ndz = vz; }
-    else { *ndx = -vx; *ndy = -vy; *ndz = -vz; }
-    WAVE_SYNC();
-    return 1;
+    return ind;
 }
+
+// The getter draws one uniform a step from lane 0's stream.  The slot's
+// lanes (32 or 64) hold consecutive blocks of it, 4 draws each, so a Philox
+// evaluation serves 128 or 256 steps.
+template <int LANES>
+struct ProbStream {
+    uint32_t k0, k1, s0, s1;
+    uint32_t r0, r1, r2, r3;
+    uint32_t k;  // draws taken
+
+    __device__ __forceinline__ void refill() {
+        Philox p;
+        p.k0 = k0; p.k1 = k1; p.s0 = s0; p.s1 = s1;
+        p.c0 = (k >> 2) + (threadIdx.x & (LANES - 1));
+        p.c1 = 0u;
+        p.refill();
+        r0 = p.r0; r1 = p.r1; r2 = p.r2; r3 = p.r3;
+    }
+    __device__ __forceinline__ void init(uint64_t seed, uint64_t sub) {
+        k0 = (uint32_t)seed; k1 = (uint32_t)(seed >> 32);
+        s0 = (uint32_t)sub; s1 = (uint32_t)(sub >> 32);
+        k = 0u;
+        refill();
+    }
+    // the next draw's uniform; take() moves past it
+    __device__ __forceinline__ float peek() const {
+        const uint32_t a = (k & 1u) ? r1 : r0, b = (k & 1u) ? r3 : r2;
+        const int w = (int)((k & 2u) ? b : a), from = (int)((k >> 2) & (LANES - 1));
+        const uint32_t x =
+            (uint32_t)((LANES == 64) ? __builtin_amdgcn_readlane(w, __builtin_amdgcn_readfirstlane(from)) : shfl32(w, from));
+        return 2.32830644e-10f + (float)x * 2.32830644e-10f;
+    }
+    __device__ __forceinline__ void take() {
+        if ((++k & (4u * LANES - 1u)) == 0u) refill();
+    }
+};
+
+template <bool IS_START>
+__device__ int get_direction_prob(const DevParams &P, const DevBufs &B, const float *sv, ProbLds &S,
+                                  ProbStream<32> &rng, float dx, float dy, float dz, float px, float py,
+                                  float pz, float *ndx, float *ndy, float *ndz) {
+    float *pmf = S.pmf;
+    if (trilinear<3>(P, B.data, P.t32, P.dimt, px, py, pz, pmf) != 0) return 0;
+    WAVE_SYNC();
+    const int l = lane32();
+    const int nv = P.nverts;
+    if (!IS_START) {
+        const float last = prob_sum(nv, P.sphere_symm, P.cos_max_angle, sv, pmf, dx, dy, dz);
+        if (last == 0.0f) return 0;
+        const int ind = prob_pick(pmf, nv, rng.peek() * last);
+        rng.take();
+        const float vx = sv[3 * ind], vy = sv[3 * ind + 1], vz = sv[3 * ind + 2];
+        if (dot3(dx, dy, dz, vx, vy, vz) > 0.0f) { *ndx = vx; *ndy = vy; *ndz = vz; }
+        else { *ndx = -vx; *ndy = -vy; *ndz = -vz; }
+        WAVE_SYNC();
+        return 1;
+    }
+    float mx = REAL_MIN;
+    for (int i = l; i < nv; i += 32) mx = (mx > pmf[i]) ? mx : pmf[i];
+    mx = max32(mx);
+    const float thr = (float)(PMF_THRESHOLD_P * (double)mx);
+    for (int i = l; i < nv; i += 32)
+        if (pmf[i] < thr) pmf[i] = 0.0f;
+    WAVE_SYNC();
+    return peak_directions(P, B, pmf, S.marks, S.cand, sv);
+}
+
+// The random streams of a slot: the probabilistic getter's one, the others' 32.
+template <int MODEL>
+struct SlotRng {
+    typedef Philox type;
+};
+template <>
+struct SlotRng<CUSLINES_PROB> {
+    typedef ProbStream<32> type;
+};
 
 // -------------------------------------------------------------------------
 // Bootstrap getter (boot.cu:19-113, 115-193, 330-608)
@@ -1517,8 +1618,8 @@ struct SlotLds {
 // training pairs (tag identifies seed, direction and pass for the hash), 3
 // plain getter counting its taps and sub-steps into *ntap and *nsub.
 template <int MODEL, int V = 0>
-__device__ int tracker(const DevParams &P, const DevBufs &B, const float *sv, SlotLds &S, Philox &rng,
-                       float sx, float sy, float sz, float dx, float dy, float dz, float *frame,
+__device__ int tracker(const DevParams &P, const DevBufs &B, const float *sv, SlotLds &S,
+                       typename SlotRng<MODEL>::type &rng, float sx, float sy, float sz, float dx, float dy, float dz, float *frame,
                        float *__restrict__ sl, uint32_t tag = 0, uint32_t *ntap = nullptr,
                        uint32_t *nsub = nullptr) {
     const int l = lane32();
@@ -1534,9 +1635,9 @@ __device__ int tracker(const DevParams &P, const DevBufs &B, const float *sv, Sl
     for (i = 1; i < MAXL * step_frac; ++i) {
         float nx = 0.0f, ny = 0.0f, nz = 0.0f;
         int ndir;
-        if (MODEL == CUSLINES_PROB)
+        if constexpr (MODEL == CUSLINES_PROB)
             ndir = get_direction_prob<false>(P, B, sv, S.prob, rng, dx, dy, dz, px, py, pz, &nx, &ny, &nz);
-        else if (MODEL == CUSLINES_PTT && V == 1) {
+        else if constexpr (MODEL == CUSLINES_PTT && V == 1) {
             int fell = 0;
             ndir = get_direction_ptt_learned(P, B, S.ptt, frame, rng, learned, dx, dy, dz, px, py, pz, &nx, &ny, &nz,
                                              &fell, &lmiss);
@@ -1547,7 +1648,7 @@ __device__ int tracker(const DevParams &P, const DevBufs &B, const float *sv, Sl
             } else {
                 ++nplain;
             }
-        } else if (MODEL == CUSLINES_PTT && V == 2) {
+        } else if constexpr (MODEL == CUSLINES_PTT && V == 2) {
             float fr0[9];
 #pragma unroll
             for (int q = 0; q < 9; ++q) fr0[q] = frame[q];
@@ -1555,11 +1656,11 @@ __device__ int tracker(const DevParams &P, const DevBufs &B, const float *sv, Sl
             ndir = get_direction_ptt<false>(P, B, S.ptt, frame, rng, dx, dy, dz, px, py, pz, &nx, &ny, &nz, nullptr,
                                             rec ? S.ptt.act + ACT_O : nullptr);
             if (rec) record_pair(P, B, S.ptt, px, py, pz, dx, dy, dz, fr0, S.ptt.act + ACT_O);
-        } else if (MODEL == CUSLINES_PTT && V == 3) {
+        } else if constexpr (MODEL == CUSLINES_PTT && V == 3) {
             ++*nsub;
             ndir = get_direction_ptt<false, true>(P, B, S.ptt, frame, rng, dx, dy, dz, px, py, pz, &nx, &ny, &nz,
                                                   nullptr, nullptr, ntap);
-        } else if (MODEL == CUSLINES_PTT)
+        } else if constexpr (MODEL == CUSLINES_PTT)
             ndir = get_direction_ptt<false>(P, B, S.ptt, frame, rng, dx, dy, dz, px, py, pz, &nx, &ny, &nz);
         else
             ndir = get_direction_boot<MODEL>(P, B, sv, S.boot, rng, 5, dx, dy, dz, px, py, pz, &nx, &ny, &nz);
@@ -2362,15 +2463,16 @@ __global__ void __launch_bounds__(256) phase1_kernel(DevParams P, DevBufs B, con
     SlotLds S;
     bind_slot<MODEL>(P, true, base, S);
     const float px = seeds[3 * s], py = seeds[3 * s + 1], pz = seeds[3 * s + 2];
-    Philox rng;
-    rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo, (uint64_t)32 * (uint64_t)(s % rng_chunk) + l);
+    typename SlotRng<MODEL>::type rng;  // the bootstrap getter draws from it
+    if (MODEL == CUSLINES_OPDT || MODEL == CUSLINES_CSA)
+        rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo, (uint64_t)32 * (uint64_t)(s % rng_chunk) + l);
     int n;
     const uint16_t *kept;
-    if (MODEL == CUSLINES_PROB) {
+    if constexpr (MODEL == CUSLINES_PROB) {
         float a, b, c;
         n = get_direction_prob<true>(P, B, sv, S.prob, rng, 0.0f, 0.0f, 0.0f, px, py, pz, &a, &b, &c);
         kept = S.prob.cand;
-    } else if (MODEL == CUSLINES_PTT) {
+    } else if constexpr (MODEL == CUSLINES_PTT) {
         float *pmf = S.prob.pmf;
         for (int i = l; i < P.nverts; i += 32) {
             const int tx = i & (P.nx - 1), ty = (i >> P.log2x) & (P.ny - 1), tz = i >> (P.log2x + P.log2y);
@@ -2400,8 +2502,9 @@ __device__ void track_seed(const DevParams &P, const DevBufs &B, const float *sv
                            float *__restrict__ sline) {
     const int l = lane32();
     const float sx = seeds[3 * s], sy = seeds[3 * s + 1], sz = seeds[3 * s + 2];
-    Philox rng;
-    rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo, (uint64_t)32 * (uint64_t)(s % rng_chunk) + l + 1);
+    typename SlotRng<MODEL>::type rng;
+    rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo,
+             (uint64_t)32 * (uint64_t)(s % rng_chunk) + (MODEL == CUSLINES_PROB ? 0 : l) + 1);
     const int ndir = (P.slot_cap > 0 && offsets[s + 1] > P.slot_cap) ? 0 : offsets[s + 1] - offsets[s];
     int off = offsets[s];
     const size_t slot_f = (size_t)2 * P.max_sline_len * 3;
@@ -2411,7 +2514,7 @@ __device__ void track_seed(const DevParams &P, const DevBufs &B, const float *sv
         const float fx = B.verts[3 * vi], fy = B.verts[3 * vi + 1], fz = B.verts[3 * vi + 2];
         float *cur = sline + (size_t)off * slot_f;
         if (l == 0) sline_seed[off] = s;
-        if (MODEL == CUSLINES_PTT) {
+        if constexpr (MODEL == CUSLINES_PTT) {
             if (!init_frame_ptt<V == 3>(P, B, S.ptt, rng, fx, fy, fz, sx, sy, sz, &ntap)) {
                 if (l == 0) {
                     sline_len[off] = 1;
@@ -2499,7 +2602,7 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
     float *sf = st + 8;                     // seed point [0..2], direction [3..5]
     if (l == 0) { si[1] = 0; si[2] = 0; }
     WAVE_SYNC();
-    Philox rng;
+    typename SlotRng<MODEL>::type rng;
     int qk = 0;
     bool have = false;
     int pass = 0, i = 1, ri = 1, qi = 0;  // step i = qi * step_frac + ri
@@ -2525,7 +2628,8 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
                     if (lo + q >= hi) { ++qk; continue; }
                     const int s = order ? order[lo + q] : lo + q;
                     const int nd = (P.slot_cap > 0 && offsets[s + 1] > P.slot_cap) ? 0 : offsets[s + 1] - offsets[s];
-                    rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo, (uint64_t)32 * (uint64_t)(s % rng_chunk) + l + 1);
+                    rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo,
+                             (uint64_t)32 * (uint64_t)(s % rng_chunk) + (MODEL == CUSLINES_PROB ? 0 : l) + 1);
                     WAVE_SYNC();
                     if (l == 0) {
                         si[0] = s; si[1] = nd; si[2] = 0; si[3] = offsets[s];
@@ -2655,6 +2759,528 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
             have = false;
         }
     }
+}
+
+// -------------------------------------------------------------------------
+// Probabilistic phase 2 with the pmf and the cell in registers (rows of up to
+// 768 channels), one seed per wavefront.
+//
+// The step of flat_slot<PROB> reads 8 corners x 724 channels (23 KB) through
+// L2 whether or not the seed left its cell, and is a chain of short dependent
+// pieces: 8 rounds of loads, 23 blocks of 5 lane shuffles that each wait for
+// the block before (the running sum's carry), a 5-level binary search through
+// LDS, 8 branchy stop-map reads.  A lone slot took 14 us a step, and 25,000
+// seeds, which share few cells, ran at the rate of the fabric.  Here
+//  - a lane owns channels 256 c + 4 l .. + 3, and the cell's 8 corners stay
+//    in its registers: a step of 1/4 voxel leaves the cell about every third
+//    time, usually by one face, and then reads 4 corners (about 1/5 of the
+//    bytes; nothing is kept beyond the wave's own last cell);
+//  - the threshold, the cone test and the running sum work on registers;
+//  - the stop map of the point just stored is read with the next step;
+//  - the position, the cell, the search and every branch are the wave's, so
+//    addresses and control flow are scalar.
+//
+// The running sum keeps the additions of prefix_sum (utils.cu:81-120) and
+// their order.  In its Hillis-Steele block only values that include element 0
+// see the carry: with m the highest power of two <= e,
+//     out[e] = W[e] + out[e - m],  out[0] = x[0] + carry,
+// W[e] the sum of the m elements ending at e as the first log2(m) rounds form
+// it.  So W needs no carry (4 rounds of in-lane adds and row-shift DPP, all
+// blocks at once); the block carries are a chain of 6 adds per block over
+// W[0], W[1], W[3], W[7], W[15], W[31], one block per lane; and out is only
+// formed where it is read: the 31 midpoints that the 5 levels of the binary
+// search can visit (one per lane), the last element and the final window.
+//
+// What bounds it: VALU issue (737 instructions a step, 0.5 a cycle and CU at
+// 25,000 seeds) and, for the last seeds, the chain of one step (about 3 us).
+// Measured against flat_slot<PROB> (81x106x76, 724 vertices, step 1/4 voxel):
+// 64 seeds 9.8 -> 2.6 ms, 25,000 seeds 120 -> 41 ms, 100,000 255 -> 126 ms;
+// fetched from memory at 25,000 seeds: 17 GB for 9.6 M steps.  The same
+// kernel with 32 lanes a seed and the gather repeated every step: 67 and
+// 187 ms.
+//
+// Fast values only: a NaN or a value of 1e30 or more anywhere in the pmf
+// sends the step to prob_sum and prob_pick.  Values left by the threshold are
+// never negative (a negative maximum zeroes everything), so masked additions
+// of +0 change nothing.
+// -------------------------------------------------------------------------
+// 2 waves per SIMD: 96 registers hold the cell.  At 3 (168 registers) 82 spill
+// and a 25,000-seed chunk takes 59.9 ms instead of 42.8.
+constexpr int PROB_WAVES = 2;
+constexpr int PROB_W_BLOCK = 36;  // LDS floats per 32-value block: the 4 extra spread the lanes' block reads over banks
+constexpr float PROB_FAST_MAX = 1e30f;
+constexpr int prob_slot_floats(int nch) { return PROB_W_BLOCK * 8 * nch + 64; }
+
+constexpr int DPP_ROW_SHR = 0x110, DPP_ROW_ROR = 0x120, DPP_WAVE_SHR1 = 0x138;
+template <int CTRL>
+__device__ __forceinline__ float dpp0(float x) {  // 0 where the shift has no source lane
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+
+// Maximum over the wave, NaN if any value is.
+__device__ __forceinline__ float nan_max64(float v) {
+    v = __builtin_elementwise_maximum(v, dpp0<DPP_ROW_ROR + 8>(v));
+    v = __builtin_elementwise_maximum(v, dpp0<DPP_ROW_ROR + 4>(v));
+    v = __builtin_elementwise_maximum(v, dpp0<DPP_ROW_ROR + 2>(v));
+    v = __builtin_elementwise_maximum(v, dpp0<DPP_ROW_ROR + 1>(v));
+    const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __builtin_elementwise_maximum(__uint_as_float(s16[0]), __uint_as_float(s16[1]));
+    const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __builtin_elementwise_maximum(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
+}
+
+__device__ __forceinline__ float uniform_f(float x) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+__device__ __forceinline__ float lane_f(float x, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
+
+// out[i] of the running sum, from the blocks' W and carries.
+__device__ __forceinline__ float prob_cdf(const float *W, const float *carry, int i) {
+    const int b = i >> 5, e = i & 31;
+    const float *w = W + PROB_W_BLOCK * b;
+    const float c = carry[b], w0 = w[0], w1 = w[e & 1], w2 = w[e & 3], w3 = w[e & 7], w4 = w[e & 15], w5 = w[e];
+    float s = w0 + c;
+    s = (e & 1) ? w1 + s : s;
+    s = (e & 2) ? w2 + s : s;
+    s = (e & 4) ? w3 + s : s;
+    s = (e & 8) ? w4 + s : s;
+    s = (e & 16) ? w5 + s : s;
+    return s;
+}
+
+// The midpoint that node k of the binary search's tree compares (root 0, the
+// children of k at 2 k + 1 for "below", 2 k + 2 for "not below").
+__device__ __forceinline__ int prob_node_mid(int nv, int k) {
+    int low = 0, high = nv - 1;
+    const int path = k + 1;
+    for (int d = 30 - __clz(path); d >= 0; --d) {
+        const int mid = (low + high) >> 1;
+        if ((path >> d) & 1) high = mid; else low = mid;
+    }
+    return (low + high) >> 1;
+}
+
+// The step's choice by the general routines (out of line: rare); -1: none.
+// Both halves of the wave do the same work on the same array.
+__device__ __noinline__ int prob_slow(int nv, int symm, float cos_max_angle, const float *verts, float *pmf, float u,
+                                      float dx, float dy, float dz) {
+    const float last = prob_sum(nv, symm, cos_max_angle, verts, pmf, dx, dy, dz);
+    return (last == 0.0f) ? -1 : prob_pick(pmf, nv, u * last);
+}
+
+typedef float prob_v4 __attribute__((ext_vector_type(4)));
+
+// A wave's last cell: its corners (bit 2 x, bit 1 y, bit 0 z, as trilinear's).
+template <int NCH>
+struct ProbCell {
+    prob_v4 v[8][NCH];
+    int x, y, z;
+};
+
+// Move the corners one cell along the axis of corner bit BIT (e: -1, 0, 1);
+// returns the corners that hold the new cell's values (bit mask).
+template <int NCH, int BIT>
+__device__ __forceinline__ uint32_t prob_shift(ProbCell<NCH> &C, int e) {
+    constexpr uint32_t LOW = (BIT == 1) ? 0x55u : (BIT == 2) ? 0x33u : 0x0fu;  // corners with the bit clear
+    constexpr int U = (BIT == 1) ? 2 : 1, V = (BIT == 4) ? 2 : 4;              // the other two bits
+    // The empty asm keeps the two branches apart: merged, their stores would
+    // index the register array at run time and send it to scratch.
+    if (e > 0) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            C.v[0][c] = C.v[BIT][c];
+            C.v[U][c] = C.v[U | BIT][c];
+            C.v[V][c] = C.v[V | BIT][c];
+            C.v[U | V][c] = C.v[7][c];
+        }
+        asm volatile("; cell up");
+        return LOW;
+    }
+    if (e < 0) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            C.v[BIT][c] = C.v[0][c];
+            C.v[U | BIT][c] = C.v[U][c];
+            C.v[V | BIT][c] = C.v[V][c];
+            C.v[7][c] = C.v[U | V][c];
+        }
+        asm volatile("; cell down");
+        return 0xffu & ~LOW;
+    }
+    return 0xffu;
+}
+
+// Bring the cell to (x0, y0, z0): corners shared with the last cell move,
+// the others are read.
+template <int NCH>
+__device__ __forceinline__ void prob_move_cell(const DevParams &P, const float *__restrict__ data, ProbCell<NCH> &C,
+                                               int x0, int y0, int z0, uint32_t off, uint32_t off_last) {
+    const int ex = x0 - C.x, ey = y0 - C.y, ez = z0 - C.z;
+    if ((ex | ey | ez) == 0) return;
+    C.x = x0; C.y = y0; C.z = z0;
+    uint32_t valid = 0u;
+    if ((uint32_t)(ex + 1) <= 2u && (uint32_t)(ey + 1) <= 2u && (uint32_t)(ez + 1) <= 2u) {
+        valid = 0xffu;
+        valid &= prob_shift<NCH, 1>(C, ez);
+        valid &= prob_shift<NCH, 2>(C, ey);
+        valid &= prob_shift<NCH, 4>(C, ex);
+    }
+    const uint32_t dzv = (z0 + 1 < P.dimz) ? 1u : 0u;
+    const uint32_t dyv = (y0 + 1 < P.dimy) ? (uint32_t)P.dimz : 0u;
+    const uint32_t dxv = (x0 + 1 < P.dimx) ? (uint32_t)P.dimy * (uint32_t)P.dimz : 0u;
+    const uint32_t vox = ((uint32_t)x0 * (uint32_t)P.dimy + (uint32_t)y0) * (uint32_t)P.dimz + (uint32_t)z0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if ((valid >> k) & 1u) continue;
+        const uint32_t vk = vox + ((k & 4) ? dxv : 0u) + ((k & 2) ? dyv : 0u) + ((k & 1) ? dzv : 0u);
+        const char *row = reinterpret_cast<const char *>(data + (uint64_t)vk * (uint32_t)P.t32);
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            C.v[k][c] = *reinterpret_cast<const prob_v4 *>(row + ((c == NCH - 1) ? off_last : off + 1024u * c));
+    }
+}
+
+// check_point for a wave whose lanes share the point: lane k (of every 8)
+// reads texel k and forms its weight, and the sum moves along the lanes, one
+// fused multiply-add each, in check_point's order.
+struct WaveTap {
+    float w, t;
+};
+
+__device__ __forceinline__ WaveTap wave_stop_begin(const DevParams &P, const float *__restrict__ stop, float px,
+                                                   float py, float pz) {
+    const int kz = threadIdx.x & 1, ky = (threadIdx.x >> 1) & 1, kx = (threadIdx.x >> 2) & 1;
+    int iz, iy, ix;
+    const float a = tex_weight(pz, &iz), b = tex_weight(py, &iy), g = tex_weight(px, &ix);
+    const float wa = kz ? a : 1.0f - a, wb = ky ? b : 1.0f - b, wg = kx ? g : 1.0f - g;
+    // i = -k .. D - 1 - k is inside; outside reads a clamped texel, replaced
+    const bool in = (ix >= -kx) & (ix < P.dimx - kx) & (iy >= -ky) & (iy < P.dimy - ky) & (iz >= -kz) &
+                    (iz < P.dimz - kz);
+    const uint32_t x = (uint32_t)(min(max(ix, -kx), P.dimx - 1 - kx) + kx),
+                   y = (uint32_t)(min(max(iy, -ky), P.dimy - 1 - ky) + ky),
+                   z = (uint32_t)(min(max(iz, -kz), P.dimz - 1 - kz) + kz);
+    WaveTap r;
+    const float t = stop[(size_t)((x * (uint32_t)P.dimy + y) * (uint32_t)P.dimz + z)];
+    r.t = in ? t : -1.0f;
+    r.w = (wa * wb) * wg;
+    return r;
+}
+
+__device__ __forceinline__ int wave_stop_end(const DevParams &P, const WaveTap &r) {
+    float acc = r.w * r.t;
+#pragma unroll
+    for (int k = 1; k < 8; ++k) acc = __builtin_fmaf(r.w, r.t, dpp0<DPP_ROW_SHR + 1>(acc));
+    acc = lane_f(acc, 7);
+    if (acc == -1.0f) return CUSLINES_OUTSIDEIMAGE;
+    return (acc > P.tc_threshold) ? CUSLINES_TRACKPOINT : CUSLINES_ENDPOINT;
+}
+
+// One direction draw at (px, py, pz).  `check`: the point's stop-map check
+// is still to do (not at a pass's first point).  Returns 1 with the new
+// direction, 0 when there is none, -1 when the stop check ends the pass.
+template <int NCH>
+__device__ __forceinline__ int prob_step(const DevParams &P, const DevBufs &B, const float *sv, float *W, float *carry,
+                                         ProbCell<NCH> &C, int my_mid, float m1, float m2, float m4, bool tail,
+                                         uint32_t off, uint32_t off_last, bool check, ProbStream<64> &rng, float dx,
+                                         float dy, float dz, float px, float py, float pz, float *ndx, float *ndy,
+                                         float *ndz) {
+    const int l = threadIdx.x & 63;
+    const int nv = P.nverts;
+    const WaveTap tap = wave_stop_begin(P, B.stop, px, py, pz);
+    // trilinear()'s cell and weights, the cell clamped so that a point
+    // outside reads in bounds (its values are dropped)
+    const bool outside = (px < -0.5f) | (px + 0.5f >= (float)P.dimx) | (py < -0.5f) | (py + 0.5f >= (float)P.dimy) |
+                         (pz < -0.5f) | (pz + 0.5f >= (float)P.dimz);
+    const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+    const float wx1 = px - fx, wy1 = py - fy, wz1 = pz - fz;
+    const float wx0 = 1.0f - wx1, wy0 = 1.0f - wy1, wz0 = 1.0f - wz1;
+    const float w[8] = {(wx0 * wy0) * wz0, (wx0 * wy0) * wz1, (wx0 * wy1) * wz0, (wx0 * wy1) * wz1,
+                        (wx1 * wy0) * wz0, (wx1 * wy0) * wz1, (wx1 * wy1) * wz0, (wx1 * wy1) * wz1};
+    const int x0 = min((int)((0.0f > fx) ? 0.0f : fx), P.dimx - 1), y0 = min((int)((0.0f > fy) ? 0.0f : fy), P.dimy - 1),
+              z0 = min((int)((0.0f > fz) ? 0.0f : fz), P.dimz - 1);
+    prob_move_cell<NCH>(P, B.data, C, __builtin_amdgcn_readfirstlane(x0), __builtin_amdgcn_readfirstlane(y0),
+                        __builtin_amdgcn_readfirstlane(z0), off, off_last);
+    if (check && wave_stop_end(P, tap) != CUSLINES_TRACKPOINT) return -1;
+    if (__builtin_amdgcn_readfirstlane(outside)) return 0;
+    prob_v4 acc[NCH];
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+        acc[c] = prob_v4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            acc[c].x = __builtin_fmaf(w[k], C.v[k][c].x, acc[c].x);
+            acc[c].y = __builtin_fmaf(w[k], C.v[k][c].y, acc[c].y);
+            acc[c].z = __builtin_fmaf(w[k], C.v[k][c].z, acc[c].z);
+            acc[c].w = __builtin_fmaf(w[k], C.v[k][c].w, acc[c].w);
+        }
+    }
+    if (!tail) acc[NCH - 1] = prob_v4{0.0f, 0.0f, 0.0f, 0.0f};
+    // channels nverts.. of a row are 0 in memory: they leave a maximum that
+    // would be negative at 0, and either way the threshold drops everything
+    float mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(acc[0].x, acc[0].y),
+                                             __builtin_elementwise_maximum(acc[0].z, acc[0].w));
+#pragma unroll
+    for (int c = 1; c < NCH; ++c)
+        mx = __builtin_elementwise_maximum(
+            mx, __builtin_elementwise_maximum(__builtin_elementwise_maximum(acc[c].x, acc[c].y),
+                                              __builtin_elementwise_maximum(acc[c].z, acc[c].w)));
+    mx = uniform_f(nan_max64(mx));
+    const float u = rng.peek();
+    int ind;
+    if (!(mx < PROB_FAST_MAX)) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) *reinterpret_cast<prob_v4 *>(W + 256 * c + 4 * l) = acc[c];
+        WAVE_SYNC();
+        ind = __builtin_amdgcn_readfirstlane(
+            prob_slow(nv, P.sphere_symm, P.cos_max_angle, B.verts, W, u, dx, dy, dz));
+        if (ind < 0) return 0;
+        rng.take();
+    } else {
+        const float thr = (float)(PMF_THRESHOLD_P * (double)mx);
+        const float cosm = P.cos_max_angle;
+        const uint32_t dmask = P.sphere_symm ? 0x7fffffffu : 0xffffffffu;
+        auto keep = [&](float v, float x, float y, float z) {
+            // |d| on a symmetric sphere: the sign bit masked off
+            const float d = __uint_as_float(__float_as_uint(dot3(dx, dy, dz, x, y, z)) & dmask);
+            return ((v < thr) | (d < cosm)) ? 0.0f : v;
+        };
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            const prob_v4 vx = *reinterpret_cast<const prob_v4 *>(sv + 256 * c + 4 * l);
+            const prob_v4 vy = *reinterpret_cast<const prob_v4 *>(sv + 256 * (NCH + c) + 4 * l);
+            const prob_v4 vz = *reinterpret_cast<const prob_v4 *>(sv + 256 * (2 * NCH + c) + 4 * l);
+            acc[c].x = keep(acc[c].x, vx.x, vy.x, vz.x);
+            acc[c].y = keep(acc[c].y, vx.y, vy.y, vz.y);
+            acc[c].z = keep(acc[c].z, vx.z, vy.z, vz.z);
+            acc[c].w = keep(acc[c].w, vx.w, vy.w, vz.w);
+        }
+        // rounds 1, 2, 4, 8 for elements >= 2, 4, 8, 16 of a block (8 lanes),
+        // round by round over the independent chunks; a factor 0 or 1 masks
+        // the addition
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            const prob_v4 q = acc[c];
+            acc[c].w = q.w + q.z;
+            acc[c].z = q.z + q.y;
+            acc[c].y = __builtin_fmaf(q.x, m1, q.y);
+            acc[c].x = __builtin_fmaf(dpp0<DPP_ROW_SHR + 1>(q.w), m1, q.x);
+        }
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            const prob_v4 q = acc[c];
+            acc[c].w = __builtin_fmaf(q.y, m1, q.w);
+            acc[c].z = __builtin_fmaf(q.x, m1, q.z);
+            acc[c].y = __builtin_fmaf(dpp0<DPP_ROW_SHR + 1>(q.w), m1, q.y);
+            acc[c].x = __builtin_fmaf(dpp0<DPP_ROW_SHR + 1>(q.z), m1, q.x);
+        }
+        // v <- v + m * shift(v) in one instruction each; a DPP source must be
+        // two instructions old, hence the s_nop at both ends of a round
+#define PROB_SHIFT_ADD(SHIFT, MASK)                                                                              \
+    _Pragma("unroll") for (int c = 0; c < NCH; ++c) {                                                            \
+        float ax = acc[c].x, ay = acc[c].y, az = acc[c].z, aw = acc[c].w;                                        \
+        asm volatile("s_nop 1\n\t"                                                                                            \
+        "v_fmac_f32_dpp %0, %0, %4 row_shr:" SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"                 \
+        "v_fmac_f32_dpp %1, %1, %4 row_shr:" SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"                 \
+        "v_fmac_f32_dpp %2, %2, %4 row_shr:" SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"                 \
+        "v_fmac_f32_dpp %3, %3, %4 row_shr:" SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"                 \
+        "s_nop 1"                                                                                                \
+        : "+v"(ax), "+v"(ay), "+v"(az), "+v"(aw)                                                                 \
+        : "v"(MASK));                                                                                            \
+        acc[c] = prob_v4{ax, ay, az, aw};                                                                        \
+    }
+        PROB_SHIFT_ADD("1", m2)
+        PROB_SHIFT_ADD("2", m4)
+#undef PROB_SHIFT_ADD
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            *reinterpret_cast<prob_v4 *>(W + PROB_W_BLOCK * (8 * c + (l >> 3)) + 4 * (l & 7)) = acc[c];
+        WAVE_SYNC();
+        // lane b: block b's part of the carry chain
+        const int nblk = (nv + 31) >> 5;
+        {
+            const float *wb = W + PROB_W_BLOCK * min(l, nblk - 1);
+            const float4 q = *reinterpret_cast<const float4 *>(wb);
+            const float s7 = wb[7], s15 = wb[15], s31 = wb[31];
+            float x = 0.0f;
+            for (int it = 1; it < nblk; ++it) {
+                float t = q.x + dpp0<DPP_WAVE_SHR1>(x);
+                t = q.y + t;
+                t = q.w + t;
+                t = s7 + t;
+                t = s15 + t;
+                x = s31 + t;
+            }
+            carry[l] = dpp0<DPP_WAVE_SHR1>(x);
+        }
+        WAVE_SYNC();
+        // lane k < 31: node k of the search tree; lane 31: the last element
+        const float node = prob_cdf(W, carry, my_mid);
+        const float last = lane_f(node, 31);
+        if (last == 0.0f) return 0;
+        rng.take();
+        const float sel = u * last;
+        const uint32_t below = (uint32_t)__ballot(node < sel);
+        int low = 0, high = nv - 1, k = 0;
+#pragma unroll
+        for (int lev = 0; lev < 5; ++lev) {
+            const int mid = (low + high) >> 1;
+            const bool open = (high - low) >= 32;
+            const bool bl = (below >> k) & 1u;
+            low = (open && bl) ? mid : low;
+            high = (open && !bl) ? mid : high;
+            k = 2 * k + (bl ? 1 : 2);
+        }
+        const float win = prob_cdf(W, carry, min(low + l, nv - 1));
+        const unsigned long long msk = __ballot(low + l <= high && sel < win);
+        ind = max(low + __ffsll(msk) - 1, 0);
+    }
+    const float ux = sv[ind], uy = sv[256 * NCH + ind], uz = sv[512 * NCH + ind];
+    const bool fwd = dot3(dx, dy, dz, ux, uy, uz) > 0.0f;
+    *ndx = fwd ? ux : -ux;
+    *ndy = fwd ? uy : -uy;
+    *ndz = fwd ? uz : -uz;
+    WAVE_SYNC();
+    return 1;
+}
+
+// flat_slot's loop for one wave.
+template <int NCH>
+__device__ void flat_wave_prob(const DevParams &P, const DevBufs &B, const float *sv, float *lds,
+                               const float *__restrict__ seeds, int nseeds, int rng_chunk,
+                               const int *__restrict__ offsets, const int *__restrict__ dirs,
+                               int *__restrict__ sline_seed, int *__restrict__ sline_len, float *__restrict__ sline,
+                               const int *__restrict__ order, int *__restrict__ work) {
+    const int l = threadIdx.x & 63;
+    const int xcd = blockIdx.x & (QUEUES - 1);
+    const int MAXL = P.max_sline_len;
+    const double sub = P.step_d;
+    const size_t slot_f = (size_t)2 * MAXL * 3;
+    float *W = lds, *carry = lds + PROB_W_BLOCK * 8 * NCH;
+    const int my_mid = (l < 31) ? prob_node_mid(P.nverts, l) : (l == 31) ? P.nverts - 1 : 0;
+    const float m1 = ((l & 7) >= 1) ? 1.0f : 0.0f, m2 = ((l & 7) >= 2) ? 1.0f : 0.0f, m4 = ((l & 7) >= 4) ? 1.0f : 0.0f;
+    // NCH is the number of chunks of a padded row, so only the last can be
+    // partial: its lanes past the row re-read chunk 0 and drop it
+    const bool tail = 256 * (NCH - 1) + 4 * l < P.t32;
+    const uint32_t off = 16u * l, off_last = off + (tail ? 1024u * (NCH - 1) : 0u);
+    ProbCell<NCH> C;
+    C.x = C.y = C.z = -4;  // no cell's neighbour
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) C.v[k][c] = prob_v4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    ProbStream<64> rng;
+    int qk = 0, s = 0, ndir = 0, di = 0, slot = 0, nb = 0;  // seed, its directions, the next, output slot, backward points
+    float sx = 0.0f, sy = 0.0f, sz = 0.0f, fx = 0.0f, fy = 0.0f, fz = 0.0f;
+    bool have = false, check = false;
+    int pass = 0, i = 1;
+    float px = 0.0f, py = 0.0f, pz = 0.0f, dx = 0.0f, dy = 0.0f, dz = 0.0f;
+    float *sl = sline;
+    for (;;) {
+        if (!have) {
+            // the next direction of this seed, or of the next seeds
+            while (di >= ndir && qk < QUEUES) {
+                const int qx = (xcd + qk) & (QUEUES - 1);
+                const int lo = (int)((long long)nseeds * qx / QUEUES);
+                const int hi = (int)((long long)nseeds * (qx + 1) / QUEUES);
+                int q = 0;
+                if (l == 0) q = atomicAdd(work + qx, 1);
+                q = __builtin_amdgcn_readfirstlane(q);
+                if (lo + q >= hi) { ++qk; continue; }
+                s = __builtin_amdgcn_readfirstlane(order[lo + q]);
+                const int o0 = __builtin_amdgcn_readfirstlane(offsets[s]),
+                          o1 = __builtin_amdgcn_readfirstlane(offsets[s + 1]);
+                ndir = (P.slot_cap > 0 && o1 > P.slot_cap) ? 0 : o1 - o0;
+                di = 0;
+                slot = o0 - 1;
+                sx = seeds[3 * (size_t)s]; sy = seeds[3 * (size_t)s + 1]; sz = seeds[3 * (size_t)s + 2];
+                rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo, (uint64_t)32 * (uint64_t)(s % rng_chunk) + 1);
+            }
+            if (di >= ndir) break;  // the queues are empty
+            const int vi = __builtin_amdgcn_readfirstlane(dirs[(size_t)s * P.nverts + di]);
+            fx = B.verts[3 * vi]; fy = B.verts[3 * vi + 1]; fz = B.verts[3 * vi + 2];
+            ++di;
+            ++slot;
+            sl = sline + (size_t)slot * slot_f;
+            // backward pass (-dir)
+            px = sx; py = sy; pz = sz;
+            dx = -fx; dy = -fy; dz = -fz;
+            if (l == 0) {
+                sline_seed[slot] = s;
+                sl[0] = px; sl[1] = py; sl[2] = pz;
+            }
+            pass = 0;
+            i = 1;
+            check = false;
+            have = true;
+        }
+        // one step of the pass: `i` points are stored; the stop check of the
+        // last one, left over from the step that stored it, comes with this
+        // step's reads
+        float nx = 0.0f, ny = 0.0f, nz = 0.0f;
+        int nsteps;
+        if (i >= MAXL) {
+            const bool bad = check && wave_stop_end(P, wave_stop_begin(P, B.stop, px, py, pz)) != CUSLINES_TRACKPOINT;
+            nsteps = bad ? i - 1 : i;
+        } else {
+            const int nd = prob_step<NCH>(P, B, sv, W, carry, C, my_mid, m1, m2, m4, tail, off, off_last, check, rng, dx,
+                                          dy, dz, px, py, pz, &nx, &ny, &nz);
+            if (nd > 0) {
+                dx = nx; dy = ny; dz = nz;
+                px = (float)__builtin_fma((double)(dx / 1.0f), sub, (double)px);
+                py = (float)__builtin_fma((double)(dy / 1.0f), sub, (double)py);
+                pz = (float)__builtin_fma((double)(dz / 1.0f), sub, (double)pz);
+                if (l < 3) sl[3 * (size_t)i + l] = (l == 0) ? px : (l == 1) ? py : pz;
+                ++i;
+                check = true;
+                continue;
+            }
+            nsteps = (nd < 0) ? i - 1 : i;
+        }
+        // the pass ends with nsteps points (tracker's tail)
+        check = false;
+        if (pass == 0) {
+            MEM_SYNC();
+            for (int j = l; j < nsteps / 2; j += 64) {
+                float *a = sl + 3 * (size_t)j, *b = sl + 3 * (size_t)(nsteps - 1 - j);
+                const float a0 = a[0], a1 = a[1], a2 = a[2];
+                a[0] = b[0]; a[1] = b[1]; a[2] = b[2];
+                b[0] = a0; b[1] = a1; b[2] = a2;
+            }
+            MEM_SYNC();
+            nb = nsteps;
+            // forward pass (+dir), from the seed point at index nsteps - 1
+            pass = 1;
+            px = sx; py = sy; pz = sz;
+            dx = fx; dy = fy; dz = fz;
+            sl += 3 * (size_t)(nsteps - 1);
+            if (l == 0) { sl[0] = px; sl[1] = py; sl[2] = pz; }
+            i = 1;
+        } else {
+            if (l == 0) sline_len[slot] = nb - 1 + nsteps;
+            have = false;
+        }
+    }
+}
+
+template <int NCH>
+__global__ void __launch_bounds__(256, PROB_WAVES)
+    phase2_prob_kernel(DevParams P, DevBufs B, const float *__restrict__ seeds, int nseeds, int rng_chunk,
+                       const int *__restrict__ offsets, const int *__restrict__ dirs, int *__restrict__ sline_seed,
+                       int *__restrict__ sline_len, float *__restrict__ sline, const int *__restrict__ order,
+                       int *__restrict__ work) {
+    extern __shared__ float4 smem4[];
+    float *smem = reinterpret_cast<float *>(smem4);
+    // vertices as x[], y[], z[], 0 past the last
+    for (int i = threadIdx.x; i < 3 * 256 * NCH; i += blockDim.x) {
+        const int a = i / (256 * NCH), v = i - a * (256 * NCH);
+        smem[i] = (v < P.nverts) ? B.verts[3 * v + a] : 0.0f;
+    }
+    __syncthreads();
+    flat_wave_prob<NCH>(P, B, smem, smem + 3 * 256 * NCH + (threadIdx.x >> 6) * prob_slot_floats(NCH), seeds, nseeds,
+                        rng_chunk, offsets, dirs, sline_seed, sline_len, sline, order, work);
 }
 
 // One seed per 32-lane slot, static assignment.
@@ -3991,6 +4617,37 @@ static int launch_phase2_v(cuslines_tracker *t, const float *seeds, int n, int c
     return CUSLINES_OK;
 }
 
+// Probabilistic phase 2 with the cell in registers: NCH chunks of 256
+// channels.  Work queue and spatial order as launch_phase2_v; one wave per
+// workgroup, so that few seeds spread over the CUs.
+template <int NCH>
+static int launch_prob(cuslines_tracker *t, const float *seeds, int n, int chunk, const int *offsets, const int *dirs,
+                       int *sseed, int *slen, float *sl, int *ws) {
+    const DevParams &d = t->dp;
+    const int threads = t->threads > 0 ? t->threads : 64;
+    const int nslots = threads / 64;
+    const size_t lds = sizeof(float) * (3 * 256 * NCH + (size_t)nslots * prob_slot_floats(NCH));
+    const void *kfn = (const void *)phase2_prob_kernel<NCH>;
+    HIPC(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int per_cu = 0;
+    HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, threads, lds));
+    if (per_cu < 1) per_cu = 1;
+    if (t->blocks_per_cu > 0 && t->blocks_per_cu < per_cu) per_cu = t->blocks_per_cu;
+    long long grid = (long long)per_cu * t->num_cu;
+    const long long need = (n + nslots - 1) / nslots;
+    if (grid > need) grid = need;
+    if (grid < 1) grid = 1;
+    int *order = nullptr;
+    if (int rc = spatial_order(t, seeds, n, &order, ws)) return rc;
+    hipLaunchKernelGGL(zero_ints, dim3(1), dim3(QUEUES), 0, t->stream, t->d_work, QUEUES);
+    hipLaunchKernelGGL(phase2_prob_kernel<NCH>, dim3((unsigned)grid), dim3(threads), lds, t->stream, d, bufs_of(t),
+                       seeds, n, chunk, offsets, dirs, sseed, slen, sl, order, t->d_work);
+    hipError_t e = hipGetLastError();
+    if (!ws) (void)hipFreeAsync(order, t->stream);
+    if (e != hipSuccess) return fail(CUSLINES_EHIP, std::string("phase 2 (prob): ") + hipGetErrorString(e));
+    return CUSLINES_OK;
+}
+
 // Limits of the batched bootstrap kernel's tile counts per wave.
 static bool boot_batch_fits(const DevParams &d) {
     return d.hr16 <= 320 && d.dn16 <= 128 && d.nv16 <= 768 && d.dn16 <= d.t32;
@@ -4066,6 +4723,15 @@ static int launch_phase2(cuslines_tracker *t, const float *seeds, int n, int chu
             return launch_phase2_v<MODEL, 3>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
         if (t->ptt_lanes > 0 && t->schedule != CUSLINES_SCHED_STATIC)
             return launch_ptt_groups(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
+    }
+    if constexpr (MODEL == CUSLINES_PROB) {
+        // a lane keeps 4 of a chunk's 256 channels, 8 corners each: 3 chunks fit the registers
+        if (t->flat && t->schedule != CUSLINES_SCHED_STATIC) switch ((t->dp.t32 + 255) / 256) {
+            case 1: return launch_prob<1>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
+            case 2: return launch_prob<2>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
+            case 3: return launch_prob<3>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
+            default: break;
+        }
     }
     if (t->flat && t->schedule != CUSLINES_SCHED_STATIC)
         return launch_phase2_v<MODEL, 4>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);

@@ -189,7 +189,8 @@ enum {
 
 /* Launch configuration of phase 2 (chosen by gpustreamlines_amd.autotune):
  * schedule, threads per block (0 = getter default, else 64..256 in steps of
- * 64; every 32 threads are one seed slot) and resident blocks per CU of the
+ * 64; every 32 threads are one seed slot, every 64 in the probabilistic
+ * getter's queue kernel for up to 768 vertices) and resident blocks per CU of the
  * persistent grid (0 = the occupancy maximum).  The reference's launch shape
  * is fixed at 2 seeds per 64-thread block (cu_propagate_seeds.py:45-54). */
 int cuslines_set_launch(cuslines_tracker *t, int schedule, int threads, int blocks_per_cu);
