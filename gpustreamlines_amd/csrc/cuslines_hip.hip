@@ -392,9 +392,9 @@ __device__ int trilinear(const DevParams &P, const float *__restrict__ data, int
 // weight = frac(xB) with 8 fractional bits.
 __device__ __forceinline__ float tex_weight(float c, int *i0) {
     const float b = c - 0.5f;
-    const float fl = floorf(b);
-    *i0 = (int)fl;
-    return __builtin_rintf((b - fl) * 256.0f) * 0.00390625f;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(*i0) : "v"(b));
+    // v_fract_f32: b - floor(b), held below 1, which rounds to the same 1/256
+    return __builtin_rintf(__builtin_amdgcn_fractf(b) * 256.0f) * 0.00390625f;
 }
 
 // check_point_d (tracking_helpers.cu:63-73): linear filter of the stop map,
@@ -507,14 +507,22 @@ __device__ float tiled_sample(const DevParams &P, const float *__restrict__ odfv
 // (point sampling, normalised coordinates, clamp).  Index products use
 // 24-bit multiplies (full rate; every operand is below 2^24: LUT coordinates,
 // tile indices, cell coordinates).
+// v_cvt_u32_f32 takes negative values and NaN to 0 and truncates, so one
+// minimum is left of floor and clamp.
+__device__ __forceinline__ uint32_t cvt_u32_sat(float x) {
+    uint32_t r;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
 __device__ __forceinline__ uint32_t lut_index(const DevParams &P, float f0, float f1, float f2) {
     const int res = P.lut_res;
-    const float rf = (float)res, rmax = (float)(res - 1);
+    const float rf = (float)res;
+    const uint32_t imax = (uint32_t)res - 1u;
     const float u0 = __builtin_fmaf(f0, 0.5f, 0.5f), u1 = __builtin_fmaf(f1, 0.5f, 0.5f),
                 u2 = __builtin_fmaf(f2, 0.5f, 0.5f);
-    const uint32_t i0 = (uint32_t)fminf(fmaxf(floorf(u0 * rf), 0.0f), rmax);
-    const uint32_t i1 = (uint32_t)fminf(fmaxf(floorf(u1 * rf), 0.0f), rmax);
-    const uint32_t i2 = (uint32_t)fminf(fmaxf(floorf(u2 * rf), 0.0f), rmax);
+    const uint32_t i0 = min(cvt_u32_sat(u0 * rf), imax), i1 = min(cvt_u32_sat(u1 * rf), imax),
+                   i2 = min(cvt_u32_sat(u2 * rf), imax);
     if (P.lut_brick) {
         const uint32_t nb = (uint32_t)res >> 2;
         return (__umul24(__umul24(i0 >> 2, nb) + (i1 >> 2), nb) + (i2 >> 2)) * 64u + ((i0 & 3u) << 4) +
@@ -2572,7 +2580,8 @@ __device__ __forceinline__ int stage_network(const DevBufs &B, float *lds, DevBu
 }
 
 // Phase 2 of one 32-lane slot with the stepping loop flattened (the queue
-// kernel's V == 4).  In track_seed a slot whose streamline pass, direction
+// kernel's V == 4: the exact bootstrap getters and spheres too large for the
+// probabilistic getter's own kernel; V == 5: the learned proposal).  In track_seed a slot whose streamline pass, direction
 // or seed ends leaves its loops and waits at their exit until the wave's
 // other slot leaves them too; here one iteration of a single loop is one
 // step (PTT: sub-step) of whichever pass the slot holds, and a slot whose
@@ -2592,6 +2601,7 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
                           const int *__restrict__ dirs, int *__restrict__ sline_seed, int *__restrict__ sline_len,
                           float *__restrict__ sline, const int *__restrict__ order, int *__restrict__ work) {
     constexpr bool PTT = MODEL == CUSLINES_PTT;
+    static_assert(PTT == LEARNED, "plain PTT: flat_slot_ptt");
     const int l = lane32();
     const int xcd = blockIdx.x & (QUEUES - 1);
     const int step_frac = PTT ? P.step_frac : 1, MAXL = P.max_sline_len;
@@ -2679,7 +2689,7 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
             int nd;
             if constexpr (MODEL == CUSLINES_PROB) {
                 nd = get_direction_prob<false>(P, B, sv, S.prob, rng, dx, dy, dz, px, py, pz, &nx, &ny, &nz);
-            } else if constexpr (PTT && LEARNED) {
+            } else if constexpr (LEARNED) {
                 int fell = 0;
                 nd = get_direction_ptt_learned(P, B, S.ptt, S.ptt.frame + (pass ? 9 : 0), rng, learned, dx, dy, dz, px,
                                                py, pz, &nx, &ny, &nz, &fell, &lmiss);
@@ -2690,9 +2700,6 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
                 } else {
                     ++nplain;
                 }
-            } else if constexpr (PTT) {
-                nd = get_direction_ptt<false>(P, B, S.ptt, S.ptt.frame + (pass ? 9 : 0), rng, dx, dy, dz, px, py, pz,
-                                              &nx, &ny, &nz);
             } else
                 nd = get_direction_boot<MODEL>(P, B, sv, S.boot, rng, 5, dx, dy, dz, px, py, pz, &nx, &ny, &nz);
             if (nd == 0) {
@@ -3283,6 +3290,527 @@ __global__ void __launch_bounds__(256, PROB_WAVES)
                         rng_chunk, offsets, dirs, sline_seed, sline_len, sline, order, work);
 }
 
+// -------------------------------------------------------------------------
+// Plain PTT phase 2 (the queue's flat stepping).
+//
+// Same sub-step as ptt_substep, arranged for the latency of a lone wave and
+// for issue slots:
+//  - the vertex phase's 24 curves first run all their frames (no load is
+//    waited for: each probe's LUT entry arrives while the next frame is
+//    propagated and goes to LDS with the probe's position); then the 192
+//    taps are shared by the slot's 32 lanes, 6 each instead of 8 on 24
+//    lanes, their block reads in flight 3 at a time, and lane v adds its 8
+//    values in probe order.  data_support instead waits for a LUT entry and
+//    a block per probe;
+//  - the tangent's own tap is read under the frames;
+//  - frames skip their three norms' range tests one by one (one test of the
+//    smallest and largest square; the rare failure redoes the frame), and
+//    the last probe's normal and binormal, which nothing reads;
+//  - a rejection round ends as soon as lane 0's candidate passes: the lowest
+//    passing lane wins, and every lane has taken its three draws already;
+//  - the disc's propagators and faces come from LDS, the face search from
+//    two LDS reads (levels 1-3, then 4-5) instead of five dependent ones, and
+//    the face scan from row shifts; the frame stays in registers.
+// Same additions, products and draws in the same order: bit-identical.
+//
+// What bounds it: VALU instructions (1,498 a sub-step and slot; data_support's
+// loop took 1,881), a third of them the 24 x 8 frames; a dependent one takes
+// 8.4 cycles, so a lone wave needs about 21,000 cycles a sub-step.  Against
+// flat_slot<PTT>: 40 seeds 193 -> 148 ms, 4,001 361 -> 267 ms, 25,000 760 ->
+// 640 ms, 250,000 4.67 -> 4.39 s.
+// -------------------------------------------------------------------------
+// 2 waves per SIMD and all of a group's taps in flight: at 3 waves (168
+// registers, 29 spilled) with 3 taps 25,000 seeds take 714 ms instead of 618
+// and 250,000 seeds 4.75 s instead of 4.39.
+constexpr int PTT_WAVES = 2;
+constexpr int PTT_BATCH = 6;                          // tap rounds in flight
+constexpr int PTT_GROUP = 8;                          // probes whose taps are in LDS together
+constexpr int PTT_ENTRIES = DISC_VERT_CNT * PTT_GROUP;
+constexpr int PTT_TAB_FLOATS = DISC_VERT_CNT * 12 + 32 * 8;  // propagators [24][12], faces [32][8]
+// frame 32, vertex pdf 32, face cdf 32, search 40, tap entries, tap values, flat state
+constexpr int PTT_FLAT_FLOATS = 32 + 32 + 32 + 40 + 4 * PTT_ENTRIES + PTT_ENTRIES + FLAT_STATE_FLOATS;
+
+struct PttFlatLds {
+    PttLds init;       // the initial frame's arrays (init_frame_ptt)
+    float *search;     // cdf of faces 0..30 ([30] = inf), then the midpoints of levels 1-3
+    float4 *entry;     // probe position and LUT entry
+    float *tap;        // tap values
+    const float *tab;  // the workgroup's tables
+};
+
+constexpr int DPP_ROW_NEWBCAST = 0x150;
+
+// check_point on the slot's lanes: wave_stop_begin's lane-parallel texels.
+__device__ __forceinline__ int slot_stop_end(const DevParams &P, const WaveTap &r) {
+    float acc = r.w * r.t;
+#pragma unroll
+    for (int k = 1; k < 8; ++k) acc = __builtin_fmaf(r.w, r.t, dpp0<DPP_ROW_SHR + 1>(acc));
+    acc = dpp0<DPP_ROW_NEWBCAST + 7>(acc);
+    if (acc == -1.0f) return CUSLINES_OUTSIDEIMAGE;
+    return (acc > P.tc_threshold) ? CUSLINES_TRACKPOINT : CUSLINES_ENDPOINT;
+}
+
+// Value of the lane I places below in the slot (rows of 16 joined); what the
+// lanes below I get is not used.
+template <int I>
+__device__ __forceinline__ float slot_shr(float v) {
+    if (I == 16) return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false)[0]);
+    const float r = dpp0<DPP_ROW_ROR + (I & 15)>(v);
+    const float x = __uint_as_float(
+        __builtin_amdgcn_permlane16_swap(__float_as_uint(r), __float_as_uint(r), false, false)[0]);
+    return ((threadIdx.x & 15) < I) ? x : r;
+}
+
+// norm3 without its range test (the caller tests the squares).
+__device__ __forceinline__ float norm3_raw(float &x, float &y, float &z) {
+    const float n2 = __builtin_fmaf(z, z, __builtin_fmaf(y, y, x * x));
+    const float inv = rsqrt_nr(n2);
+    x *= inv; y *= inv; z *= inv;
+    return n2;
+}
+
+// propagate_frame; the norms' range tests as one.
+__device__ __forceinline__ void propagate_frame_fast(const float *p, float *f, float *direc) {
+    float t[3], w[3], u[3], v[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        direc[i] = __builtin_fmaf(p[2], f[6 + i], __builtin_fmaf(p[1], f[3 + i], p[0] * f[i]));
+        t[i] = __builtin_fmaf(p[5], f[6 + i], __builtin_fmaf(p[4], f[3 + i], p[3] * f[i]));
+        w[i] = __builtin_fmaf(p[8], f[6 + i], __builtin_fmaf(p[7], f[3 + i], p[6] * f[i]));
+    }
+    const float nt = norm3_raw(t[0], t[1], t[2]);
+    u[0] = __builtin_fmaf(w[1], t[2], -(w[2] * t[1]));
+    u[1] = __builtin_fmaf(w[2], t[0], -(w[0] * t[2]));
+    u[2] = __builtin_fmaf(w[0], t[1], -(w[1] * t[0]));
+    const float nu = norm3_raw(u[0], u[1], u[2]);
+    v[0] = __builtin_fmaf(t[1], u[2], -(t[2] * u[1]));
+    v[1] = __builtin_fmaf(t[2], u[0], -(t[0] * u[2]));
+    v[2] = __builtin_fmaf(t[0], u[1], -(t[1] * u[0]));
+    const float nv = norm3_raw(v[0], v[1], v[2]);
+    const float lo = __builtin_elementwise_minimum(__builtin_elementwise_minimum(nt, nu), nv);
+    const float hi = __builtin_elementwise_maximum(__builtin_elementwise_maximum(nt, nu), nv);
+    float g[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) g[i] = f[i];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        f[i] = t[i]; f[3 + i] = u[i]; f[6 + i] = v[i];
+        // here, not inside the branch below: no copies at its end
+        asm volatile("" : "+v"(f[i]), "+v"(f[3 + i]), "+v"(f[6 + i]), "+v"(direc[i]));
+    }
+    if (__builtin_expect(!(lo > PTT_MIN_NORM2 && hi <= 3.40282347e+38f), 0)) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) f[i] = g[i];
+        propagate_frame(p, f, direc);
+    }
+}
+
+// The tangent alone (the last probe of a curve).
+__device__ __forceinline__ void propagate_tangent(const float *p, float *f, float *direc) {
+    float t[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        direc[i] = __builtin_fmaf(p[2], f[6 + i], __builtin_fmaf(p[1], f[3 + i], p[0] * f[i]));
+        t[i] = __builtin_fmaf(p[5], f[6 + i], __builtin_fmaf(p[4], f[3 + i], p[3] * f[i]));
+    }
+    norm3<0>(t[0], t[1], t[2]);
+    f[0] = t[0]; f[1] = t[1]; f[2] = t[2];
+}
+
+// Vertex phase of a sub-step on frame `fr` at (px, py, pz): the 24 supports
+// (0 below the cut) into S.init.vert_pdf, the tangent's tap into first_val.
+// `check`: the point's stop-map check, left over from the sub-step before,
+// is done under the frames.  1, 0 when no vertex passes, -1 when the check
+// ends the pass.
+__device__ __forceinline__ int ptt_vertices(const DevParams &P, const DevBufs &B, const PttFlatLds &S, const float *fr,
+                                            bool check, float px, float py, float pz, float *first_val) {
+    const int l = lane32();
+    const int Q = P.probe_quality;
+    const uint32_t lv0 = B.lut[lut_index(P, fr[0], fr[1], fr[2])];
+    const WaveTap stop = wave_stop_begin(P, B.stop, px, py, pz);
+    float f[9], p[9];
+    float x = px, y = py, z = pz;
+    const float4 pa = *reinterpret_cast<const float4 *>(S.tab + 12 * min(l, DISC_VERT_CNT - 1));
+    const float4 pb = *reinterpret_cast<const float4 *>(S.tab + 12 * min(l, DISC_VERT_CNT - 1) + 4);
+    p[0] = pa.x; p[1] = pa.y; p[2] = pa.z; p[3] = pa.w;
+    p[4] = pb.x; p[5] = pb.y; p[6] = pb.z; p[7] = pb.w;
+    p[8] = S.tab[12 * min(l, DISC_VERT_CNT - 1) + 8];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) f[i] = fr[i];
+    Tap t0;
+    float sup = 0.0f;
+    for (int g = 0; g < Q; g += PTT_GROUP) {
+        const int cnt = min(PTT_GROUP, Q - g);
+        if (l < DISC_VERT_CNT) {
+            // LUT entries of the last three probes, on their way
+            uint32_t lv1 = 0u, lv2 = 0u, lv3 = 0u;
+            for (int i = 0; i < cnt; ++i) {
+                float d[3];
+                if (g + i + 1 < Q) propagate_frame_fast(p, f, d); else propagate_tangent(p, f, d);
+                x += d[0]; y += d[1]; z += d[2];
+                const uint32_t nlv = B.lut[lut_index(P, f[0], f[1], f[2])];
+                float *e = reinterpret_cast<float *>(S.entry + i * DISC_VERT_CNT + l);
+                e[0] = x; e[1] = y; e[2] = z;
+                if (i >= 3) e[3 - 3 * 4 * DISC_VERT_CNT] = __uint_as_float(lv3);
+                lv3 = lv2; lv2 = lv1; lv1 = nlv;
+            }
+            float *e = reinterpret_cast<float *>(S.entry + (cnt - 1) * DISC_VERT_CNT + l);
+            if (cnt >= 3) e[3 - 2 * 4 * DISC_VERT_CNT] = __uint_as_float(lv3);
+            if (cnt >= 2) e[3 - 4 * DISC_VERT_CNT] = __uint_as_float(lv2);
+            e[3] = __uint_as_float(lv1);
+        }
+        if (g == 0) {
+            t0 = tap_begin(P, B, lv0, px, py, pz);
+            if (check && slot_stop_end(P, stop) != CUSLINES_TRACKPOINT) return -1;
+        }
+        WAVE_SYNC();
+        // the group's taps: entry 32 r + l in round r
+        const int ne = cnt * DISC_VERT_CNT;
+        uint32_t slow = 0u;  // rounds whose cell has no corner block
+        constexpr int BATCH = PTT_BATCH, ROUNDS = (PTT_ENTRIES + 31) / 32;
+#pragma unroll
+        for (int r0 = 0; r0 < ROUNDS; r0 += BATCH) {
+            Tap t[BATCH];
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) {
+                const int e = 32 * (r0 + u) + l;
+                const float4 q = S.entry[min(e, ne - 1)];
+                t[u] = tap_begin(P, B, __float_as_uint(q.w), q.x, q.y, q.z);
+            }
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) {
+                const int e = 32 * (r0 + u) + l;
+                if (e < ne) S.tap[e] = corner_blend(t[u].a, t[u].b, t[u].g, t[u].lo, t[u].hi);
+                if (!t[u].fast) slow |= 1u << (r0 + u);
+            }
+        }
+        if (half_ballot(slow != 0u)) {
+            for (int r = 0; r < ROUNDS; ++r) {
+                const int e = 32 * r + l;
+                if (((slow >> r) & 1u) && e < ne) {
+                    const float4 q = S.entry[e];
+                    const uint32_t lv = __float_as_uint(q.w);
+                    const int idx = (int)(lv & 0xffffu);
+                    const int tx = idx & (P.nx - 1), ty = (idx >> P.log2x) & (P.ny - 1), tz = idx >> (P.log2x + P.log2y);
+                    S.tap[e] = tiled_sample(P, B.data, (float)(tx * P.dimx) + q.x, (float)(ty * P.dimy) + q.y,
+                                            (float)(tz * P.dimz) + q.z, tx, ty, tz);
+                }
+            }
+        }
+        WAVE_SYNC();
+        if (g == 0) {
+            *first_val = tap_end(P, B, t0);
+            sup = *first_val;
+        }
+        if (l < DISC_VERT_CNT) {
+            float v[PTT_GROUP];
+#pragma unroll
+            for (int i = 0; i < PTT_GROUP; ++i) v[i] = S.tap[i * DISC_VERT_CNT + l];  // past cnt: not used
+#pragma unroll
+            for (int i = 0; i < PTT_GROUP; ++i) sup = (i < cnt) ? sup + v[i] : sup;
+        }
+        if (g + PTT_GROUP < Q) WAVE_SYNC();
+    }
+    const bool ok = l < DISC_VERT_CNT && !(sup < P.min_support_f);
+    S.init.vert_pdf[l] = ok ? sup : 0.0f;
+    const uint32_t any = half_ballot(ok);
+    WAVE_SYNC();
+    return any != 0u ? 1 : 0;
+}
+
+// Support of a rejection candidate, up to stop_at; ends early when lane 0's
+// candidate has passed.
+__device__ __forceinline__ float ptt_candidate(const DevParams &P, const DevBufs &B, float support, float px, float py,
+                                               float pz, float k1, float k2, const float *fr, float stop_at) {
+    uint32_t pass = half_ballot(support >= stop_at);
+    if (pass & 1u) return support;
+    float prop[9], pf[9], direc[3];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) pf[i] = fr[i];
+    prepare_propagator(k1, k2, P.probe_step, prop);
+    propagate_frame_fast(prop, pf, direc);
+    px += direc[0]; py += direc[1]; pz += direc[2];
+    uint32_t idx = B.lut[lut_index(P, pf[0], pf[1], pf[2])];
+    for (int i = 0; i < P.probe_quality; ++i) {
+        if (!(support >= stop_at)) {
+            const Tap t = tap_begin(P, B, idx, px, py, pz);
+            if (i + 1 < P.probe_quality) {
+                propagate_frame_fast(prop, pf, direc);
+                px += direc[0]; py += direc[1]; pz += direc[2];
+                idx = B.lut[lut_index(P, pf[0], pf[1], pf[2])];
+            }
+            support += tap_end(P, B, t);
+        }
+        pass = half_ballot(support >= stop_at);
+        if ((pass & 1u) || pass == 0xffffffffu) break;
+    }
+    return support;
+}
+
+// One sub-step (non-initial): 1 with the frame `fr` moved and the new
+// direction, 0 when there is none, -1 when the point's pending stop check
+// ends the pass.
+__device__ __forceinline__ int ptt_flat_substep(const DevParams &P, const DevBufs &B, const PttFlatLds &S, float *fr,
+                                                int face, bool check, Philox &rng, float px, float py, float pz,
+                                                float *nx, float *ny, float *nz) {
+    const int l = lane32();
+    float first_val;
+    const int vt = ptt_vertices(P, B, S, fr, check, px, py, pz, &first_val);
+    if (vt <= 0) return vt;
+    // face CDF (ptt_face_cdf): lane f < 31 holds face f; `face` packs its vertices
+    float c = 0.0f;
+    {
+        const float a = S.init.vert_pdf[face & 0xff], b = S.init.vert_pdf[(face >> 8) & 0xff],
+                    d = S.init.vert_pdf[face >> 16];
+        c = (a == 0.0f || b == 0.0f || d == 0.0f || l >= DISC_FACE_CNT) ? 0.0f : (a + b) + d;
+    }
+    {
+        float o = slot_shr<1>(c);
+        c = (l >= 1 && l < DISC_FACE_CNT) ? c + o : c;
+        o = slot_shr<2>(c);
+        c = (l >= 2 && l < DISC_FACE_CNT) ? c + o : c;
+        o = slot_shr<4>(c);
+        c = (l >= 4 && l < DISC_FACE_CNT) ? c + o : c;
+        o = slot_shr<8>(c);
+        c = (l >= 8 && l < DISC_FACE_CNT) ? c + o : c;
+        o = slot_shr<16>(c);
+        c = (l >= 16 && l < DISC_FACE_CNT) ? c + o : c;
+    }
+    // the search's order: 31 values, the last one's test always true, and
+    // the midpoints of levels 1-3 (15; 7, 23; 3, 11, 19, 27)
+    S.search[l] = (l >= DISC_FACE_CNT - 1) ? __builtin_inff() : c;
+    if ((l & 3) == 3 && l < 28) S.search[32 + (l >> 2)] = c;
+    const float last = shfl32(c, DISC_FACE_CNT - 1);
+    WAVE_SYNC();
+    if (last == 0.0f) return 0;
+    const float4 ma = *reinterpret_cast<const float4 *>(S.search + 32);      // cdf at 3, 7, 11, 15
+    const float4 mb = *reinterpret_cast<const float4 *>(S.search + 32 + 4);  // cdf at 19, 23, 27, -
+    const float stop_at = P.ptt_nonneg ? P.min_support_f : __builtin_inff();
+    for (int round = 0; round < 1024 / 32; ++round) {
+        float r1 = rng.uniform(), r2 = rng.uniform();
+        if (r1 + r2 > 1.0f) { r1 = 1.0f - r1; r2 = 1.0f - r2; }
+        const float tmp = rng.uniform() * last;
+        // ptt_substep's binary search over [0, 30]
+        const bool l1 = ma.w >= tmp;
+        const bool l2 = (l1 ? ma.y : mb.y) >= tmp;
+        const float m3 = l1 ? (l2 ? ma.x : ma.z) : (l2 ? mb.x : mb.z);
+        const bool l3 = m3 >= tmp;
+        const int base = (l1 ? 0 : 16) + (l2 ? 0 : 8) + (l3 ? 0 : 4);
+        const float4 q = *reinterpret_cast<const float4 *>(S.search + base);
+        const bool l4 = q.y >= tmp;
+        const bool l5 = (l4 ? q.x : q.z) >= tmp;
+        const int jj = min(base + (l4 ? 0 : 2) + (l5 ? 0 : 1), DISC_FACE_CNT - 1);
+        const float4 fa = *reinterpret_cast<const float4 *>(S.tab + DISC_VERT_CNT * 12 + 8 * jj);
+        const float2 fb = *reinterpret_cast<const float2 *>(S.tab + DISC_VERT_CNT * 12 + 8 * jj + 4);
+        float k1 = __builtin_fmaf(r2, fa.z, __builtin_fmaf(r1, fa.y, fa.x));
+        float k2 = __builtin_fmaf(r2, fb.y, __builtin_fmaf(r1, fb.x, fa.w));
+        const float sup = ptt_candidate(P, B, first_val, px, py, pz, k1, k2, fr, stop_at);
+        const uint32_t msk = half_ballot(sup >= P.min_support_f);
+        if (msk == 0u) continue;
+        const int win = __ffs(msk) - 1;
+        k1 = shfl32(k1, win);
+        k2 = shfl32(k2, win);
+        float prop[9], d[3];
+        prepare_propagator(k1, k2, P.ptt_sub_step, prop);
+        propagate_frame_fast(prop, fr, d);
+        norm3<0>(d[0], d[1], d[2]);
+        *nx = d[0]; *ny = d[1]; *nz = d[2];
+        return 1;
+    }
+    return 0;
+}
+
+// flat_slot's loop for a plain PTT slot.
+__device__ void flat_slot_ptt(const DevParams &P, const DevBufs &B, const PttFlatLds &S, float *st,
+                              const float *__restrict__ seeds, int nseeds, int rng_chunk,
+                              const int *__restrict__ offsets, const int *__restrict__ dirs,
+                              int *__restrict__ sline_seed, int *__restrict__ sline_len, float *__restrict__ sline,
+                              const int *__restrict__ order, int *__restrict__ work) {
+    const int l = lane32();
+    const int xcd = blockIdx.x & (QUEUES - 1);
+    const int step_frac = P.step_frac, MAXL = P.max_sline_len;
+    const int nsub_max = MAXL * step_frac;
+    const double sub = P.step_d / (double)step_frac;
+    const size_t slot_f = (size_t)2 * MAXL * 3;
+    int *si = reinterpret_cast<int *>(st);  // s, ndir, next direction, offsets[s], slot, nb
+    float *sf = st + 8;                     // seed point [0..2], direction [3..5]
+    if (l == 0) { si[1] = 0; si[2] = 0; }
+    WAVE_SYNC();
+    const int fl = min(l, DISC_FACE_CNT - 1);
+    const int face = c_disc_face[fl * 3] | (c_disc_face[fl * 3 + 1] << 8) | (c_disc_face[fl * 3 + 2] << 16);
+    Philox rng;
+    int qk = 0;
+    bool have = false, check = false;
+    int pass = 0, i = 1, ri = 1, qi = 0;  // step i = qi * step_frac + ri
+    float px = 0.0f, py = 0.0f, pz = 0.0f;
+    float fr[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) fr[k] = 0.0f;
+    float *sl = sline;
+    for (;;) {
+        if (!have) {
+            // the next direction of this seed, or of the next seeds
+            while (qk < QUEUES) {
+                const int di = si[2];
+                if (di >= si[1]) {
+                    const int qx = (xcd + qk) & (QUEUES - 1);
+                    const int lo = (int)((long long)nseeds * qx / QUEUES);
+                    const int hi = (int)((long long)nseeds * (qx + 1) / QUEUES);
+                    int q = 0;
+                    if (l == 0) q = atomicAdd(work + qx, 1);
+                    q = shfl32(q, 0);
+                    if (lo + q >= hi) { ++qk; continue; }
+                    const int s = order[lo + q];
+                    const int nd = (P.slot_cap > 0 && offsets[s + 1] > P.slot_cap) ? 0 : offsets[s + 1] - offsets[s];
+                    rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo, (uint64_t)32 * (uint64_t)(s % rng_chunk) + l + 1);
+                    WAVE_SYNC();
+                    if (l == 0) {
+                        si[0] = s; si[1] = nd; si[2] = 0; si[3] = offsets[s];
+                        sf[0] = seeds[3 * s]; sf[1] = seeds[3 * s + 1]; sf[2] = seeds[3 * s + 2];
+                    }
+                    WAVE_SYNC();
+                    continue;
+                }
+                const int s = si[0], off = si[3] + di;
+                const float sx = sf[0], sy = sf[1], sz = sf[2];
+                const int vi = dirs[(size_t)s * P.nverts + di];
+                const float fx = B.verts[3 * vi], fy = B.verts[3 * vi + 1], fz = B.verts[3 * vi + 2];
+                float *cur = sline + (size_t)off * slot_f;
+                WAVE_SYNC();
+                if (l == 0) {
+                    sline_seed[off] = s;
+                    si[2] = di + 1; si[4] = off;
+                    sf[3] = fx; sf[4] = fy; sf[5] = fz;
+                }
+                WAVE_SYNC();
+                PttLds in = S.init;
+                if (!init_frame_ptt(P, B, in, rng, fx, fy, fz, sx, sy, sz)) {
+                    if (l == 0) {
+                        sline_len[off] = 1;
+                        cur[0] = sx; cur[1] = sy; cur[2] = sz;
+                    }
+                    continue;
+                }
+                // backward pass on the frame at [0..8]
+                pass = 0;
+                px = sx; py = sy; pz = sz;
+#pragma unroll
+                for (int k = 0; k < 9; ++k) fr[k] = S.init.frame[k];
+                sl = cur;
+                if (l == 0) { sl[0] = px; sl[1] = py; sl[2] = pz; }
+                i = 1; qi = (step_frac == 1) ? 1 : 0; ri = (step_frac == 1) ? 0 : 1;
+                have = true;
+                break;
+            }
+            if (!have) break;  // the queues are empty
+        }
+        // One sub-step of the pass (tracker's loop body).  With `check` the
+        // point is that of step i, already moved and stored, and its stop
+        // check comes with the next sub-step; it passes before i counts on.
+        const int ni = check ? i + 1 : i;  // the step to take now
+        bool end = true;
+        if (ni < nsub_max) {
+            float dx = 0.0f, dy = 0.0f, dz = 0.0f;
+            const int nd = ptt_flat_substep(P, B, S, fr, face, check, rng, px, py, pz, &dx, &dy, &dz);
+            if (check && nd >= 0) {
+                ++i;
+                if (++ri == step_frac) { ri = 0; ++qi; }
+            }
+            if (nd > 0) {
+                px = (float)__builtin_fma((double)(dx / 1.0f), sub, (double)px);
+                py = (float)__builtin_fma((double)(dy / 1.0f), sub, (double)py);
+                pz = (float)__builtin_fma((double)(dz / 1.0f), sub, (double)pz);
+                if (l == 0 && ri == 0) {
+                    float *o = sl + 3 * (size_t)qi;
+                    o[0] = px; o[1] = py; o[2] = pz;
+                }
+                check = true;
+                end = false;
+            }
+        } else if (check && slot_stop_end(P, wave_stop_begin(P, B.stop, px, py, pz)) == CUSLINES_TRACKPOINT) {
+            ++i;
+            if (++ri == step_frac) { ri = 0; ++qi; }
+        }
+        if (!end) continue;
+        check = false;
+        // the pass ends at step i (tracker's tail)
+        int nsteps = qi;
+        if (ri != 0 && i < step_frac * (MAXL - 1)) {
+            ++nsteps;
+            if (l == 0) {
+                float *o = sl + 3 * (size_t)nsteps;
+                o[0] = px; o[1] = py; o[2] = pz;
+            }
+        }
+        const int off = si[4];
+        float *cur = sline + (size_t)off * slot_f;
+        if (pass == 0) {
+            const int nb = nsteps;
+            MEM_SYNC();
+            for (int j = l; j < nb / 2; j += 32) {
+                float *a = cur + 3 * (size_t)j, *b = cur + 3 * (size_t)(nb - 1 - j);
+                const float a0 = a[0], a1 = a[1], a2 = a[2];
+                a[0] = b[0]; a[1] = b[1]; a[2] = b[2];
+                b[0] = a0; b[1] = a1; b[2] = a2;
+            }
+            MEM_SYNC();
+            if (l == 0) si[5] = nb;
+            // forward pass on the frame at [9..17], from the seed point at index nb - 1
+            pass = 1;
+            px = sf[0]; py = sf[1]; pz = sf[2];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) fr[k] = S.init.frame[9 + k];
+            sl = cur + 3 * (size_t)(nb - 1);
+            if (l == 0) { sl[0] = px; sl[1] = py; sl[2] = pz; }
+            i = 1; qi = (step_frac == 1) ? 1 : 0; ri = (step_frac == 1) ? 0 : 1;
+            WAVE_SYNC();
+        } else {
+            if (l == 0) sline_len[off] = si[5] - 1 + nsteps;
+            have = false;
+        }
+    }
+}
+
+__global__ void __launch_bounds__(256, PTT_WAVES)
+    phase2_ptt_kernel(DevParams P, DevBufs B, const float *__restrict__ seeds, int nseeds, int rng_chunk,
+                      const int *__restrict__ offsets, const int *__restrict__ dirs, int *__restrict__ sline_seed,
+                      int *__restrict__ sline_len, float *__restrict__ sline, const int *__restrict__ order,
+                      int *__restrict__ work) {
+    extern __shared__ float4 smem4[];
+    float *smem = reinterpret_cast<float *>(smem4);
+    for (int i = threadIdx.x; i < DISC_VERT_CNT * 12; i += blockDim.x) {
+        const int v = i / 12, k = i - 12 * v;
+        smem[i] = (k < 9) ? B.vprop[9 * v + k] : 0.0f;
+    }
+    // per face: the curvatures of vertex 0 and the two edges from it
+    for (int f = threadIdx.x; f < 32; f += blockDim.x) {
+        float *o = smem + DISC_VERT_CNT * 12 + 8 * f;
+        const int g = min(f, DISC_FACE_CNT - 1);
+        const float *vk = B.vprop + VPROP_K;
+        const int f0 = c_disc_face[g * 3], f1 = c_disc_face[g * 3 + 1], f2 = c_disc_face[g * 3 + 2];
+        o[0] = vk[2 * f0];
+        o[1] = vk[2 * f1] - vk[2 * f0];
+        o[2] = vk[2 * f2] - vk[2 * f0];
+        o[3] = vk[2 * f0 + 1];
+        o[4] = vk[2 * f1 + 1] - vk[2 * f0 + 1];
+        o[5] = vk[2 * f2 + 1] - vk[2 * f0 + 1];
+        o[6] = o[7] = 0.0f;
+    }
+    __syncthreads();
+    float *base = smem + PTT_TAB_FLOATS + (threadIdx.x >> 5) * PTT_FLAT_FLOATS;
+    PttFlatLds S;
+    S.init.frame = base;
+    S.init.vert_pdf = base + 32;
+    S.init.face_cdf = base + 64;
+    S.init.act = nullptr;
+    S.search = base + 96;
+    S.entry = reinterpret_cast<float4 *>(base + 136);
+    S.tap = base + 136 + 4 * PTT_ENTRIES;
+    S.tab = smem;
+    flat_slot_ptt(P, B, S, base + PTT_FLAT_FLOATS - FLAT_STATE_FLOATS, seeds, nseeds, rng_chunk, offsets, dirs,
+                  sline_seed, sline_len, sline, order, work);
+}
+
 // One seed per 32-lane slot, static assignment.
 template <int MODEL, int V = 0>
 __global__ void __launch_bounds__(256) phase2_kernel(DevParams P, DevBufs B, const float *__restrict__ seeds,
@@ -3318,15 +3846,14 @@ __global__ void __launch_bounds__(256) phase2_kernel(DevParams P, DevBufs B, con
 // Plain PTT is held to 128 VGPRs (4 waves per SIMD): the few spills cost less
 // than the latency hiding gained (+8% at 200k seeds).  Bootstrap likewise
 // (4 waves per SIMD, which its 5 KB of LDS per slot allows: +13% CSA).  The
-// flat PTT loop (V == 4) needs about 170 VGPRs and at 128 spills inside its
-// loop, so it runs at 3 waves per SIMD (168 VGPRs, no spills); its learned
-// form (V == 5) likewise, in 768-thread workgroups (3 waves per SIMD in one
-// workgroup, so one staged copy of the network serves 24 slots).
+// flat loop of the learned proposal (V == 5) needs about 170 VGPRs and at 128
+// spills inside its loop, so it runs at 3 waves per SIMD (168 VGPRs), in
+// 768-thread workgroups (one staged copy of the network serves 24 slots).
 template <int MODEL, int V = 0>
 __global__ void __launch_bounds__((MODEL == CUSLINES_PTT && V == 1)   ? 512
                                   : (MODEL == CUSLINES_PTT && V == 5) ? 768
                                                                       : 256,
-                                  (MODEL == CUSLINES_PTT && (V == 4 || V == 5)) ? 3
+                                  (MODEL == CUSLINES_PTT && V == 5) ? 3
                                   : (MODEL == CUSLINES_PTT && V != 2)           ? 4
                                                                                 : (MODEL <= CUSLINES_PROB ? 4 : 1))
     phase2_queue_kernel(DevParams P, DevBufs B, const float *__restrict__ seeds,
@@ -4617,20 +5144,15 @@ static int launch_phase2_v(cuslines_tracker *t, const float *seeds, int n, int c
     return CUSLINES_OK;
 }
 
-// Probabilistic phase 2 with the cell in registers: NCH chunks of 256
-// channels.  Work queue and spatial order as launch_phase2_v; one wave per
-// workgroup, so that few seeds spread over the CUs.
-template <int NCH>
-static int launch_prob(cuslines_tracker *t, const float *seeds, int n, int chunk, const int *offsets, const int *dirs,
-                       int *sseed, int *slen, float *sl, int *ws) {
+// A persistent queue kernel over the spatial seed order, as launch_phase2_v:
+// `threads` a workgroup, `nslots` seed slots in it, `lds` bytes.
+template <typename K>
+static int launch_queue(cuslines_tracker *t, K kernel, int threads, int nslots, size_t lds, const float *seeds, int n,
+                        int chunk, const int *offsets, const int *dirs, int *sseed, int *slen, float *sl, int *ws) {
     const DevParams &d = t->dp;
-    const int threads = t->threads > 0 ? t->threads : 64;
-    const int nslots = threads / 64;
-    const size_t lds = sizeof(float) * (3 * 256 * NCH + (size_t)nslots * prob_slot_floats(NCH));
-    const void *kfn = (const void *)phase2_prob_kernel<NCH>;
-    HIPC(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    HIPC(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int per_cu = 0;
-    HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, threads, lds));
+    HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)kernel, threads, lds));
     if (per_cu < 1) per_cu = 1;
     if (t->blocks_per_cu > 0 && t->blocks_per_cu < per_cu) per_cu = t->blocks_per_cu;
     long long grid = (long long)per_cu * t->num_cu;
@@ -4640,12 +5162,33 @@ static int launch_prob(cuslines_tracker *t, const float *seeds, int n, int chunk
     int *order = nullptr;
     if (int rc = spatial_order(t, seeds, n, &order, ws)) return rc;
     hipLaunchKernelGGL(zero_ints, dim3(1), dim3(QUEUES), 0, t->stream, t->d_work, QUEUES);
-    hipLaunchKernelGGL(phase2_prob_kernel<NCH>, dim3((unsigned)grid), dim3(threads), lds, t->stream, d, bufs_of(t),
-                       seeds, n, chunk, offsets, dirs, sseed, slen, sl, order, t->d_work);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(threads), lds, t->stream, d, bufs_of(t), seeds, n, chunk,
+                       offsets, dirs, sseed, slen, sl, order, t->d_work);
     hipError_t e = hipGetLastError();
     if (!ws) (void)hipFreeAsync(order, t->stream);
-    if (e != hipSuccess) return fail(CUSLINES_EHIP, std::string("phase 2 (prob): ") + hipGetErrorString(e));
+    if (e != hipSuccess) return fail(CUSLINES_EHIP, std::string("phase 2: ") + hipGetErrorString(e));
     return CUSLINES_OK;
+}
+
+// Probabilistic phase 2 with the cell in registers: NCH chunks of 256
+// channels; one wave a workgroup, so that few seeds spread over the CUs.
+template <int NCH>
+static int launch_prob(cuslines_tracker *t, const float *seeds, int n, int chunk, const int *offsets, const int *dirs,
+                       int *sseed, int *slen, float *sl, int *ws) {
+    const int threads = t->threads > 0 ? t->threads : 64;
+    const int nslots = threads / 64;
+    const size_t lds = sizeof(float) * (3 * 256 * NCH + (size_t)nslots * prob_slot_floats(NCH));
+    return launch_queue(t, phase2_prob_kernel<NCH>, threads, nslots, lds, seeds, n, chunk, offsets, dirs, sseed, slen,
+                        sl, ws);
+}
+
+// Plain PTT phase 2; one wave a workgroup.
+static int launch_ptt(cuslines_tracker *t, const float *seeds, int n, int chunk, const int *offsets, const int *dirs,
+                      int *sseed, int *slen, float *sl, int *ws) {
+    const int threads = t->threads > 0 ? t->threads : 64;
+    const int nslots = threads / 32;
+    const size_t lds = sizeof(float) * (PTT_TAB_FLOATS + (size_t)nslots * PTT_FLAT_FLOATS);
+    return launch_queue(t, phase2_ptt_kernel, threads, nslots, lds, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
 }
 
 // Limits of the batched bootstrap kernel's tile counts per wave.
@@ -4723,6 +5266,8 @@ static int launch_phase2(cuslines_tracker *t, const float *seeds, int n, int chu
             return launch_phase2_v<MODEL, 3>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
         if (t->ptt_lanes > 0 && t->schedule != CUSLINES_SCHED_STATIC)
             return launch_ptt_groups(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
+        if (t->flat && t->schedule != CUSLINES_SCHED_STATIC)
+            return launch_ptt(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
     }
     if constexpr (MODEL == CUSLINES_PROB) {
         // a lane keeps 4 of a chunk's 256 channels, 8 corners each: 3 chunks fit the registers
@@ -4733,8 +5278,10 @@ static int launch_phase2(cuslines_tracker *t, const float *seeds, int n, int chu
             default: break;
         }
     }
-    if (t->flat && t->schedule != CUSLINES_SCHED_STATIC)
-        return launch_phase2_v<MODEL, 4>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
+    if constexpr (MODEL != CUSLINES_PTT) {
+        if (t->flat && t->schedule != CUSLINES_SCHED_STATIC)
+            return launch_phase2_v<MODEL, 4>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
+    }
     return launch_phase2_v<MODEL, 0>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
 }
 

@@ -150,8 +150,10 @@ struct Philox {
         uint32_t key0 = k0, key1 = k1;
 #pragma unroll
         for (int r = 0; r < 10; ++r) {
-            const uint32_t lo0 = 0xD2511F53u * x0, hi0 = __umulhi(0xD2511F53u, x0);
-            const uint32_t lo1 = 0xCD9E8D57u * x2, hi1 = __umulhi(0xCD9E8D57u, x2);
+            // one quarter-rate multiply each for both halves of the product
+            const uint64_t m0 = (uint64_t)0xD2511F53u * x0, m1 = (uint64_t)0xCD9E8D57u * x2;
+            const uint32_t lo0 = (uint32_t)m0, hi0 = (uint32_t)(m0 >> 32);
+            const uint32_t lo1 = (uint32_t)m1, hi1 = (uint32_t)(m1 >> 32);
             const uint32_t n0 = hi1 ^ x1 ^ key0, n2 = hi0 ^ x3 ^ key1;
             x0 = n0; x1 = lo1; x2 = n2; x3 = lo0;
             key0 += 0x9E3779B9u;
