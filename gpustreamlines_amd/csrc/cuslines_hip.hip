@@ -44,7 +44,10 @@ constexpr float CSA_C0 = 0.28209479177387814f;         // boot.cu:363
 constexpr int DISC_VERT_CNT = 24;                      // disc.h:20
 constexpr int DISC_FACE_CNT = 31;                      // disc.h:21
 constexpr int SORT_LAYERS = 15;
-constexpr int QUEUES = 8;  // persistent-queue counters, one per XCD
+constexpr int XCDS = 8;
+constexpr int SEED_CLASSES = 8;                          // by direction count; the last has none and is not queued
+constexpr int QUEUES = XCDS * (SEED_CLASSES - 1);        // persistent-queue counters, one per class and XCD
+constexpr int WORK_INTS = QUEUES + SEED_CLASSES;         // counters, then where each class starts in the seed order
 constexpr int VPROP_K = 24 * 9;                        // PTT table: curvatures after the 24 propagators
 constexpr int VPROP_FLOATS = VPROP_K + 2 * 24;
 
@@ -137,6 +140,29 @@ struct DevBufs {
     int *rec_count;
     unsigned long long *stats;  // learned sub-steps, fallbacks, plain sub-steps
 };
+
+// Queue k of an XCD's order: its counter and its range [lo, hi) of the seed
+// order.  The seeds with the most directions come first, each class in
+// spatial order and split in one range per XCD: an XCD drains its own range
+// (one region of the volume, for its L2), helps with the others', and goes on
+// to the next class.  A seed is tracked by one slot, direction after
+// direction on one random stream, and most of a run of a few seeds per slot
+// is the wait for the seeds that take longest; those now start first
+// (25,000 seeds on 6,144 slots of equal speed: 3,284 instead of 4,376 steps;
+// the longest seed has 3,284).
+struct QueueRange {
+    int counter, lo, hi;
+};
+
+__device__ __forceinline__ QueueRange queue_range(const int *work, int k) {
+    const int cls = k / XCDS, x = ((int)blockIdx.x + k) & (XCDS - 1);
+    const int a = work[QUEUES + cls], b = work[QUEUES + cls + 1];
+    QueueRange q;
+    q.counter = cls * XCDS + x;
+    q.lo = a + (int)((long long)(b - a) * x / XCDS);
+    q.hi = a + (int)((long long)(b - a) * (x + 1) / XCDS);
+    return q;
+}
 
 // -------------------------------------------------------------------------
 // Sorting, scans and peak extraction (per half-wave)
@@ -2192,7 +2218,6 @@ __device__ void flat_group_ptt(const DevParams &P, const DevBufs &B, const PttCo
                                const int *__restrict__ order, int *__restrict__ work) {
     using G = Grp<L>;
     const int p = G::lane();
-    const int xcd = blockIdx.x & (QUEUES - 1);
     const int step_frac = P.step_frac, MAXL = P.max_sline_len;
     const int nsub_max = MAXL * step_frac;
     const double sub = P.step_d / (double)step_frac;
@@ -2214,11 +2239,10 @@ __device__ void flat_group_ptt(const DevParams &P, const DevBufs &B, const PttCo
             while (qk < QUEUES) {
                 const int di = si[2];
                 if (di >= si[1]) {
-                    const int qx = (xcd + qk) & (QUEUES - 1);
-                    const int lo = (int)((long long)nseeds * qx / QUEUES);
-                    const int hi = (int)((long long)nseeds * (qx + 1) / QUEUES);
+                    const QueueRange qr = queue_range(work, qk);
+                    const int lo = qr.lo, hi = qr.hi;
                     int q = 0;
-                    if (p == 0) q = atomicAdd(work + qx, 1);
+                    if (p == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
                     q = G::shfl(q, 0);
                     if (lo + q >= hi) { ++qk; continue; }
                     const int s = order ? order[lo + q] : lo + q;
@@ -2603,7 +2627,6 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
     constexpr bool PTT = MODEL == CUSLINES_PTT;
     static_assert(PTT == LEARNED, "plain PTT: flat_slot_ptt");
     const int l = lane32();
-    const int xcd = blockIdx.x & (QUEUES - 1);
     const int step_frac = PTT ? P.step_frac : 1, MAXL = P.max_sline_len;
     const int nsub_max = MAXL * step_frac;
     const double sub = P.step_d / (double)step_frac;
@@ -2629,11 +2652,10 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
             while (qk < QUEUES) {
                 const int di = si[2];
                 if (di >= si[1]) {
-                    const int qx = (xcd + qk) & (QUEUES - 1);
-                    const int lo = (int)((long long)nseeds * qx / QUEUES);
-                    const int hi = (int)((long long)nseeds * (qx + 1) / QUEUES);
+                    const QueueRange qr = queue_range(work, qk);
+                    const int lo = qr.lo, hi = qr.hi;
                     int q = 0;
-                    if (l == 0) q = atomicAdd(work + qx, 1);
+                    if (l == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
                     q = shfl32(q, 0);
                     if (lo + q >= hi) { ++qk; continue; }
                     const int s = order ? order[lo + q] : lo + q;
@@ -3160,7 +3182,6 @@ __device__ void flat_wave_prob(const DevParams &P, const DevBufs &B, const float
                                int *__restrict__ sline_seed, int *__restrict__ sline_len, float *__restrict__ sline,
                                const int *__restrict__ order, int *__restrict__ work) {
     const int l = threadIdx.x & 63;
-    const int xcd = blockIdx.x & (QUEUES - 1);
     const int MAXL = P.max_sline_len;
     const double sub = P.step_d;
     const size_t slot_f = (size_t)2 * MAXL * 3;
@@ -3189,11 +3210,10 @@ __device__ void flat_wave_prob(const DevParams &P, const DevBufs &B, const float
         if (!have) {
             // the next direction of this seed, or of the next seeds
             while (di >= ndir && qk < QUEUES) {
-                const int qx = (xcd + qk) & (QUEUES - 1);
-                const int lo = (int)((long long)nseeds * qx / QUEUES);
-                const int hi = (int)((long long)nseeds * (qx + 1) / QUEUES);
+                const QueueRange qr = queue_range(work, qk);
+                const int lo = qr.lo, hi = qr.hi;
                 int q = 0;
-                if (l == 0) q = atomicAdd(work + qx, 1);
+                if (l == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
                 q = __builtin_amdgcn_readfirstlane(q);
                 if (lo + q >= hi) { ++qk; continue; }
                 s = __builtin_amdgcn_readfirstlane(order[lo + q]);
@@ -3627,7 +3647,6 @@ __device__ void flat_slot_ptt(const DevParams &P, const DevBufs &B, const PttFla
                               int *__restrict__ sline_seed, int *__restrict__ sline_len, float *__restrict__ sline,
                               const int *__restrict__ order, int *__restrict__ work) {
     const int l = lane32();
-    const int xcd = blockIdx.x & (QUEUES - 1);
     const int step_frac = P.step_frac, MAXL = P.max_sline_len;
     const int nsub_max = MAXL * step_frac;
     const double sub = P.step_d / (double)step_frac;
@@ -3653,11 +3672,10 @@ __device__ void flat_slot_ptt(const DevParams &P, const DevBufs &B, const PttFla
             while (qk < QUEUES) {
                 const int di = si[2];
                 if (di >= si[1]) {
-                    const int qx = (xcd + qk) & (QUEUES - 1);
-                    const int lo = (int)((long long)nseeds * qx / QUEUES);
-                    const int hi = (int)((long long)nseeds * (qx + 1) / QUEUES);
+                    const QueueRange qr = queue_range(work, qk);
+                    const int lo = qr.lo, hi = qr.hi;
                     int q = 0;
-                    if (l == 0) q = atomicAdd(work + qx, 1);
+                    if (l == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
                     q = shfl32(q, 0);
                     if (lo + q >= hi) { ++qk; continue; }
                     const int s = order[lo + q];
@@ -3886,14 +3904,12 @@ __global__ void __launch_bounds__((MODEL == CUSLINES_PTT && V == 1)   ? 512
     // Workgroups are dispatched to the 8 XCDs round-robin.  Each XCD first
     // drains its own eighth of the (spatially sorted) seed order, so an XCD's
     // L2 serves one region of the volume, then helps with the others.
-    const int xcd = blockIdx.x & (QUEUES - 1);
     for (int k = 0; k < QUEUES; ++k) {
-        const int qx = (xcd + k) & (QUEUES - 1);
-        const int lo = (int)((long long)nseeds * qx / QUEUES);
-        const int hi = (int)((long long)nseeds * (qx + 1) / QUEUES);
+        const QueueRange qr = queue_range(work, k);
+        const int lo = qr.lo, hi = qr.hi;
         for (;;) {
             int q = 0;
-            if (l == 0) q = atomicAdd(work + qx, 1);
+            if (l == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
             q = shfl32(q, 0);
             if (lo + q >= hi) break;
             const int s = order ? order[lo + q] : lo + q;
@@ -4165,13 +4181,11 @@ __device__ void bb_next_seed(const DevParams &P, const DevBufs &B, BbSlot &st, P
                              const int *__restrict__ dirs, const int *__restrict__ order, int *__restrict__ work,
                              float *__restrict__ sline) {
     const int l = lane32();
-    const int xcd = blockIdx.x & (QUEUES - 1);
     while (st.qk < QUEUES) {
-        const int qx = (xcd + st.qk) & (QUEUES - 1);
-        const int lo = (int)((long long)nseeds * qx / QUEUES);
-        const int hi = (int)((long long)nseeds * (qx + 1) / QUEUES);
+        const QueueRange qr = queue_range(work, st.qk);
+        const int lo = qr.lo, hi = qr.hi;
         int q = 0;
-        if (l == 0) q = atomicAdd(work + qx, 1);
+        if (l == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
         q = shfl32(q, 0);
         if (lo + q >= hi) { ++st.qk; continue; }
         const int s = order ? order[lo + q] : lo + q;
@@ -4417,7 +4431,7 @@ __global__ void zero_scalar(TO *p) {
     *p = 0;
 }
 
-// Spatial processing order of the persistent queue: seeds bucketed by the
+// Processing order of the persistent queue: seeds bucketed by class and by the
 // Morton code of their 2^brick_log2-voxel brick (counting sort).
 __device__ __forceinline__ uint32_t spread3(uint32_t v) {  // bits 0..9 to every third bit
     v &= 0x3ffu;
@@ -4428,8 +4442,14 @@ __device__ __forceinline__ uint32_t spread3(uint32_t v) {  // bits 0..9 to every
     return v;
 }
 
-__global__ void seed_keys(DevParams P, const float *__restrict__ seeds, int n, int brick_log2, int *__restrict__ key,
-                          int *__restrict__ count) {
+// Class of a seed with n directions: the more, the earlier.
+__device__ __forceinline__ int seed_class(int n) {
+    if (n >= 8) return 0;
+    return (n >= 6) ? 1 : (n >= 1) ? 7 - n : SEED_CLASSES - 1;
+}
+
+__global__ void seed_keys(DevParams P, const float *__restrict__ seeds, const int *__restrict__ offsets, int n,
+                          int brick_log2, int nbrick, int *__restrict__ key, int *__restrict__ count) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     uint32_t c[3];
@@ -4439,9 +4459,16 @@ __global__ void seed_keys(DevParams P, const float *__restrict__ seeds, int n, i
         const int i = (f != f || f < 0.0f) ? 0 : (f > (float)(dims[a] - 1) ? dims[a] - 1 : (int)f);
         c[a] = (uint32_t)i >> brick_log2;
     }
-    const int k = (int)(spread3(c[0]) | (spread3(c[1]) << 1) | (spread3(c[2]) << 2));
+    const int k = seed_class(offsets[s + 1] - offsets[s]) * nbrick +
+                  (int)(spread3(c[0]) | (spread3(c[1]) << 1) | (spread3(c[2]) << 2));
     key[s] = k;
     atomicAdd(count + k, 1);
+}
+
+// Counters at zero and the classes' starts in the seed order.
+__global__ void queue_init(int *__restrict__ work, const int *__restrict__ start, int nbrick) {
+    const int i = threadIdx.x;
+    if (i < WORK_INTS) work[i] = (i < QUEUES) ? 0 : start[(i - QUEUES) * nbrick];
 }
 
 __global__ void seed_scatter(const int *__restrict__ key, int n, const int *__restrict__ start, int *__restrict__ cursor,
@@ -4863,7 +4890,7 @@ struct cuslines_tracker {
     int *d_b0 = nullptr, *d_dwi = nullptr;
     uint32_t *d_lut = nullptr;
     std::vector<uint16_t> rank_vertex;  // PTT: vertex of each direction rank (corner-block order)
-    int *d_work = nullptr;      // work-queue counters of the persistent phase-2 kernels (QUEUES)
+    int *d_work = nullptr;      // work-queue counters and class starts of the persistent phase-2 kernels (WORK_INTS)
     void *scratch = nullptr;    // device address of this device's `scratch` array
     float *d_blocks = nullptr;  // PTT corner blocks
     int use_blocks = 1;
@@ -4982,7 +5009,7 @@ static int launch_phase1(cuslines_tracker *t, const float *seeds, int n, int chu
     return CUSLINES_OK;
 }
 
-static int spatial_order(cuslines_tracker *t, const float *seeds, int n, int **order, int *ws);
+static int spatial_order(cuslines_tracker *t, const float *seeds, const int *offsets, int n, int **order, int *ws);
 
 // PTT with L lanes per seed: with flat stepping (t->flat, the default) the
 // flat grouped kernel over the XCD-ordered queues of the spatial seed order
@@ -5005,8 +5032,8 @@ static int launch_ptt_l(cuslines_tracker *t, int threads, const float *seeds, in
     if (grid < 1) grid = 1;
     int *order = nullptr;
     if (flat)
-        if (int rc = spatial_order(t, seeds, n, &order, ws)) return rc;
-    hipLaunchKernelGGL(zero_ints, dim3(1), dim3(QUEUES), 0, t->stream, t->d_work, QUEUES);
+        if (int rc = spatial_order(t, seeds, offsets, n, &order, ws)) return rc;
+    if (!flat) hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, t->stream, t->d_work, 1);
     if (flat)
         hipLaunchKernelGGL(phase2_ptt_flat_kernel<L>, dim3((unsigned)grid), dim3(threads), lds, t->stream, d,
                            bufs_of(t), seeds, n, chunk, offsets, dirs, sseed, slen, sl, order, t->d_work);
@@ -5032,17 +5059,17 @@ static int launch_ptt_groups(cuslines_tracker *t, const float *seeds, int n, int
 template <typename TO>
 static int run_scan(cuslines_tracker *t, const int *in, int n, TO *out, TO *bsum_ws = nullptr);
 
-// Buckets of the spatial seed order: 4-voxel bricks (coarser when a
-// dimension exceeds 512 voxels), at most 2^21 of them.
+// Buckets of the seed order: 4-voxel bricks (coarser when a dimension
+// exceeds 256 voxels), at most 2^18 of them in each of the 8 classes.
 static int order_buckets(const DevParams &d, int *brick_log2_out) {
     int mx = d.dimx > d.dimy ? d.dimx : d.dimy;
     mx = mx > d.dimz ? mx : d.dimz;
     int brick_log2 = 2;
-    while (((mx - 1) >> brick_log2) >= 128) ++brick_log2;
+    while (((mx - 1) >> brick_log2) >= 64) ++brick_log2;
     int bits = 0;
     while ((1 << bits) <= ((mx - 1) >> brick_log2)) ++bits;
     *brick_log2_out = brick_log2;
-    return 1 << (3 * bits);
+    return SEED_CLASSES << (3 * bits);
 }
 
 // ints of the seed-order workspace: order and keys (n each), bucket counts
@@ -5051,11 +5078,12 @@ static size_t order_ws_ints(int n, int nb) {
     return 2 * (size_t)n + 2 * (size_t)nb + 1 + (size_t)((nb + 1023) / 1024);
 }
 
-// Seeds in Morton order of their brick, by a counting sort on the tracker's
-// stream.  With `ws` (order_ws_ints(n, nb) ints of device memory) every
+// Seeds by class and, in a class, in Morton order of their brick, by a counting
+// sort on the tracker's stream; the queue's counters and class starts in
+// t->d_work.  With `ws` (order_ws_ints(n, nb) ints of device memory) every
 // buffer is carved from it and *order points into it; without, they are
 // stream-ordered allocations and the caller frees *order with hipFreeAsync.
-static int spatial_order(cuslines_tracker *t, const float *seeds, int n, int **order, int *ws) {
+static int spatial_order(cuslines_tracker *t, const float *seeds, const int *offsets, int n, int **order, int *ws) {
     const DevParams &d = t->dp;
     int brick_log2 = 0;
     const int nb = order_buckets(d, &brick_log2);
@@ -5081,11 +5109,13 @@ static int spatial_order(cuslines_tracker *t, const float *seeds, int n, int **o
     }
     const dim3 gb((unsigned)((nb + 255) / 256)), gs((unsigned)((n + 255) / 256));
     hipLaunchKernelGGL(zero_ints, gb, dim3(256), 0, t->stream, count, nb);
-    hipLaunchKernelGGL(seed_keys, gs, dim3(256), 0, t->stream, d, seeds, n, brick_log2, key, count);
+    hipLaunchKernelGGL(seed_keys, gs, dim3(256), 0, t->stream, d, seeds, offsets, n, brick_log2, nb / SEED_CLASSES, key,
+                       count);
     int rc = run_scan<int>(t, count, nb, start, bsum);
     if (rc == CUSLINES_OK) {
         hipLaunchKernelGGL(zero_ints, gb, dim3(256), 0, t->stream, count, nb);
         hipLaunchKernelGGL(seed_scatter, gs, dim3(256), 0, t->stream, key, n, start, count, *order);
+        hipLaunchKernelGGL(queue_init, dim3(1), dim3(64), 0, t->stream, t->d_work, start, nb / SEED_CLASSES);
     }
     hipError_t e = hipGetLastError();
     if (!ws) {
@@ -5134,8 +5164,7 @@ static int launch_phase2_v(cuslines_tracker *t, const float *seeds, int n, int c
     if (grid > need) grid = need;
     if (grid < 1) grid = 1;
     int *order = nullptr;
-    if (int rc = spatial_order(t, seeds, n, &order, ws)) return rc;
-    hipLaunchKernelGGL(zero_ints, dim3(1), dim3(QUEUES), 0, t->stream, t->d_work, QUEUES);
+    if (int rc = spatial_order(t, seeds, offsets, n, &order, ws)) return rc;
     hipLaunchKernelGGL((phase2_queue_kernel<MODEL, V>), dim3((unsigned)grid), dim3(threads), lds, t->stream, d,
                        bufs_of(t), seeds, n, chunk, offsets, dirs, sseed, slen, sl, order, t->d_work);
     hipError_t e = hipGetLastError();
@@ -5160,8 +5189,7 @@ static int launch_queue(cuslines_tracker *t, K kernel, int threads, int nslots, 
     if (grid > need) grid = need;
     if (grid < 1) grid = 1;
     int *order = nullptr;
-    if (int rc = spatial_order(t, seeds, n, &order, ws)) return rc;
-    hipLaunchKernelGGL(zero_ints, dim3(1), dim3(QUEUES), 0, t->stream, t->d_work, QUEUES);
+    if (int rc = spatial_order(t, seeds, offsets, n, &order, ws)) return rc;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(threads), lds, t->stream, d, bufs_of(t), seeds, n, chunk,
                        offsets, dirs, sseed, slen, sl, order, t->d_work);
     hipError_t e = hipGetLastError();
@@ -5226,8 +5254,7 @@ static int launch_boot_batch(cuslines_tracker *t, const float *seeds, int n, int
         HIPC(hipMemsetAsync(t->d_stats, 0, 4 * sizeof(unsigned long long), t->stream));
     }
     int *order = nullptr;
-    if (int rc = spatial_order(t, seeds, n, &order, ws)) return rc;
-    hipLaunchKernelGGL(zero_ints, dim3(1), dim3(QUEUES), 0, t->stream, t->d_work, QUEUES);
+    if (int rc = spatial_order(t, seeds, offsets, n, &order, ws)) return rc;
     const DevBufs bb = bufs_of(t);
     const dim3 g((unsigned)grid), b(BB_THREADS);
     if (t->boot_occ == 4 && lr)
@@ -5500,7 +5527,7 @@ int cuslines_tracker_create(const cuslines_params *p, int device, cuslines_track
         delete t;
         return fail(CUSLINES_EHIP, std::string("hipStreamCreateWithFlags: ") + hipGetErrorString(e));
     }
-    e = hipMalloc(&t->d_work, QUEUES * sizeof(int));
+    e = hipMalloc(&t->d_work, WORK_INTS * sizeof(int));
     if (e == hipSuccess) e = hipDeviceGetAttribute(&t->num_cu, hipDeviceAttributeMultiprocessorCount, device);
     if (e != hipSuccess) {
         dfree(t->d_work);
@@ -5596,7 +5623,7 @@ int cuslines_tracker_fork(cuslines_tracker *t, cuslines_tracker **out) {
     f->rec_count = nullptr;
     f->count_taps = 0;
     hipError_t e = hipStreamCreateWithFlags(&f->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMalloc(&f->d_work, QUEUES * sizeof(int));
+    if (e == hipSuccess) e = hipMalloc(&f->d_work, WORK_INTS * sizeof(int));
     if (e != hipSuccess) {
         dfree(f->d_work);
         if (f->stream) (void)hipStreamDestroy(f->stream);

@@ -66,6 +66,12 @@ def test_thin_volumes(shape):
     _check(*_workload(362, shape=shape))
 
 
+@pytest.mark.parametrize("shape", [(256, 3, 2), (257, 3, 2), (3, 2, 520)])
+def test_long_volumes(shape):
+    """Seed-order bricks of 4 voxels up to 256 voxels, coarser past them."""
+    _check(*_workload(66, shape=shape))
+
+
 def test_symmetric_sphere():
     _check(*_workload(362, symm=1))
 
