@@ -176,7 +176,7 @@ class DeviceTracker:
         """Bootstrap phase-2 kernel: BOOT_EXACT (bit-identical to the CPU
         oracle) or BOOT_MFMA (16 seeds in lockstep, matrix products on the
         matrix cores; equal within float rounding).  waves_per_simd (2 or 4,
-        0 = the default 4) picks the MFMA kernel's occupancy variant;
+        0 = by the number of seeds) picks the MFMA kernel's occupancy variant;
         full_products keeps the full [H; R] product where the low-rank form
         (H = U U^T, R its leveraged centred residual matrix) would apply."""
         m = int(mode) | (int(waves_per_simd) << 8) | (self.BOOT_FULL_PRODUCTS if full_products else 0)

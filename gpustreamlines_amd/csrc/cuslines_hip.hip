@@ -43,7 +43,6 @@ constexpr float PTT_MIN_NORM2 = 1e-16f;                // (1/PTT_INV_NORM_EPS)^2
 constexpr float CSA_C0 = 0.28209479177387814f;         // boot.cu:363
 constexpr int DISC_VERT_CNT = 24;                      // disc.h:20
 constexpr int DISC_FACE_CNT = 31;                      // disc.h:21
-constexpr int SORT_LAYERS = 15;
 constexpr int XCDS = 8;
 constexpr int SEED_CLASSES = 8;                          // by direction count; the last has none and is not queued
 constexpr int QUEUES = XCDS * (SEED_CLASSES - 1);        // persistent-queue counters, one per class and XCD
@@ -67,38 +66,6 @@ __constant__ int c_disc_face[DISC_FACE_CNT * 3] = {
     13, 15, 11, 22, 18, 23, 22, 20, 16, 16, 18, 22, 16, 20, 17, 12, 10, 17, 17, 10, 16, 15, 19, 21,
     23, 18, 21, 21, 18, 15, 2, 4, 8,    2, 5, 0,    8, 5, 2,    7, 10, 12,  6, 7, 3,    10, 7, 6,
     3, 1, 6,    1, 5, 6,    11, 10, 6,  6, 5, 11,   14, 19, 15, 15, 13, 14, 14, 13, 9};
-
-// Partner lane of every layer of the 32-key sort network, lane-major: lane g
-// reads its 16 bytes (byte L = partner in layer L) with one load.  Filled at
-// tracker creation from the generator below.
-__constant__ uint4 c_sortnet4[32];
-
-// Knuth's merge exchange (TAOCP 5.2.2 Algorithm M) for 32 keys with each
-// comparator placed in the earliest layer its inputs allow: the network of
-// the reference's warp sort tables (cuwsort.cuh:37-52).
-void make_sortnet(unsigned char out[SORT_LAYERS][32], int *nlayers) {
-    int ready[32] = {0};
-    for (int L = 0; L < SORT_LAYERS; ++L)
-        for (int l = 0; l < 32; ++l) out[L][l] = (unsigned char)l;
-    int nl = 0;
-    const int n = 32, t = 5;
-    for (int p = 1 << (t - 1); p > 0; p >>= 1) {
-        int q = 1 << (t - 1), r = 0, d = p;
-        for (;;) {
-            for (int i = 0; i < n - d; ++i) {
-                if ((i & p) != r) continue;
-                const int a = i, b = i + d;
-                const int L = std::max(ready[a], ready[b]);
-                out[L][a] = (unsigned char)b;
-                out[L][b] = (unsigned char)a;
-                ready[a] = ready[b] = L + 1;
-                nl = std::max(nl, L + 1);
-            }
-            if (q != p) { d = q - p; q >>= 1; r = p; } else break;
-        }
-    }
-    *nlayers = nl;
-}
 
 struct DevParams {
     int dimx, dimy, dimz, dimt, t32;
@@ -168,22 +135,41 @@ __device__ __forceinline__ QueueRange queue_range(const int *work, int k) {
 // Sorting, scans and peak extraction (per half-wave)
 // -------------------------------------------------------------------------
 
-// warp_sort<32,32,WSORT_DIR_DEC> (cuwsort.cuh:104-168) on (key, value).
-__device__ __forceinline__ void sort_dec(float &k, int &v) {
+// warp_sort<32,32,WSORT_DIR_DEC> (cuwsort.cuh:104-168) on (key, value): Knuth's
+// merge exchange (TAOCP 5.2.2 Algorithm M) for 32 keys, the network of the
+// reference's tables (cuwsort.cuh:37-52; the same comparators in the same
+// order on every wire, so ties end where the tables put them).  One pass:
+// lanes i with i & P == R compare with i + D.
+template <int P, int R, int D>
+__device__ __forceinline__ void sort_pass(float &k, int &v) {
     const int g = lane32();
-    const uint4 net = c_sortnet4[g];
-#pragma unroll
-    for (int L = 0; L < SORT_LAYERS; ++L) {
-        const uint32_t w = (L < 4) ? net.x : (L < 8) ? net.y : (L < 12) ? net.z : net.w;
-        const int src = (int)((w >> (8 * (L & 3))) & 0xffu);
-        const float a = shfl32(k, src);
-        const int b = shfl32(v, src);
-        if (g >= src) {
-            if (a < k) { k = a; v = b; }
-        } else {
-            if (a > k) { k = a; v = b; }
-        }
-    }
+    const bool lo = (g & P) == R && g + D < 32, hi = g >= D && ((g - D) & P) == R;
+    const int src = lo ? g + D : hi ? g - D : g;
+    const float a = shfl32(k, src);
+    const int b = shfl32(v, src);
+    if (lo ? (a > k) : (a < k)) { k = a; v = b; }
+}
+
+// n keys, the lanes past them at the lowest value: a comparator that reaches a
+// lane past the keys finds it in order, so 16 keys need 10 of the 15 passes
+// and 8 need 6.
+__device__ __forceinline__ void sort_dec(float &k, int &v, int n) {
+    const bool n16 = n > 16, n8 = n > 8;
+    if (n16) sort_pass<16, 0, 16>(k, v);
+    if (n8) sort_pass<8, 0, 8>(k, v);
+    if (n16) sort_pass<8, 8, 8>(k, v);
+    sort_pass<4, 0, 4>(k, v);
+    if (n16) sort_pass<4, 4, 12>(k, v);
+    if (n8) sort_pass<4, 4, 4>(k, v);
+    sort_pass<2, 0, 2>(k, v);
+    if (n16) sort_pass<2, 2, 14>(k, v);
+    if (n8) sort_pass<2, 2, 6>(k, v);
+    sort_pass<2, 2, 2>(k, v);
+    sort_pass<1, 0, 1>(k, v);
+    if (n16) sort_pass<1, 1, 15>(k, v);
+    if (n8) sort_pass<1, 1, 7>(k, v);
+    sort_pass<1, 1, 3>(k, v);
+    sort_pass<1, 1, 1>(k, v);
 }
 
 // prefix_sum_sh_d (utils.cu:81-120): blocks of 32, lane 0 adds the previous
@@ -306,43 +292,50 @@ __device__ int peak_directions(const DevParams &P, const DevBufs &B, const float
 
 // The tail of peak_directions_d (tracking_helpers.cu:182-245) on the n
 // candidates in cand: descending sort when n < 32, then the greedy
-// minimum-separation filter on lane 0.
+// minimum-separation filter.
 __device__ int sort_dedup_peaks(const DevParams &P, const float *odf, uint16_t *cand, const float *sv, int n) {
     const int l = lane32();
-    if (n < 32) {
-        float k = REAL_MIN;
-        int v = 0;
-        if (l < n) { v = cand[l]; k = odf[v]; }
-        sort_dec(k, v);
-        if (l < n) cand[l] = (uint16_t)v;
-        WAVE_SYNC();
-    }
     if (n == 0) return 0;
     if (n <= 32) {
+        int ci = (l < n) ? cand[l] : 0;
+        if (n < 32) {
+            float k = (l < n) ? odf[ci] : REAL_MIN;
+            sort_dec(k, ci, half_ballot(k < REAL_MIN) ? 32 : n);
+        }
         // remove_similar_vertices (tracking_helpers.cu:195-223) on 32 lanes:
         // lane i holds candidate i's direction and marks which earlier
         // candidates j lie within the minimum separation (the same dot
-        // product and test as the greedy loop below); the greedy pass then
-        // keeps candidate i iff none of its marked candidates was kept, and
-        // the kept indices are compacted in order.  Same kept set as the
-        // single-lane loop, without its chain of dependent vertex loads.
-        int ci = 0;
+        // product and test as the greedy loop below).  Candidate i is kept
+        // iff none of its marked candidates is: each round decides those
+        // whose marked candidates are all decided, a few rounds instead of
+        // one step per candidate.  Four directions are read at a time.
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
-        if (l < n) {
-            ci = cand[l];
-            ax = sv[3 * ci]; ay = sv[3 * ci + 1]; az = sv[3 * ci + 2];
-        }
+        if (l < n) { ax = sv[3 * ci]; ay = sv[3 * ci + 1]; az = sv[3 * ci + 2]; }
         uint32_t conf = 0u;
-        for (int j = 0; j < n - 1; ++j) {
-            const float bx = shfl32(ax, j), by = shfl32(ay, j), bz = shfl32(az, j);
-            float c = dot3(ax, ay, az, bx, by, bz);
-            if (P.sphere_symm) c = fabsf(c);
-            if (j < l && c > P.cos_min_sep) conf |= 1u << j;
+        for (int j0 = 0; j0 < n - 1; j0 += 4) {
+            float bx[4], by[4], bz[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {  // lanes past n - 2 hold nothing that is marked
+                bx[u] = shfl32(ax, (j0 + u) & 31);
+                by[u] = shfl32(ay, (j0 + u) & 31);
+                bz[u] = shfl32(az, (j0 + u) & 31);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                float c = dot3(ax, ay, az, bx[u], by[u], bz[u]);
+                if (P.sphere_symm) c = fabsf(c);
+                if (j0 + u < l && c > P.cos_min_sep) conf |= 1u << ((j0 + u) & 31);
+            }
         }
-        uint32_t keep = 1u;
-        for (int i = 1; i < n; ++i) {
-            const uint32_t ci_conf = (uint32_t)shfl32((int)conf, i);
-            if ((ci_conf & keep) == 0u) keep |= 1u << i;
+        uint32_t keep = 0u, decided = ~0u << (n & 31);  // lanes n.. count as decided
+        if (n == 32) decided = 0u;
+        while (decided != 0xffffffffu) {
+            const bool open = !((decided >> l) & 1u);
+            const bool gone = open && (conf & keep) != 0u;
+            const bool kept = open && !gone && (conf & ~decided) == 0u;
+            const uint32_t kmask = half_ballot(kept);
+            decided |= half_ballot(gone) | kmask;
+            keep |= kmask;
         }
         WAVE_SYNC();
         if (l < n && ((keep >> l) & 1u)) cand[__popc(keep & ((1u << l) - 1u))] = (uint16_t)ci;
@@ -3933,17 +3926,29 @@ __global__ void __launch_bounds__((MODEL == CUSLINES_PTT && V == 1)   ? 512
 //   phase B  [H; R] (2 hr16 x hr16) . X (hr16 x 16)    -> H.d, R.d
 //   phase D  [dq | -db] (dn16 x 2 hr16) . [xf; msk]    -> model coefficients
 //   phase E  S (nv16 x dn16) . C (dn16 x 16)           -> ODF on the sphere
+//   phase F  the peak tests of every slot's vertices on all 8 waves, then each
+//            slot's sort, closest peak and step on its own lanes
 // Each matrix element read from L2 thus serves 16 seeds instead of one.  The
 // products sum in another order than the reference's lane-strided dot
 // products, so results agree with the scalar path within float rounding:
 // peak indices are the same except at near-ties, and a streamline is
 // identical up to the first step whose peak choice flips.
+// What bounds it: a run lasts as long as its longest seed's chain of rounds
+// (some 3000 of them), and a round is a chain of latencies -- barriers, L2
+// reads of matrix rows, LDS -- of 54 k cycles for a lone slot when every phase
+// ran on the slot's own lanes and one load was in flight at a time, about 40 k
+// now; past some 50 000 seeds it is the vector work of 16 slots a workgroup.
+// Measured with both variants below at their best, before | after: CSA 100
+// seeds on 46x55x41 14.4 | 7.9 ms, 25 000 on 81x106x76 122 | 74 ms, 150 000
+// 326 | 229 ms; 6001 seeds of 270 directions, order 8, 115 | 68 ms; OPDT
+// 40 000 96 | 64 ms.
 // Matrices (uploaded zero padded, row-major): hr_mat [2 hr16][hr16],
 // fit_mat [dn16][2 hr16], odf_mat [nv16][dn16].  LDS per slot: the scalar
 // slot's regions, the stride padded to 4 mod 32 floats so the 16 slots' rows
 // sit in distinct LDS banks for the MFMA operand reads and result writes.
 // -------------------------------------------------------------------------
 constexpr int BB_SLOTS = 16, BB_THREADS = 512, BB_WAVES = BB_THREADS / 64;
+constexpr int BB_ROWS = 320 / 32;  // rows of 32 DWI channels (boot_batch_fits)
 constexpr int BB_MAX_ATTEMPTS = 5;  // NATTEMPTS of tracker_boot_d (boot.cu:757)
 
 typedef float bb_v4 __attribute__((ext_vector_type(4)));
@@ -3960,54 +3965,76 @@ __host__ __device__ inline int bb_slot_stride(int nv32, int t32, int hr32) {
 // A[l % 16][k] and X_{l % 16}[k] of each step and holds Y rows 4 (l / 16) + r;
 // within a 16-wide chunk of K, lane group q = l / 16 reads the contiguous k =
 // 16 c + 4 q + (0..3) as one 16-byte load and MFMA step s takes component s.
-// wmax (optional): this wave's maximum of each slot's result rows < ymax,
-// written to wmax[wave * 16 + slot].
-template <int MAXT, bool CSA_ROW0 = false>
+// wmax, wmin (optional): this wave's maximum (NaN passed over) and minimum
+// (NaN if any is) of each slot's result rows < ymax, written to
+// wmax / wmin[wave * 16 + slot].
+// UN steps of K have their loads in flight together (the wave index is made
+// scalar, so that no tile's loads sit behind a divergent branch): a step's
+// matrix rows come from L2, and one load round trip per step was most of
+// these products' time.
+template <int MAXT, int UN, bool CSA_ROW0 = false>
 __device__ __forceinline__ void bb_gemm(const float *__restrict__ A, int lda, int K, int ntiles, const float *X,
                                         const float *X2, int ksplit, float *Y, float *Y2, int ysplit, int ymax,
-                                        int ss, float *wmax = nullptr) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+                                        int ss, float *wmax = nullptr, float *wmin = nullptr) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // addresses are formed here, not kept in registers around the round
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, q = lane >> 4;
     bb_v4 acc[MAXT];
 #pragma unroll
     for (int i = 0; i < MAXT; ++i) acc[i] = bb_v4{0.0f, 0.0f, 0.0f, 0.0f};
-    const float *ap = A + (size_t)n * lda + 4 * q;
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        const float *xs = (k0 < ksplit) ? X + n * ss + k0 : X2 + n * ss + (k0 - ksplit);
-        const float4 b = *reinterpret_cast<const float4 *>(xs + 4 * q);
-        float4 a[MAXT];
+    if (w < ntiles) {
+        const int aoff = n * lda + 4 * q;
+        for (int k0 = 0; k0 < K; k0 += 16 * UN) {
+            float4 a[UN][MAXT], b[UN];
 #pragma unroll
-        for (int i = 0; i < MAXT; ++i) {
-            const int t = w + BB_WAVES * i;
-            if (t < ntiles) a[i] = *reinterpret_cast<const float4 *>(ap + (size_t)t * 16 * lda + k0);
-        }
+            for (int u = 0; u < UN; ++u) {
+                const int k = min(k0 + 16 * u, K - 16);  // past the end: re-read, not used
 #pragma unroll
-        for (int i = 0; i < MAXT; ++i) {
-            const int t = w + BB_WAVES * i;
-            if (t < ntiles) {
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].x, b.x, acc[i], 0, 0, 0);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].y, b.y, acc[i], 0, 0, 0);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].z, b.z, acc[i], 0, 0, 0);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].w, b.w, acc[i], 0, 0, 0);
+                for (int i = 0; i < MAXT; ++i) {
+                    const int t = min(w + BB_WAVES * i, ntiles - 1);  // past the last tile: re-read, dropped below
+                    a[u][i] = *reinterpret_cast<const float4 *>(A + (size_t)t * 16 * lda + k + aoff);
+                }
+                const float *xs = (k < ksplit) ? X + n * ss + k : X2 + n * ss + (k - ksplit);
+                b[u] = *reinterpret_cast<const float4 *>(xs + 4 * q);
+            }
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                if (k0 + 16 * u < K) {
+#pragma unroll
+                    for (int i = 0; i < MAXT; ++i) {
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i].x, b[u].x, acc[i], 0, 0, 0);
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i].y, b[u].y, acc[i], 0, 0, 0);
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i].z, b[u].z, acc[i], 0, 0, 0);
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i].w, b[u].w, acc[i], 0, 0, 0);
+                    }
+                }
             }
         }
     }
     if (wmax) {
-        float pm = REAL_MIN;
+        float pm = REAL_MIN, mn = REAL_MAX;
 #pragma unroll
         for (int i = 0; i < MAXT; ++i) {
             const int t = w + BB_WAVES * i;
             const int row = 16 * t + 4 * q;
             if (t < ntiles) {
-                if (row < ymax) pm = fmaxf(pm, acc[i].x);
-                if (row + 1 < ymax) pm = fmaxf(pm, acc[i].y);
-                if (row + 2 < ymax) pm = fmaxf(pm, acc[i].z);
-                if (row + 3 < ymax) pm = fmaxf(pm, acc[i].w);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (row + r < ymax) {
+                        pm = fmaxf(pm, acc[i][r]);
+                        mn = __builtin_elementwise_minimum(mn, acc[i][r]);
+                    }
             }
         }
         pm = fmaxf(pm, __shfl_xor(pm, 16));
         pm = fmaxf(pm, __shfl_xor(pm, 32));
-        if (q == 0) wmax[w * 16 + n] = pm;
+        mn = __builtin_elementwise_minimum(mn, __shfl_xor(mn, 16));
+        mn = __builtin_elementwise_minimum(mn, __shfl_xor(mn, 32));
+        if (q == 0) {
+            wmax[w * 16 + n] = pm;
+            wmin[w * 16 + n] = mn;
+        }
     }
 #pragma unroll
     for (int i = 0; i < MAXT; ++i) {
@@ -4050,7 +4077,7 @@ __device__ __forceinline__ float bb_xf(float x) {
 // peak is never below thr (its thresholded value would be 0 with no
 // strictly smaller neighbour), so the kept candidates' values, the sort
 // keys, are the raw ODF values.  Needs the adjacency table (B.nbr).
-__device__ int bb_peaks(const DevParams &P, const DevBufs &B, const float *odf, float thr, uint16_t *cand,
+__device__ int bb_peaks_all(const DevParams &P, const DevBufs &B, const float *odf, float thr, uint16_t *cand,
                         const float *sv) {
     const int l = lane32();
     const int nv = P.nverts;
@@ -4146,6 +4173,109 @@ __device__ int bb_peaks(const DevParams &P, const DevBufs &B, const float *odf, 
     }
     WAVE_SYNC();
     return sort_dedup_peaks(P, odf, cand, sv, n);
+}
+
+// bb_peaks_all, or the edge form without an adjacency table (out of line:
+// rare, or a sphere with a vertex of more than 8 neighbours).
+__device__ __noinline__ int bb_peaks_slow(int nv, int nedges, int symm, float cos_min_sep, float rel_peak,
+                                          const uint16_t *nbr, const uint32_t *edges, const float *verts, float *odf,
+                                          float thr, uint32_t *marks, uint16_t *cand) {
+    DevParams P;
+    DevBufs B;
+    P.nverts = nv; P.nedges = nedges; P.sphere_symm = symm; P.cos_min_sep = cos_min_sep; P.rel_peak = rel_peak;
+    B.nbr = nbr; B.edges = edges;
+    if (nbr) return bb_peaks_all(P, B, odf, thr, cand, verts);
+    for (int j = lane32(); j < nv; j += 32)
+        if (odf[j] < thr) odf[j] = 0.0f;
+    WAVE_SYNC();
+    return peak_directions(P, B, odf, marks, cand, verts);
+}
+
+// sort_dedup_peaks out of line, for the kernel of 4 waves per SIMD: inlined
+// there it costs 20 spilled vector registers.
+__device__ __noinline__ int bb_tail(int symm, float cos_min_sep, const float *odf, uint16_t *cand, const float *verts,
+                                    int n) {
+    DevParams P;
+    P.sphere_symm = symm;
+    P.cos_min_sep = cos_min_sep;
+    return sort_dedup_peaks(P, odf, cand, verts, n);
+}
+
+// bb_peaks_all's kept candidates (before the sort), from the vertices that
+// can pass its last test: x >= thr and x - mn >= rel_peak (pmax - mn), with
+// the ODF's maximum mx in place of the largest peak value pmax.  The two are
+// the same whenever a kept peak has the value mx; the caller checks that.
+// The 64 lanes of every wave test 64 vertices of each slot in `todo` in turn,
+// so the neighbour rows q0, q1 of the wave's vertices (64 w + lane, and 64 (w +
+// 8) + lane) are the same for all slots, and a lone slot has 8 waves at work.
+// thr, mn, comp: of slot (lane % 16).  One bit per vertex goes to the slot's
+// marks, 64 at a time.  On each slot's own lanes, 24 compactions and the
+// candidates' neighbour rows from L2 took 12.4 k of a lone slot's 54 k cycles
+// (6000 CSA seeds 72 ms that way, 62 ms this way).
+__device__ __forceinline__ void bb_peak_bits(uint32_t todo, int nv, int ss, float *smem, int off_marks, const uint4 &q0,
+                                             const uint4 &q1, float thr, float mn, float comp) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    while (todo) {
+        const int s = __builtin_ctz(todo);
+        todo &= todo - 1u;
+        const float *odf = smem + s * ss;
+        uint64_t *marks = reinterpret_cast<uint64_t *>(smem + s * ss + off_marks);
+        const float st = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(thr), s));
+        const float sm = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mn), s));
+        const float sc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(comp), s));
+        const float x0 = odf[min(64 * w + lane, nv - 1)], x1 = odf[min(64 * (w + BB_WAVES) + lane, nv - 1)];
+        auto peak = [&](const uint4 &q, float x, bool valid) {
+            bool p = valid && x >= st && (x - sm) >= sc;
+            if (p) {
+                const uint32_t v[4] = {q.x, q.y, q.z, q.w};
+                float y[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) y[k] = odf[(v[k >> 1] >> (16 * (k & 1))) & 0xffffu];
+                float lo = y[0], hi = y[0];
+#pragma unroll
+                for (int k = 1; k < 8; ++k) {
+                    lo = fminf(lo, y[k]);
+                    hi = fmaxf(hi, y[k]);
+                }
+                p = lo < x && !(hi > x);
+            }
+            return __ballot(p);
+        };
+        if (64 * w < nv) {
+            const uint64_t m = peak(q0, x0, 64 * w + lane < nv);
+            if (lane == 0) marks[w] = m;
+        }
+        if (64 * (w + BB_WAVES) < nv) {
+            const uint64_t m = peak(q1, x1, 64 * (w + BB_WAVES) + lane < nv);
+            if (lane == 0) marks[w + BB_WAVES] = m;
+        }
+    }
+}
+
+// The vertices marked by bb_peak_bits, in order, to cand; -1 if none has the value mx.
+__device__ __forceinline__ int bb_peak_list(int nv, const float *odf, float mx, const uint32_t *marks, uint16_t *cand) {
+    const int l = lane32();
+    uint32_t m = (32 * l < nv) ? marks[l] : 0u;
+    const int c = __popc(m);
+    int e = c;
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) {
+        const int o = __shfl_up(e, d, 32);
+        if (l >= d) e += o;
+    }
+    const int n = shfl32(e, 31);
+    int pos = e - c;
+    bool top = false;
+    while (m) {
+        const int j = 32 * l + __builtin_ctz(m);
+        m &= m - 1u;
+        top = top || odf[j] == mx;
+        cand[pos++] = (uint16_t)j;
+    }
+    WAVE_SYNC();
+    return half_ballot(top) ? n : -1;
 }
 
 // Per-slot state of the batched kernel (registers of the slot's 32 lanes).
@@ -4248,11 +4378,51 @@ __device__ void bb_end_pass(const DevParams &P, const DevBufs &B, BbSlot &st, Ph
     if (!st.done) bb_start_pass(P, st, sline);
 }
 
-// OCC: waves per SIMD the kernel is compiled for (2: 256 VGPRs and one
-// workgroup per CU; 4: 128 VGPRs with spills and two workgroups per CU, the
-// default: 99.8 against 71.9 M steps/s for CSA at 1M seeds when the two were
-// compared, before the min/max peak test and the low-rank form, as the two
-// workgroups' lockstep phases overlap).
+// trilinear on 16-byte loads: lane l owns channels 128 c + 4 l .. + 3, a
+// chunk's 8 corner loads in flight (two chunks' 64 registers spill at 4 waves
+// per SIMD: 25,000 seeds 101 instead of 91 ms).  False outside the volume.
+__device__ __forceinline__ bool bb_gather(const DevParams &P, const float *__restrict__ data, float px, float py,
+                                          float pz, float *out) {
+    if ((px < -0.5f) | (px + 0.5f >= (float)P.dimx) | (py < -0.5f) | (py + 0.5f >= (float)P.dimy) | (pz < -0.5f) |
+        (pz + 0.5f >= (float)P.dimz))
+        return false;
+    const int l = lane32();
+    const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+    const float wx1 = px - fx, wy1 = py - fy, wz1 = pz - fz;
+    const float wx0 = 1.0f - wx1, wy0 = 1.0f - wy1, wz0 = 1.0f - wz1;
+    const int x0 = (int)((0.0f > fx) ? 0.0f : fx), y0 = (int)((0.0f > fy) ? 0.0f : fy),
+              z0 = (int)((0.0f > fz) ? 0.0f : fz);
+    const float w[8] = {(wx0 * wy0) * wz0, (wx0 * wy0) * wz1, (wx0 * wy1) * wz0, (wx0 * wy1) * wz1,
+                        (wx1 * wy0) * wz0, (wx1 * wy0) * wz1, (wx1 * wy1) * wz0, (wx1 * wy1) * wz1};
+    const uint32_t dzv = (z0 + 1 < P.dimz) ? 1u : 0u;
+    const uint32_t dyv = (y0 + 1 < P.dimy) ? (uint32_t)P.dimz : 0u;
+    const uint32_t dxv = (x0 + 1 < P.dimx) ? (uint32_t)P.dimy * (uint32_t)P.dimz : 0u;
+    const uint32_t vox = ((uint32_t)x0 * (uint32_t)P.dimy + (uint32_t)y0) * (uint32_t)P.dimz + (uint32_t)z0;
+    const float *c[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        c[k] = data + (uint64_t)(vox + ((k & 4) ? dxv : 0u) + ((k & 2) ? dyv : 0u) + ((k & 1) ? dzv : 0u)) *
+                          (uint32_t)P.t32;
+    for (int t0 = 0; t0 < P.t32; t0 += 128) {
+        const int ta = t0 + 4 * l;
+        const int sa = min(ta, P.t32 - 4);  // past the row: re-read, dropped
+        float4 va[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) va[k] = *reinterpret_cast<const float4 *>(c[k] + sa);
+        float4 a = float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            a.x = __builtin_fmaf(w[k], va[k].x, a.x); a.y = __builtin_fmaf(w[k], va[k].y, a.y);
+            a.z = __builtin_fmaf(w[k], va[k].z, a.z); a.w = __builtin_fmaf(w[k], va[k].w, a.w);
+        }
+        if (ta < P.t32) *reinterpret_cast<float4 *>(out + ta) = a;
+    }
+    return true;
+}
+
+// OCC: waves per SIMD the kernel is compiled for (2: 185 VGPRs and one
+// workgroup per CU; 4: 128 VGPRs, 40 spilled, and two workgroups per CU, whose
+// lockstep phases overlap).  launch_boot_batch has the rule and its figures.
 // LR: the low-rank form of the [H; R] product (P.rk16 > 0), a separate
 // instantiation so that each form's kernel carries only its own registers.
 template <int MODEL, int OCC, bool LR>
@@ -4261,6 +4431,7 @@ __global__ void __launch_bounds__(BB_THREADS, OCC)
                              const int *__restrict__ offsets, const int *__restrict__ dirs,
                              int *__restrict__ sline_seed, int *__restrict__ sline_len, float *__restrict__ sline,
                              const int *__restrict__ order, int *__restrict__ work) {
+    constexpr int UN_ODF = (OCC == 4) ? 1 : 2;
     extern __shared__ float smem[];
     const int ss = bb_slot_stride(P.nv32, P.t32, P.hr32);
     const int slot = threadIdx.x >> 5;
@@ -4272,26 +4443,65 @@ __global__ void __launch_bounds__(BB_THREADS, OCC)
     const int off_h = 0;
     const int off_vox = (int)(S.vox - smem) - slot * ss, off_msk = (int)(S.msk - smem) - slot * ss,
               off_r = (int)(S.r - smem) - slot * ss;
-    const int hr = P.hr, T = P.dimt, nv = P.nverts, hr16 = P.hr16;
+    const int hr = P.hr, T = P.dimt, nv = P.nverts;
     const int MAXL = P.max_sline_len;
-    float *wmax = smem + BB_SLOTS * ss;  // [BB_WAVES][16] partial ODF maxima of phase E
+    float *wmax = smem + BB_SLOTS * ss;  // [BB_WAVES][16] partial ODF maxima of phase E, and minima
+    float *wmin = wmax + BB_WAVES * 16;
+    int *live = reinterpret_cast<int *>(wmin + BB_WAVES * 16);  // [16] slots with a signal this round
+    // the lane's rows of the signal: its DWI channels (two to a register) and which of its channels are b0
+    uint32_t dwi2[BB_ROWS / 2];
+#pragma unroll
+    for (int r = 0; r < BB_ROWS; ++r) {
+        const uint32_t d = (l + 32 * r < hr) ? (uint32_t)B.dwi_idx[l + 32 * r] : 0u;
+        dwi2[r >> 1] = (r & 1) ? dwi2[r >> 1] | (d << 16) : d;
+    }
+    uint32_t b0_rows = 0u;
+    for (int r = 0, j = l; r < 32 && j < T; ++r, j += 32) b0_rows |= (B.b0[j] ? 1u : 0u) << r;
+    // floor(2^32 / hr), for hr 1 the largest 32-bit number: the high product of a draw is its quotient or one less
+    const uint32_t hr_magic = (hr > 1) ? (uint32_t)(0x100000000ull / (uint32_t)hr) : 0xffffffffu;
     BbSlot st;
     st.s = -1; st.qk = 0; st.done = false; st.nb = 0; st.pass = 0;
     Philox rng;
-    bb_next_seed(P, B, st, rng, nseeds, seeds, rng_chunk, offsets, dirs, order, work, sline);
+    // fewer seeds than slots: spread over the workgroups, the rest of their slots idle
+    if ((unsigned)slot * gridDim.x >= (unsigned)nseeds) st.done = true;
+    else bb_next_seed(P, B, st, rng, nseeds, seeds, rng_chunk, offsets, dirs, order, work, sline);
     if (!st.done) bb_start_pass(P, st, sline);
     unsigned long long attempts = 0, rounds = 0;  // slot attempts and rounds of this workgroup
     for (;;) {
+        // Formed anew each round: kept around it, the row tests of the
+        // unrolled loops below take 90 scalar and their addresses as many
+        // vector registers, and the 128 of 4 waves per SIMD spill.
+        int l = lane32(), hr = P.hr, hr16 = P.hr16;
+        asm volatile("" : "+v"(l), "+s"(hr), "+s"(hr16));
         // ---- phase A: gather the signal at the point -----------------------
+        // The masked signal, and the normalisation by the b0 mean, which the
+        // resampling does not touch.
         const bool active = !st.done;
         bool data = false;
+        float inv = 0.0f;
         if (active) {
-            data = trilinear<3>(P, B.data, P.t32, T, st.px, st.py, st.pz, S.vox) == 0;
+            data = bb_gather(P, B.data, st.px, st.py, st.pz, S.vox);
             WAVE_SYNC();
             if (data) {
-                for (int m = l; m < hr16; m += 32) S.msk[m] = (m < hr) ? S.vox[B.dwi_idx[m]] : 0.0f;
+                float part = 0.0f;
+                for (int r = 0, j = l; j < T; ++r, j += 32) {
+                    if ((r < 32) ? ((b0_rows >> r) & 1u) : (uint32_t)(B.b0[j] != 0)) {
+                        float v = S.vox[j];
+                        v = (P.min_signal > v) ? P.min_signal : v;
+                        part = part + v;
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < BB_ROWS; ++r)
+                    if (32 * r < hr16) {
+                        const int m = l + 32 * r;
+                        const float v = S.vox[(dwi2[r >> 1] >> (16 * (r & 1))) & 0xffffu];
+                        if (m < hr16) S.msk[m] = (m < hr) ? v : 0.0f;
+                    }
+                inv = (float)(T - hr) / tree_sum32(part);
             }
         }
+        if (l == 0) live[slot] = data;
         const int nact = __syncthreads_count(active) / 32;  // active slots (32 lanes each)
         if (nact == 0) break;
         attempts += (unsigned long long)nact;
@@ -4300,70 +4510,99 @@ __global__ void __launch_bounds__(BB_THREADS, OCC)
         if (LR) {
             // low-rank form: z = U^T d into the R.d region, then H.d = U z;
             // R.d follows in phase C
-            bb_gemm<1>(B.ut_mat, hr16, hr16, P.rk16 / 16, smem + off_msk, smem + off_msk, hr16, smem + off_r,
-                       smem + off_r, 1 << 30, P.rk16, ss);
+            bb_gemm<1, 5>(B.ut_mat, hr16, hr16, P.rk16 / 16, smem + off_msk, smem + off_msk, hr16, smem + off_r,
+                          smem + off_r, 1 << 30, P.rk16, ss);
             __syncthreads();
-            bb_gemm<(320 / 16 + BB_WAVES - 1) / BB_WAVES>(B.u_mat, P.rk16, P.rk16, hr16 / 16, smem + off_r,
-                                                          smem + off_r, 1 << 30, smem + off_h, smem + off_h, 1 << 30,
-                                                          hr16, ss);
+            bb_gemm<(320 / 16 + BB_WAVES - 1) / BB_WAVES, 2>(B.u_mat, P.rk16, P.rk16, hr16 / 16, smem + off_r,
+                                                             smem + off_r, 1 << 30, smem + off_h, smem + off_h,
+                                                             1 << 30, hr16, ss);
         } else {
-            bb_gemm<(2 * 320 / 16 + BB_WAVES - 1) / BB_WAVES>(B.hr_mat, hr16, hr16, 2 * hr16 / 16, smem + off_msk,
-                                                              smem + off_msk, hr16, smem + off_h, smem + off_r, hr16,
-                                                              2 * hr16, ss);
+            bb_gemm<(2 * 320 / 16 + BB_WAVES - 1) / BB_WAVES, UN_ODF>(B.hr_mat, hr16, hr16, 2 * hr16 / 16,
+                                                                      smem + off_msk, smem + off_msk, hr16,
+                                                                      smem + off_h, smem + off_r, hr16, 2 * hr16, ss);
         }
         __syncthreads();
         // ---- phase C: residual bootstrap, normalisation, model transform -----
-        if (LR && active && data) {
-            // R.d = v - mean(v), v = (d - H.d) / sqrt(1 - H_ii)
-            float part = 0.0f;
-            for (int j = l; j < hr; j += 32) {
-                const float v = (S.msk[j] - S.h[j]) * B.invlev[j];
-                S.r[j] = v;
-                part = part + v;
-            }
-            const float mean = tree_sum32(part) / (float)hr;
-            for (int j = l; j < hr; j += 32) S.r[j] = S.r[j] - mean;
-            WAVE_SYNC();
-        }
         if (active && data) {
-            for (int j = l; j < hr; j += 32) {
-                const int src = (int)(rng.next() % (uint32_t)hr);
-                S.h[j] = S.h[j] + S.r[src];
+            if (LR) {
+                // R.d = v - mean(v), v = (d - H.d) / sqrt(1 - H_ii)
+                float v[BB_ROWS], part = 0.0f;
+#pragma unroll
+                for (int r = 0; r < BB_ROWS; ++r) {
+                    const int j = l + 32 * r;
+                    v[r] = 0.0f;
+                    if (j < hr) {
+                        v[r] = (S.msk[j] - S.h[j]) * B.invlev[j];
+                        part = part + v[r];
+                    }
+                }
+                const float mean = tree_sum32(part) / (float)hr;
+#pragma unroll
+                for (int r = 0; r < BB_ROWS; ++r)
+                    if (l + 32 * r < hr) S.r[l + 32 * r] = v[r] - mean;
+                WAVE_SYNC();
+            }
+            float h[BB_ROWS];
+#pragma unroll
+            for (int r = 0; r < BB_ROWS; ++r) {
+                const int j = l + 32 * r;
+                h[r] = 0.0f;
+                if (j < hr) {
+                    // draw % hr: the high product is the quotient or one less
+                    const uint32_t x = rng.next();
+                    const uint32_t rem = x - __umulhi(x, hr_magic) * (uint32_t)hr;
+                    h[r] = S.h[j] + S.r[min(rem, rem - (uint32_t)hr)];
+                }
             }
             WAVE_SYNC();
-            for (int m = l; m < hr; m += 32) S.vox[B.dwi_idx[m]] = S.h[m];
-            WAVE_SYNC();
-            float part = 0.0f;
-            int cnt = 0;
-            for (int j = l; j < T; j += 32) {
-                float v = S.vox[j];
-                v = (P.min_signal > v) ? P.min_signal : v;
-                S.vox[j] = v;
-                if (B.b0[j]) { ++cnt; part = part + v; }
-            }
-            const float sum = tree_sum32(part);
-            for (int m = 16; m; m >>= 1) cnt += shfl_xor32(cnt, m);
-            const float inv = (float)cnt / sum;
-            for (int j = l; j < T; j += 32) S.vox[j] = S.vox[j] * inv;
-            WAVE_SYNC();
-            for (int m = l; m < hr16; m += 32) {
-                const float v = (m < hr) ? S.vox[B.dwi_idx[m]] : 0.0f;
-                S.msk[m] = v;
-                S.h[m] = (m < hr) ? bb_xf<(MODEL == CUSLINES_OPDT) ? 1 : 2>(v) : 0.0f;
+#pragma unroll
+            for (int r = 0; r < BB_ROWS; ++r) {
+                const int m = l + 32 * r;
+                if (m < hr16) {
+                    const float c = (P.min_signal > h[r]) ? P.min_signal : h[r];
+                    const float v = (m < hr) ? c * inv : 0.0f;
+                    S.msk[m] = v;
+                    S.h[m] = (m < hr) ? bb_xf<(MODEL == CUSLINES_OPDT) ? 1 : 2>(v) : 0.0f;
+                }
             }
         }
         __syncthreads();
         // ---- phase D: model coefficients (CSA: dq.xf; OPDT: dq.xf - db.msk) --
-        bb_gemm<1, MODEL == CUSLINES_CSA>(B.fit_mat, 2 * hr16, (MODEL == CUSLINES_OPDT) ? 2 * hr16 : hr16,
-                                           P.dn16 / 16, smem + off_h, smem + off_msk, hr16, smem + off_vox,
-                                           smem + off_vox, 1 << 30, P.dn16, ss);
+        bb_gemm<1, 5, MODEL == CUSLINES_CSA>(B.fit_mat, 2 * hr16, (MODEL == CUSLINES_OPDT) ? 2 * hr16 : hr16,
+                                             P.dn16 / 16, smem + off_h, smem + off_msk, hr16, smem + off_vox,
+                                             smem + off_vox, 1 << 30, P.dn16, ss);
         __syncthreads();
         // ---- phase E: the ODF on the sphere ---------------------------------
-        bb_gemm<(768 / 16 + BB_WAVES - 1) / BB_WAVES>(B.odf_mat, P.dn16, P.dn16, P.nv16 / 16, smem + off_vox,
-                                                      smem + off_vox, 1 << 30, smem + off_h, smem + off_h, 1 << 30,
-                                                      nv, ss, wmax);
+        bb_gemm<(768 / 16 + BB_WAVES - 1) / BB_WAVES, UN_ODF>(B.odf_mat, P.dn16, P.dn16, P.nv16 / 16, smem + off_vox,
+                                                              smem + off_vox, 1 << 30, smem + off_h, smem + off_h,
+                                                              1 << 30, nv, ss, wmax, wmin);
+        uint4 nb0 = uint4{0u, 0u, 0u, 0u}, nb1 = nb0;
+        if (B.nbr) {
+            int t = threadIdx.x;
+            asm volatile("" : "+v"(t));
+            nb0 = reinterpret_cast<const uint4 *>(B.nbr)[min(t, nv - 1)];
+            nb1 = reinterpret_cast<const uint4 *>(B.nbr)[min(t + BB_THREADS, nv - 1)];
+        }
         __syncthreads();
         // ---- phase F: peaks, closest peak, the step --------------------------
+        uint32_t fast = 0u;  // slots whose peaks bb_peak_bits marks
+        if (B.nbr) {
+            // lane: slot lane % 16
+            const int k = threadIdx.x & 63;
+            float mx = fmaxf(wmax[k], wmax[k + 64]);
+            float mn = __builtin_elementwise_minimum(wmin[k], wmin[k + 64]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            mn = __builtin_elementwise_minimum(mn, __shfl_xor(mn, 16));
+            mn = __builtin_elementwise_minimum(mn, __shfl_xor(mn, 32));
+            const float thr = (float)(PMF_THRESHOLD_P * (double)mx);
+            // a value below thr reads as 0 (and thr > 0), a NaN is left to bb_peaks_all
+            fast = (uint32_t)__ballot(live[k & 15] && thr > 0.0f && mn == mn) & 0xffffu;
+            mn = (mn < thr) ? 0.0f : mn;
+            const float comp = (float)((double)P.rel_peak * (double)(mx + (-mn)));
+            bb_peak_bits(fast, nv, ss, smem, (int)((float *)S.marks - smem) - slot * ss, nb0, nb1, thr, mn, comp);
+            __syncthreads();
+        }
         if (active) {
             int ns = -1;  // >= 0: the pass ends with ns points
             if (!data) {
@@ -4375,15 +4614,13 @@ __global__ void __launch_bounds__(BB_THREADS, OCC)
                 float mx = (l < BB_WAVES) ? wmax[l * 16 + slot] : REAL_MIN;
                 mx = max32(mx);
                 const float thr = (float)(PMF_THRESHOLD_P * (double)mx);
-                int npk;
-                if (B.nbr) {
-                    npk = bb_peaks(P, B, S.h, thr, S.cand, B.verts);
-                } else {
-                    for (int j = l; j < nv; j += 32)
-                        if (S.h[j] < thr) S.h[j] = 0.0f;
-                    WAVE_SYNC();
-                    npk = peak_directions(P, B, S.h, S.marks, S.cand, B.verts);
-                }
+                int npk = ((fast >> slot) & 1u) ? bb_peak_list(nv, S.h, mx, S.marks, S.cand) : -1;
+                if (npk >= 0)
+                    npk = (OCC == 4) ? bb_tail(P.sphere_symm, P.cos_min_sep, S.h, S.cand, B.verts, npk)
+                                     : sort_dedup_peaks(P, S.h, S.cand, B.verts, npk);
+                else
+                    npk = bb_peaks_slow(nv, P.nedges, P.sphere_symm, P.cos_min_sep, P.rel_peak, B.nbr, B.edges, B.verts,
+                                        S.h, thr, S.marks, S.cand);
                 float nx = 0.0f, ny = 0.0f, nz = 0.0f;
                 const bool ok = npk > 0 && closest_peak(P, B.verts, st.dx, st.dy, st.dz, npk, S.cand, &nx, &ny, &nz);
                 WAVE_SYNC();
@@ -4886,7 +5123,7 @@ struct cuslines_tracker {
     int rk16 = 0, hrank = 0;                                      // rank of H and rounded to 16 (0: not that form)
     int boot_full = 0;                                            // batched bootstrap: always the [H; R] product
     int boot_mode = CUSLINES_BOOT_EXACT;
-    int boot_occ = 4;  // batched bootstrap: waves per SIMD of the kernel variant
+    int boot_occ = 0;  // batched bootstrap: waves per SIMD of the kernel variant (0: by the number of seeds)
     int *d_b0 = nullptr, *d_dwi = nullptr;
     uint32_t *d_lut = nullptr;
     std::vector<uint16_t> rank_vertex;  // PTT: vertex of each direction rank (corner-block order)
@@ -5232,10 +5469,16 @@ static int launch_boot_batch(cuslines_tracker *t, const float *seeds, int n, int
     if (!boot_batch_fits(d))
         return fail(CUSLINES_EINVAL, "batched bootstrap needs hr <= 320, delta_nr <= 128 and nverts <= 768");
     const size_t lds = sizeof(float) * ((size_t)BB_SLOTS * (size_t)bb_slot_stride(d.nv32, d.t32, d.hr32) +
-                                        (size_t)BB_WAVES * 16);
+                                        2 * (size_t)BB_WAVES * 16 + BB_SLOTS);
     if (lds > 160 * 1024) return fail(CUSLINES_EINVAL, "batched bootstrap slots too large for LDS");
     const bool lr = d.rk16 > 0;
-    const void *kfn = (t->boot_occ == 4)
+    // Up to 8 seeds for each slot of one workgroup per CU, the run lasts as
+    // long as its longest seeds, whose rounds are shorter with 256 registers;
+    // beyond that the two workgroups of the other variant fill each other's
+    // waits (CSA, 160 directions, ms at 2 | 4 waves: 6000 seeds 62 | 68,
+    // 25 000 74 | 80, 60 000 141 | 119, 150 000 327 | 230).
+    const int occ = t->boot_occ ? t->boot_occ : (n <= 8 * BB_SLOTS * t->num_cu) ? 2 : 4;
+    const void *kfn = (occ == 4)
                           ? (lr ? (const void *)phase2_boot_batch_kernel<MODEL, 4, true>
                                 : (const void *)phase2_boot_batch_kernel<MODEL, 4, false>)
                           : (lr ? (const void *)phase2_boot_batch_kernel<MODEL, 2, true>
@@ -5246,8 +5489,7 @@ static int launch_boot_batch(cuslines_tracker *t, const float *seeds, int n, int
     if (per_cu < 1) per_cu = 1;
     if (t->blocks_per_cu > 0 && t->blocks_per_cu < per_cu) per_cu = t->blocks_per_cu;
     long long grid = (long long)per_cu * t->num_cu;
-    const long long need = (n + BB_SLOTS - 1) / BB_SLOTS;
-    if (grid > need) grid = need;
+    if (grid > n) grid = n;
     if (grid < 1) grid = 1;
     if (!t->d_stats && !ws) {  // the kernel's attempt and round counters (not allocated by the no-alloc entry)
         HIPC(hipMalloc(&t->d_stats, 4 * sizeof(unsigned long long)));
@@ -5257,10 +5499,10 @@ static int launch_boot_batch(cuslines_tracker *t, const float *seeds, int n, int
     if (int rc = spatial_order(t, seeds, offsets, n, &order, ws)) return rc;
     const DevBufs bb = bufs_of(t);
     const dim3 g((unsigned)grid), b(BB_THREADS);
-    if (t->boot_occ == 4 && lr)
+    if (occ == 4 && lr)
         hipLaunchKernelGGL((phase2_boot_batch_kernel<MODEL, 4, true>), g, b, lds, t->stream, d, bb, seeds, n, chunk,
                            offsets, dirs, sseed, slen, sl, order, t->d_work);
-    else if (t->boot_occ == 4)
+    else if (occ == 4)
         hipLaunchKernelGGL((phase2_boot_batch_kernel<MODEL, 4, false>), g, b, lds, t->stream, d, bb, seeds, n, chunk,
                            offsets, dirs, sseed, slen, sl, order, t->d_work);
     else if (lr)
@@ -5540,19 +5782,6 @@ int cuslines_tracker_create(const cuslines_params *p, int device, cuslines_track
         (void)hipStreamDestroy(t->stream);
         delete t;
         return rc;
-    }
-    unsigned char net[SORT_LAYERS][32];
-    int nl = 0;
-    make_sortnet(net, &nl);
-    uint32_t packed_net[32][4] = {};
-    for (int L = 0; L < SORT_LAYERS; ++L)
-        for (int g = 0; g < 32; ++g) packed_net[g][L >> 2] |= (uint32_t)net[L][g] << (8 * (L & 3));
-    e = hipMemcpyToSymbol(HIP_SYMBOL(c_sortnet4), packed_net, sizeof(packed_net));
-    if (e != hipSuccess) {
-        dfree(t->d_work);
-        (void)hipStreamDestroy(t->stream);
-        delete t;
-        return fail(CUSLINES_EHIP, std::string("sort network upload: ") + hipGetErrorString(e));
     }
     DevParams &d = t->dp;
     d.dimx = p->dimx; d.dimy = p->dimy; d.dimz = p->dimz; d.dimt = p->dimt; d.t32 = ceil32(p->dimt);
@@ -6091,7 +6320,7 @@ int cuslines_set_boot_mode(cuslines_tracker *t, int mode) {
     if (occ != 0 && occ != 2 && occ != 4) return fail(CUSLINES_EINVAL, "waves per SIMD must be 2 or 4");
     if ((mode & ~(0xffff | CUSLINES_BOOT_FULL_PRODUCTS)) != 0) return fail(CUSLINES_EINVAL, "unknown mode flag");
     t->boot_mode = mode & 0xff;
-    t->boot_occ = occ ? occ : 4;
+    t->boot_occ = occ;
     t->boot_full = (mode & CUSLINES_BOOT_FULL_PRODUCTS) ? 1 : 0;
     return CUSLINES_OK;
 }

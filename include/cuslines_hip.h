@@ -213,8 +213,8 @@ enum {
  * layout are the same.  MFMA mode needs hr <= 320 DWI volumes, delta_nr <= 128
  * and nverts <= 768 (phase 2 returns CUSLINES_EINVAL otherwise) and the
  * queue schedule (CUSLINES_SCHED_STATIC keeps the exact kernel).  Bits 8..15
- * of `mode` choose the MFMA kernel's occupancy, 2 or 4 (default) waves per
- * SIMD (the autotuner's knob).
+ * of `mode` choose the MFMA kernel's occupancy, 2 or 4 waves per SIMD (the
+ * autotuner's knob); 0 leaves it to the number of seeds of each launch.
  * When H is a projection H = U U^T of rank r <= 64 and R its leveraged centred
  * residual matrix (boot_utils.py:86-94: R = L (I - H) - column means, L =
  * diag(1 / sqrt(1 - H_ii))), as cuslines_set_boot_matrices checks to 1e-5, the
