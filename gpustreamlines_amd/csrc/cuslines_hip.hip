@@ -4717,9 +4717,22 @@ __global__ void seed_scatter(const int *__restrict__ key, int n, const int *__re
 }
 
 // -------------------------------------------------------------------------
-// Training of the proposal network (no counterpart in the reference).  Plain
-// per-element kernels: the network is 26,920 parameters and a batch of a few
-// thousand pairs, so a training step is microseconds of arithmetic.
+// Training of the proposal network (no counterpart in the reference).
+//
+// One kernel for the forward and the backward pass and one that adds up its
+// partial gradients.  A workgroup of 8 waves takes tiles of 16 pairs, keeps
+// the three layers' weights (rounded to bf16) as MFMA operands and all weight
+// gradients as MFMA accumulators in registers over its tiles, and writes the
+// gradients once; activations stay in LDS.  The products run on
+// v_mfma_f32_16x16x4_f32 (fp32 operands and sums); wave w owns hidden neurons
+// 16 w .. 16 w + 15 of both layers.
+// At the default 4096 pairs every workgroup has one tile, and what bounds it is
+// latency: reading the weights (10 us), seven short phases between barriers
+// (8 us), writing and re-reading MLP_GROUPS partials (27 MB, 7 + 5 us).  Loss and
+// gradient of 4096 pairs 360 -> 75 us with both copies to the host; the layer
+// by layer, element by element kernels before took 13 launches and re-read
+// the weights for every pair.  60 000 pairs: 94 us, 15 tiles a workgroup at 5 us,
+// where the matrix products alone are 3.6 us.
 // -------------------------------------------------------------------------
 __device__ __forceinline__ float bf16_round(float x) {  // to the nearest bf16, ties to even
     uint32_t b = __float_as_uint(x);
@@ -4728,97 +4741,272 @@ __device__ __forceinline__ float bf16_round(float x) {  // to the nearest bf16, 
     return __uint_as_float(b & 0xffff0000u);
 }
 
-// out[s][j] = act(b[j] + sum_k W[j][k] in[s][k]), parameters rounded to bf16.
-template <int K, int N, bool RELU>
-__global__ void mlp_fwd_layer(const float *__restrict__ prm, int w_off, int b_off, const float *__restrict__ in,
-                              int in_ld, int n, float *__restrict__ out) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)n * N) return;
-    const int smp = (int)(idx / N), j = (int)(idx % N);
-    const float *w = prm + w_off + (size_t)j * K;
-    const float *x = in + (size_t)smp * in_ld;
-    float acc = bf16_round(prm[b_off + j]);
-    for (int k = 0; k < K; ++k) acc = __builtin_fmaf(bf16_round(w[k]), x[k], acc);
-    out[idx] = RELU ? ((acc > 0.0f) ? acc : 0.0f) : acc;
+constexpr int MLP_TILE = 16, MLP_GROUPS = 256, MLP_THREADS = 512;
+// A workgroup's partial gradients as its lanes hold them: 13 tiles (3 of the
+// first layer, 8 of the second, 2 of the third) of 4 floats per thread, then the
+// biases of the three layers and the loss.
+constexpr int MLP_PART_B = 13 * 4 * MLP_THREADS, MLP_PART_LOSS = MLP_PART_B + 2 * MLP_H + MLP_OUT;
+constexpr int MLP_PART = (MLP_PART_LOSS + 1 + 31) & ~31;
+static_assert(MLP_H == 16 * MLP_THREADS / 64 && MLP_IN % 4 == 0 && MLP_OUT <= 32, "tiles of the training kernel");
+// LDS row strides, 20 mod 64 floats: the rows of 16 pairs start in 16
+// different groups of four banks (16-byte reads along a row), and 4 rows
+// of 16 consecutive floats overlap little (reads across the rows).
+constexpr int MLP_LDX = 84, MLP_LDH = 148, MLP_LDO = 36;
+
+struct __attribute__((packed, aligned(4))) FloatQuad {  // 16 bytes at any float's address
+    float v[4];
+};
+
+__device__ __forceinline__ float row_sum16(float v) {  // sum over the 16 lanes of a DPP row
+    v += dpp0<DPP_ROW_ROR + 8>(v);
+    v += dpp0<DPP_ROW_ROR + 4>(v);
+    v += dpp0<DPP_ROW_ROR + 2>(v);
+    v += dpp0<DPP_ROW_ROR + 1>(v);
+    return v;
 }
 
-// Per pair: squared error of the 24 predicted supports, averaged over the
-// 24, and its gradient with respect to the outputs divided by n.
-__global__ void mlp_loss_out(const float *__restrict__ O, const float *__restrict__ pairs, int n,
-                             float *__restrict__ dO, float *__restrict__ loss) {
-    const int smp = blockIdx.x * blockDim.x + threadIdx.x;
-    if (smp >= n) return;
-    const float *o = O + (size_t)smp * MLP_OUT;
-    const float *t = pairs + (size_t)smp * CUSLINES_PAIR_FLOATS + MLP_IN;
-    float *g = dO + (size_t)smp * MLP_OUT;
-    const float sc = 2.0f / ((float)MLP_OUT * (float)n);
-    float acc = 0.0f;
-    for (int j = 0; j < MLP_OUT; ++j) {
-        const float e = o[j] - t[j];
-        acc = __builtin_fmaf(e, e, acc);
-        g[j] = e * sc;
+__global__ void __launch_bounds__(MLP_THREADS, 2)
+    mlp_train_kernel(const float *__restrict__ prm, const float *__restrict__ pairs, int n, float *__restrict__ part) {
+    __shared__ __align__(16) float sx[2][MLP_TILE * MLP_LDX];  // pairs: 40 inputs, 24 targets
+    __shared__ __align__(16) float sh1[MLP_TILE * MLP_LDH], sh2[MLP_TILE * MLP_LDH];
+    __shared__ __align__(16) float sd1[MLP_TILE * MLP_LDH], sd2[MLP_TILE * MLP_LDH];  // gradients at the hidden layers
+    __shared__ float so[4][32 * MLP_TILE];       // output sums over a quarter of the second hidden layer
+    __shared__ float sdo[MLP_TILE * MLP_LDO];    // gradient at the outputs, rows 24..31 zero
+    __shared__ float sred[MLP_THREADS / 16];
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, i = lane & 15, q = lane >> 4;
+    constexpr int H = MLP_H, K1 = MLP_IN / 4, NO = MLP_OUT;
+    const int ntile = (n + MLP_TILE - 1) / MLP_TILE;
+    auto fetch = [&](int t, float (&x)[2]) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = tid + u * MLP_THREADS;
+            const long long smp = (long long)t * MLP_TILE + (e >> 6);
+            x[u] = (smp < n) ? pairs[smp * CUSLINES_PAIR_FLOATS + (e & 63)] : 0.0f;
+        }
+    };
+    float xr[2];
+    fetch(blockIdx.x, xr);
+    // Operands: lane (i, q) holds row i; of a 16-wide chunk c of the sum, step
+    // s takes index 16 c + 4 q + s, and with fewer terms index 4 s + q.
+    float w1[K1], w2[32], w2t[32], w3[8], w3t[NO / 4];
+    const int row = 16 * w + i;
+#pragma unroll
+    for (int s = 0; s < K1; ++s) w1[s] = bf16_round(prm[MLP_W1 + row * MLP_IN + 4 * s + q]);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const FloatQuad f = *reinterpret_cast<const FloatQuad *>(prm + MLP_W2 + row * H + 16 * c + 4 * q);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            w2[4 * c + s] = bf16_round(f.v[s]);
+            w2t[4 * c + s] = bf16_round(prm[MLP_W2 + (16 * c + 4 * q + s) * H + row]);
+        }
     }
-    loss[smp] = acc / (float)MLP_OUT;
-}
-
-// din[s][k] = (sum_j W[j][k] dout[s][j]) where hin[s][k] > 0, else 0.
-template <int N, int K>
-__global__ void mlp_bwd_input(const float *__restrict__ prm, int w_off, const float *__restrict__ dout,
-                              const float *__restrict__ hin, int n, float *__restrict__ din) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)n * K) return;
-    const int smp = (int)(idx / K), k = (int)(idx % K);
-    const float *g = dout + (size_t)smp * N;
-    float acc = 0.0f;
-    for (int j = 0; j < N; ++j) acc = __builtin_fmaf(bf16_round(prm[w_off + (size_t)j * K + k]), g[j], acc);
-    din[idx] = (hin[idx] > 0.0f) ? acc : 0.0f;
-}
-
-// grad W[j][k] = sum_s dout[s][j] in[s][k]; column k == K is the bias.
-// Pass 1: blockIdx.y takes samples [y * WGRAD_CHUNK, (y + 1) * WGRAD_CHUNK)
-// and writes its partial sums to part[y][N * (K + 1)]; pass 2 adds the
-// partials in chunk order (deterministic).
-constexpr int WGRAD_CHUNK = 128;
-template <int N, int K>
-__global__ void mlp_wgrad_part(const float *__restrict__ dout, const float *__restrict__ in, int in_ld, int n,
-                               float *__restrict__ part) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= N * (K + 1)) return;
-    const int j = idx / (K + 1), k = idx % (K + 1);
-    const int s0 = blockIdx.y * WGRAD_CHUNK, s1 = min(n, s0 + WGRAD_CHUNK);
-    float acc = 0.0f;
-    if (k == K) {
-        for (int smp = s0; smp < s1; ++smp) acc += dout[(size_t)smp * N + j];
-    } else {
-        for (int smp = s0; smp < s1; ++smp)
-            acc = __builtin_fmaf(dout[(size_t)smp * N + j], in[(size_t)smp * in_ld + k], acc);
+    const int ot = w & 1, kq = w >> 1;  // third layer: rows 16 ot.., columns 32 kq..
+    uint32_t in3 = (16 * ot + i < NO) ? ~0u : 0u;
+    asm volatile("" : "+v"(in3));  // a mask: as a branch, each of the loads waits for the one before
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int j = 16 * ot + i;
+        const FloatQuad f =
+            *reinterpret_cast<const FloatQuad *>(prm + MLP_W3 + min(j, NO - 1) * H + 32 * kq + 16 * c + 4 * q);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) w3[4 * c + s] = __uint_as_float(__float_as_uint(bf16_round(f.v[s])) & in3);
     }
-    part[(size_t)blockIdx.y * (N * (K + 1)) + idx] = acc;
-}
+#pragma unroll
+    for (int s = 0; s < NO / 4; ++s) w3t[s] = bf16_round(prm[MLP_W3 + (4 * s + q) * H + row]);
+    v4 b1, b2;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        b1[r] = bf16_round(prm[MLP_B1 + 16 * w + 4 * q + r]);
+        b2[r] = bf16_round(prm[MLP_B2 + 16 * w + 4 * q + r]);
+    }
+    const int oj = tid >> 4;  // outputs: thread (output, pair i)
+    const float b3 = bf16_round(prm[MLP_B3 + min(oj, NO - 1)]);
+    const float scale = 2.0f / ((float)NO * (float)n);
 
-template <int N, int K>
-__global__ void mlp_wgrad_sum(const float *__restrict__ part, int nchunk, float *__restrict__ grad, int w_off,
-                              int b_off) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= N * (K + 1)) return;
-    float acc = 0.0f;
-    for (int c = 0; c < nchunk; ++c) acc += part[(size_t)c * (N * (K + 1)) + idx];
-    const int j = idx / (K + 1), k = idx % (K + 1);
-    if (k == K) grad[b_off + j] = acc;
-    else grad[w_off + (size_t)j * K + k] = acc;
-}
+    const v4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    v4 g1[3] = {zero, zero, zero}, g2[8], g3[2] = {zero, zero}, gb1 = zero, gb2 = zero;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) g2[k] = zero;
+    float gb3 = 0.0f, loss = 0.0f;
 
-__global__ void __launch_bounds__(256) mean_kernel(const float *__restrict__ x, int n, float *__restrict__ out) {
-    __shared__ float part[256];
-    float acc = 0.0f;
-    for (int i = threadIdx.x; i < n; i += 256) acc += x[i];
-    part[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = 128; w; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
+    int buf = 0;
+    for (int t = blockIdx.x; t < ntile; t += gridDim.x, buf ^= 1) {
+        float *X = sx[buf];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = tid + u * MLP_THREADS;
+            X[(e >> 6) * MLP_LDX + (e & 63)] = xr[u];
+        }
+        if (t + (int)gridDim.x < ntile) fetch(t + gridDim.x, xr);
+        const bool valid = (long long)t * MLP_TILE + i < n;  // pairs past the last one take no part
         __syncthreads();
+        // first hidden layer
+        v4 h1 = b1;
+#pragma unroll
+        for (int s = 0; s < K1; ++s)
+            h1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[s], X[i * MLP_LDX + 4 * s + q], h1, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h1[r] = (valid && h1[r] > 0.0f) ? h1[r] : 0.0f;
+        *reinterpret_cast<v4 *>(sh1 + i * MLP_LDH + 16 * w + 4 * q) = h1;
+        __syncthreads();
+        // second hidden layer
+        v4 h2 = b2;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const v4 x = *reinterpret_cast<const v4 *>(sh1 + i * MLP_LDH + 16 * c + 4 * q);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) h2 = __builtin_amdgcn_mfma_f32_16x16x4f32(w2[4 * c + s], x[s], h2, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h2[r] = (valid && h2[r] > 0.0f) ? h2[r] : 0.0f;
+        *reinterpret_cast<v4 *>(sh2 + i * MLP_LDH + 16 * w + 4 * q) = h2;
+        __syncthreads();
+        // outputs, a quarter of the sum per pair of waves
+        {
+            v4 o = zero;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const v4 x = *reinterpret_cast<const v4 *>(sh2 + i * MLP_LDH + 32 * kq + 16 * c + 4 * q);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) o = __builtin_amdgcn_mfma_f32_16x16x4f32(w3[4 * c + s], x[s], o, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) so[kq][(16 * ot + 4 * q + r) * MLP_TILE + i] = o[r];
+        }
+        __syncthreads();
+        // the error, the loss and the gradient at the outputs
+        {
+            float d = 0.0f;
+            if (oj < NO && valid) {
+                const float o = b3 + ((so[0][tid] + so[1][tid]) + (so[2][tid] + so[3][tid]));
+                const float e = o - X[i * MLP_LDX + MLP_IN + oj];
+                loss = __builtin_fmaf(e, e, loss);
+                d = e * scale;
+            }
+            gb3 += d;
+            sdo[i * MLP_LDO + oj] = d;
+        }
+        __syncthreads();
+        // gradient at the second hidden layer
+        v4 d2 = zero;
+#pragma unroll
+        for (int s = 0; s < NO / 4; ++s)
+            d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(w3t[s], sdo[i * MLP_LDO + 4 * s + q], d2, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d2[r] = (h2[r] > 0.0f) ? d2[r] : 0.0f;
+        gb2 += d2;
+        *reinterpret_cast<v4 *>(sd2 + i * MLP_LDH + 16 * w + 4 * q) = d2;
+        // third layer's weights: outputs x hidden neurons 16 w.., summed over the pairs
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float x = sh2[(4 * s + q) * MLP_LDH + 16 * w + i];
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                g3[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(sdo[(4 * s + q) * MLP_LDO + 16 * k + i], x, g3[k], 0, 0, 0);
+        }
+        __syncthreads();
+        // gradient at the first hidden layer
+        v4 d1 = zero;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const v4 x = *reinterpret_cast<const v4 *>(sd2 + i * MLP_LDH + 16 * c + 4 * q);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w2t[4 * c + s], x[s], d1, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d1[r] = (h1[r] > 0.0f) ? d1[r] : 0.0f;
+        gb1 += d1;
+        *reinterpret_cast<v4 *>(sd1 + i * MLP_LDH + 16 * w + 4 * q) = d1;
+        // second layer's weights
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float d = sd2[(4 * s + q) * MLP_LDH + 16 * w + i];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                g2[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(d, sh1[(4 * s + q) * MLP_LDH + 16 * k + i], g2[k], 0, 0, 0);
+        }
+        WAVE_SYNC();  // sd1's columns 16 w.. are this wave's own
+        // first layer's weights; columns 40.. are the targets' and dropped
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float d = sd1[(4 * s + q) * MLP_LDH + 16 * w + i];
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                g1[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(d, X[(4 * s + q) * MLP_LDX + 16 * k + i], g1[k], 0, 0, 0);
+        }
+        // the next tile's pairs go to the other buffer; sh1 is written after its barrier
     }
-    if (threadIdx.x == 0) out[0] = part[0] / (float)n;
+
+    float *P = part + (size_t)blockIdx.x * MLP_PART;
+    FloatQuad *P4 = reinterpret_cast<FloatQuad *>(P) + tid;
+    auto put = [&](int k, const v4 &g) { P4[k * MLP_THREADS] = FloatQuad{{g[0], g[1], g[2], g[3]}}; };
+#pragma unroll
+    for (int k = 0; k < 3; ++k) put(k, g1[k]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) put(3 + k, g2[k]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) put(11 + k, g3[k]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int j = 16 * w + 4 * q + r;
+        const float s1 = row_sum16(gb1[r]), s2 = row_sum16(gb2[r]);
+        if (i == 0) {
+            P[MLP_PART_B + j] = s1;
+            P[MLP_PART_B + H + j] = s2;
+        }
+    }
+    gb3 = row_sum16(gb3);
+    loss = row_sum16(loss);
+    if (i == 0) {
+        if (oj < NO) P[MLP_PART_B + 2 * H + oj] = gb3;
+        sred[oj] = loss;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        float l = 0.0f;
+        for (int k = 0; k < MLP_THREADS / 16; ++k) l += sred[k];
+        P[MLP_PART_LOSS] = l;
+    }
+}
+
+// Sums of the workgroups' partials in a fixed order: thread (column c, quarter
+// g) of a block adds its quarter of the workgroups.
+constexpr int MLP_SUM_COLS = 64;
+__global__ void __launch_bounds__(256)
+    mlp_sum_kernel(const float *__restrict__ part, int groups, int n, float *__restrict__ grad, float *__restrict__ loss) {
+    __shared__ float sp[4][MLP_SUM_COLS];
+    const int c = threadIdx.x & (MLP_SUM_COLS - 1), g = threadIdx.x / MLP_SUM_COLS;
+    const int col = blockIdx.x * MLP_SUM_COLS + c;
+    const int per = (groups + 3) / 4, g0 = min(groups, g * per), g1 = min(groups, g0 + per);
+    float acc = 0.0f;
+    if (col <= MLP_PART_LOSS) {
+        const float *p = part + col;
+#pragma unroll 16
+        for (int k = g0; k < g1; ++k) acc += p[(size_t)k * MLP_PART];
+    }
+    sp[g][c] = acc;
+    __syncthreads();
+    if (g != 0 || col > MLP_PART_LOSS) return;
+    const float v = (sp[0][c] + sp[1][c]) + (sp[2][c] + sp[3][c]);
+    if (col == MLP_PART_LOSS) {
+        loss[0] = v / (float)MLP_OUT / (float)n;
+    } else if (col >= MLP_PART_B) {
+        const int j = col - MLP_PART_B;
+        grad[(j < MLP_H) ? MLP_B1 + j : (j < 2 * MLP_H) ? MLP_B2 + j - MLP_H : MLP_B3 + j - 2 * MLP_H] = v;
+    } else {
+        // tile k, thread (wave w, lane (i, q)), float r: row 4 q + r and column i of the tile
+        const int k = col / (4 * MLP_THREADS), th = (col >> 2) & (MLP_THREADS - 1);
+        const int w = th >> 6, i = th & 15, row = 4 * ((th >> 4) & 3) + (col & 3);
+        if (k < 3) {
+            if (16 * k + i < MLP_IN) grad[MLP_W1 + (16 * w + row) * MLP_IN + 16 * k + i] = v;
+        } else if (k < 11) {
+            grad[MLP_W2 + (16 * w + row) * MLP_H + 16 * (k - 3) + i] = v;
+        } else if (16 * (k - 11) + row < MLP_OUT) {
+            grad[MLP_W3 + (16 * (k - 11) + row) * MLP_H + 16 * w + i] = v;
+        }
+    }
 }
 
 // Adam (Kingma and Ba, 2015); c1 = 1 - beta1^step, c2 = 1 - beta2^step.
@@ -6559,20 +6747,15 @@ int cuslines_tap_count(cuslines_tracker *t, int64_t *out2, int reset) {
     return CUSLINES_OK;
 }
 
-// H1 H2 dH2 dH1, O dO, loss; then the weight-gradient partials of the largest layer
-static size_t mlp_ws_floats(int n) {
-    const size_t nchunk = (size_t)((n + WGRAD_CHUNK - 1) / WGRAD_CHUNK);
-    return (size_t)n * (4 * MLP_H + 2 * MLP_OUT + 1) + nchunk * MLP_H * (MLP_H + 1);
-}
+// Workgroups of the training kernel: one per tile of pairs up to one per CU.
+static int mlp_groups(int n) { return std::min((n + MLP_TILE - 1) / MLP_TILE, MLP_GROUPS); }
 
-// The weight-gradient partials take one grid row per WGRAD_CHUNK pairs, and a
-// grid has at most 65535 rows.
-constexpr int MLP_MAX_PAIRS = 65535 * WGRAD_CHUNK;
+constexpr int MLP_MAX_PAIRS = 65535 * 128;
 
 int cuslines_mlp_workspace_bytes(int32_t n, size_t *bytes) {
     if (!bytes || n <= 0) return fail(CUSLINES_EINVAL, "n > 0 and bytes required");
     if (n > MLP_MAX_PAIRS) return fail(CUSLINES_EINVAL, "at most 8,388,480 pairs per training call");
-    *bytes = mlp_ws_floats(n) * sizeof(float);
+    *bytes = (size_t)mlp_groups(n) * MLP_PART * sizeof(float);
     return CUSLINES_OK;
 }
 
@@ -6582,42 +6765,12 @@ int cuslines_mlp_loss_grad_async(cuslines_tracker *t, const float *params_d, con
         return fail(CUSLINES_EINVAL, "null argument or n <= 0");
     if (n > MLP_MAX_PAIRS) return fail(CUSLINES_EINVAL, "at most 8,388,480 pairs per training call");
     HIPC(hipSetDevice(t->device));
-    float *H1 = static_cast<float *>(work_d);
-    float *H2 = H1 + (size_t)n * MLP_H;
-    float *O = H2 + (size_t)n * MLP_H;
-    float *dO = O + (size_t)n * MLP_OUT;
-    float *dH2 = dO + (size_t)n * MLP_OUT;
-    float *dH1 = dH2 + (size_t)n * MLP_H;
-    float *ls = dH1 + (size_t)n * MLP_H;
-    float *part = ls + n;
-    const unsigned nchunk = (unsigned)((n + WGRAD_CHUNK - 1) / WGRAD_CHUNK);
-    const float *X = pairs_d;
-    const int LD = CUSLINES_PAIR_FLOATS;
-    auto g1 = [](long long cnt) { return dim3((unsigned)((cnt + 255) / 256)); };
-    hipStream_t st = t->stream;
-    hipLaunchKernelGGL((mlp_fwd_layer<MLP_IN, MLP_H, true>), g1((long long)n * MLP_H), dim3(256), 0, st, params_d,
-                       MLP_W1, MLP_B1, X, LD, n, H1);
-    hipLaunchKernelGGL((mlp_fwd_layer<MLP_H, MLP_H, true>), g1((long long)n * MLP_H), dim3(256), 0, st, params_d,
-                       MLP_W2, MLP_B2, H1, MLP_H, n, H2);
-    hipLaunchKernelGGL((mlp_fwd_layer<MLP_H, MLP_OUT, false>), g1((long long)n * MLP_OUT), dim3(256), 0, st,
-                       params_d, MLP_W3, MLP_B3, H2, MLP_H, n, O);
-    hipLaunchKernelGGL(mlp_loss_out, g1(n), dim3(256), 0, st, O, X, n, dO, ls);
-    auto wgrad = [&](auto part_k, auto sum_k, int tiles, const float *dout, const float *in, int ld, int w, int b) {
-        hipLaunchKernelGGL(part_k, dim3((unsigned)((tiles + 255) / 256), nchunk), dim3(256), 0, st, dout, in, ld, n,
-                           part);
-        hipLaunchKernelGGL(sum_k, g1(tiles), dim3(256), 0, st, part, (int)nchunk, grad_d, w, b);
-    };
-    wgrad(mlp_wgrad_part<MLP_OUT, MLP_H>, mlp_wgrad_sum<MLP_OUT, MLP_H>, MLP_OUT * (MLP_H + 1), dO, H2, MLP_H, MLP_W3,
-          MLP_B3);
-    hipLaunchKernelGGL((mlp_bwd_input<MLP_OUT, MLP_H>), g1((long long)n * MLP_H), dim3(256), 0, st, params_d, MLP_W3,
-                       dO, H2, n, dH2);
-    wgrad(mlp_wgrad_part<MLP_H, MLP_H>, mlp_wgrad_sum<MLP_H, MLP_H>, MLP_H * (MLP_H + 1), dH2, H1, MLP_H, MLP_W2,
-          MLP_B2);
-    hipLaunchKernelGGL((mlp_bwd_input<MLP_H, MLP_H>), g1((long long)n * MLP_H), dim3(256), 0, st, params_d, MLP_W2,
-                       dH2, H1, n, dH1);
-    wgrad(mlp_wgrad_part<MLP_H, MLP_IN>, mlp_wgrad_sum<MLP_H, MLP_IN>, MLP_H * (MLP_IN + 1), dH1, X, LD, MLP_W1,
-          MLP_B1);
-    hipLaunchKernelGGL(mean_kernel, dim3(1), dim3(256), 0, st, ls, n, loss_d);
+    float *part = static_cast<float *>(work_d);
+    const int groups = mlp_groups(n);
+    hipLaunchKernelGGL(mlp_train_kernel, dim3((unsigned)groups), dim3(MLP_THREADS), 0, t->stream, params_d, pairs_d, n,
+                       part);
+    hipLaunchKernelGGL(mlp_sum_kernel, dim3(MLP_PART_LOSS / MLP_SUM_COLS + 1), dim3(256), 0, t->stream, part,
+                       groups, n, grad_d, loss_d);
     HIPC(hipGetLastError());
     return CUSLINES_OK;
 }
