@@ -26,9 +26,18 @@ class DeviceBuffer:
         p = C.c_void_p()
         _lib.check(dt.L.cuslines_device_alloc(dt.h, max(self.nbytes, 4), C.byref(p)), "device_alloc")
         self.ptr = p.value
+        self._owner = True
+
+    def part(self, offset: int, nbytes: int) -> "DeviceBuffer":
+        """``nbytes`` of this buffer from ``offset``; freed with this buffer."""
+        if offset < 0 or nbytes < 0 or offset + nbytes > self.nbytes:
+            raise ValueError("outside the device buffer")
+        b = DeviceBuffer.__new__(DeviceBuffer)
+        b.dt, b.nbytes, b.ptr, b._owner = self.dt, int(nbytes), self.ptr + int(offset), False
+        return b
 
     def free(self):
-        if self.ptr is not None and self.dt.h:
+        if self.ptr is not None and self.dt.h and self._owner:
             _lib.check(self.dt.L.cuslines_device_free(self.dt.h, C.c_void_p(self.ptr)), "device_free", hard=False)
         self.ptr = None
 

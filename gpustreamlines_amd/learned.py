@@ -84,10 +84,10 @@ class Trainer:
         self.batch = int(batch)
         p0 = init_params() if params is None else np.ascontiguousarray(params, dtype=np.float32)
         self.p = dt.alloc(4 * NPARAM)
-        self.g = dt.alloc(4 * NPARAM)
+        self.g = dt.alloc(4 * (NPARAM + 1))  # the gradient, then the loss: one copy fetches both
         self.m = dt.alloc(4 * NPARAM)
         self.v = dt.alloc(4 * NPARAM)
-        self.loss = dt.alloc(4)
+        self.loss = self.g.part(4 * NPARAM, 4)
         self.work = dt.alloc(dt.mlp_workspace_bytes(self.batch))
         self.p.upload(p0)
         z = np.zeros(NPARAM, np.float32)
@@ -98,8 +98,10 @@ class Trainer:
     def loss_grad(self, pairs_ptr: int, n: int):
         """(mean loss, gradient) of n <= batch pairs at the current parameters."""
         self.dt.mlp_loss_grad_async(self.p.ptr, pairs_ptr, n, self.loss.ptr, self.g.ptr, self.work.ptr)
-        self.dt.synchronize()
-        return float(self.loss.download(np.zeros(1, np.float32))[0]), self.g.download(np.zeros(NPARAM, np.float32))
+        # the copy runs on the kernels' stream and waits for itself: 50 us for 4096 pairs,
+        # 75 with a wait for the kernels and a copy each for loss and gradient
+        out = self.g.download(np.zeros(NPARAM + 1, np.float32))
+        return float(out[NPARAM]), out[:NPARAM]
 
     def fit(self, pairs, n_pairs: int, epochs: int = 3, lr: float = 1e-3, lr_final: float = 1e-4,
             holdout: int = 0):
