@@ -687,17 +687,92 @@ __device__ __forceinline__ float gemv_xf(float x) {
 // the 16-byte row loads of one instruction are 512 contiguous bytes; else
 // row-major.  x comes from LDS as broadcast reads and must be 16-byte
 // aligned, already transformed (gemv_xf).
+// Four of these products are three quarters of an exact attempt's time (170 k
+// cycles for a lone slot), and each waits for its matrix's blocks from L2
+// (some 1200 cycles) rather than for its sums: a step reads 282 KB of matrices.
+// With a block in flight behind the one being summed, no branch per column,
+// the gather on 16-byte loads and 2 waves per SIMD: CSA 200 seeds 79 -> 65 ms,
+// 3001 (46x55x41) 99 -> 82 ms, 20 000 (81x106x76) 258 -> 212 ms, OPDT 5000
+// 153 -> 127 ms.  Out of line, the products are faster for few seeds (3001: 77
+// ms) but take the kernel to one wave per SIMD (20 000: 260 ms).
 __host__ __device__ inline size_t mat_offset(int M, int i, int j) {
     return (((size_t)(i >> 5) * (size_t)(M >> 2) + (size_t)(j >> 2)) << 7) + (size_t)((i & 31) << 2) + (size_t)(j & 3);
 }
 
-__device__ void gemv_lanerow(int N, int M, const float *x, const float *__restrict__ mat, float *out) {
+__device__ __forceinline__ void gemv_lanerow(int N, int M, const float *x, const float *__restrict__ mat, float *out) {
     const int l = lane32();
-    const bool vec = (M & 3) == 0;
+    if ((M & 3) == 0) {
+        // 32 rows by 32 columns a block; the next block's loads, of the same
+        // rows or the next ones, are in flight while a block is summed.
+        const int nblk = (M + 31) >> 5, total = nblk * ((N + 31) >> 5);
+        auto load = [&](int i0, int j0, float4 (&m)[8]) {
+            const int nq = min(8, (M - j0) >> 2);
+            const float *row = mat + mat_offset(M, min(i0 + l, N - 1), j0);  // past the last row: re-read, dropped
+#pragma unroll
+            for (int q = 0; q < 8; ++q)  // past the last column: the last valid one, its product dropped
+                m[q] = *reinterpret_cast<const float4 *>(row + ((size_t)(4 * min(q, nq - 1)) << 5));
+        };
+        float p[32];
+#pragma unroll
+        for (int q = 0; q < 32; ++q) p[q] = 0.0f;
+        float4 m[2][8];
+        load(0, 0, m[0]);
+        int i0 = 0, j0 = 0;
+        auto block = [&](const float4 (&cur)[8], float4 (&nxt)[8], bool more) {
+            int i1 = i0, j1 = j0 + 32;
+            if (j1 >= M) { j1 = 0; i1 += 32; }
+            if (more) load(i1, j1, nxt);
+            const int nq = (M - j0) >> 2;
+            float4 v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = *reinterpret_cast<const float4 *>(x + j0 + 4 * min(q, nq - 1));
+            if (nq >= 8) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    p[4 * q] = __builtin_fmaf(v[q].x, cur[q].x, p[4 * q]);
+                    p[4 * q + 1] = __builtin_fmaf(v[q].y, cur[q].y, p[4 * q + 1]);
+                    p[4 * q + 2] = __builtin_fmaf(v[q].z, cur[q].z, p[4 * q + 2]);
+                    p[4 * q + 3] = __builtin_fmaf(v[q].w, cur[q].w, p[4 * q + 3]);
+                }
+            } else {
+                int nqv = nq;
+                asm volatile("" : "+v"(nqv));  // selects: a branch each would wait for each product
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const bool in = q < nqv;
+                    const float a0 = __builtin_fmaf(v[q].x, cur[q].x, p[4 * q]);
+                    const float a1 = __builtin_fmaf(v[q].y, cur[q].y, p[4 * q + 1]);
+                    const float a2 = __builtin_fmaf(v[q].z, cur[q].z, p[4 * q + 2]);
+                    const float a3 = __builtin_fmaf(v[q].w, cur[q].w, p[4 * q + 3]);
+                    p[4 * q] = in ? a0 : p[4 * q];
+                    p[4 * q + 1] = in ? a1 : p[4 * q + 1];
+                    p[4 * q + 2] = in ? a2 : p[4 * q + 2];
+                    p[4 * q + 3] = in ? a3 : p[4 * q + 3];
+                }
+            }
+            if (j1 == 0) {
+#pragma unroll
+                for (int d = 16; d >= 1; d >>= 1)
+#pragma unroll
+                    for (int q = 0; q < d; ++q) p[q] = p[q] + p[q + d];
+                if (i0 + l < N) out[i0 + l] = p[0];
+#pragma unroll
+                for (int q = 0; q < 32; ++q) p[q] = 0.0f;
+            }
+            i0 = i1;
+            j0 = j1;
+        };
+        for (int it = 0; it < total; it += 2) {
+            block(m[0], m[1], it + 1 < total);
+            if (it + 1 < total) block(m[1], m[0], it + 2 < total);
+        }
+        WAVE_SYNC();
+        return;
+    }
     for (int i0 = 0; i0 < N; i0 += 32) {
         const int i = i0 + l;
         if (i < N) {
-            const float *row = vec ? mat + mat_offset(M, i, 0) : mat + (size_t)i * M;
+            const float *row = mat + (size_t)i * M;
             float p[32];
 #pragma unroll
             for (int q = 0; q < 32; ++q) p[q] = 0.0f;
@@ -706,35 +781,17 @@ __device__ void gemv_lanerow(int N, int M, const float *x, const float *__restri
                 // column past M re-reads the block's last valid one, and its
                 // product is dropped by the select, so no load sits behind a
                 // branch (and none leaves the matrix).
-                const int nj = min(32, M - j0);
-                if (vec) {  // M % 4 == 0: a vector is all in or all out
-                    const int nq = nj >> 2;
-                    float4 m[8];
+                int nj = min(32, M - j0);
+                float m[32], v[32];
 #pragma unroll
-                    for (int q = 0; q < 8; ++q)
-                        m[q] = *reinterpret_cast<const float4 *>(row + ((size_t)(j0 + 4 * min(q, nq - 1)) << 5));
+                for (int q = 0; q < 32; ++q) m[q] = row[j0 + min(q, nj - 1)];
 #pragma unroll
-                    for (int q = 0; q < 8; ++q) {
-                        const float4 v = *reinterpret_cast<const float4 *>(x + j0 + 4 * q);
-                        const bool in = q < nq;
-                        const float a0 = __builtin_fmaf(v.x, m[q].x, p[4 * q]);
-                        const float a1 = __builtin_fmaf(v.y, m[q].y, p[4 * q + 1]);
-                        const float a2 = __builtin_fmaf(v.z, m[q].z, p[4 * q + 2]);
-                        const float a3 = __builtin_fmaf(v.w, m[q].w, p[4 * q + 3]);
-                        p[4 * q] = in ? a0 : p[4 * q];
-                        p[4 * q + 1] = in ? a1 : p[4 * q + 1];
-                        p[4 * q + 2] = in ? a2 : p[4 * q + 2];
-                        p[4 * q + 3] = in ? a3 : p[4 * q + 3];
-                    }
-                } else {
-                    float m[32];
+                for (int q = 0; q < 32; ++q) v[q] = x[j0 + min(q, nj - 1)];
+                asm volatile("" : "+v"(nj));  // selects: a branch each would wait for each product
 #pragma unroll
-                    for (int q = 0; q < 32; ++q) m[q] = row[j0 + min(q, nj - 1)];
-#pragma unroll
-                    for (int q = 0; q < 32; ++q) {
-                        const float a = __builtin_fmaf(x[j0 + q], m[q], p[q]);
-                        p[q] = (q < nj) ? a : p[q];
-                    }
+                for (int q = 0; q < 32; ++q) {
+                    const float a = __builtin_fmaf(v[q], m[q], p[q]);
+                    p[q] = (q < nj) ? a : p[q];
                 }
             }
 #pragma unroll
@@ -869,6 +926,48 @@ struct SlotRng<CUSLINES_PROB> {
     typedef ProbStream<32> type;
 };
 
+// trilinear on 16-byte loads: lane l owns channels 128 c + 4 l .. + 3, a
+// chunk's 8 corner loads in flight (two chunks' 64 registers spill at 4 waves
+// per SIMD: 25,000 seeds 101 instead of 91 ms).  False outside the volume.
+__device__ __forceinline__ bool bb_gather(const DevParams &P, const float *__restrict__ data, float px, float py,
+                                          float pz, float *out) {
+    if ((px < -0.5f) | (px + 0.5f >= (float)P.dimx) | (py < -0.5f) | (py + 0.5f >= (float)P.dimy) | (pz < -0.5f) |
+        (pz + 0.5f >= (float)P.dimz))
+        return false;
+    const int l = lane32();
+    const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+    const float wx1 = px - fx, wy1 = py - fy, wz1 = pz - fz;
+    const float wx0 = 1.0f - wx1, wy0 = 1.0f - wy1, wz0 = 1.0f - wz1;
+    const int x0 = (int)((0.0f > fx) ? 0.0f : fx), y0 = (int)((0.0f > fy) ? 0.0f : fy),
+              z0 = (int)((0.0f > fz) ? 0.0f : fz);
+    const float w[8] = {(wx0 * wy0) * wz0, (wx0 * wy0) * wz1, (wx0 * wy1) * wz0, (wx0 * wy1) * wz1,
+                        (wx1 * wy0) * wz0, (wx1 * wy0) * wz1, (wx1 * wy1) * wz0, (wx1 * wy1) * wz1};
+    const uint32_t dzv = (z0 + 1 < P.dimz) ? 1u : 0u;
+    const uint32_t dyv = (y0 + 1 < P.dimy) ? (uint32_t)P.dimz : 0u;
+    const uint32_t dxv = (x0 + 1 < P.dimx) ? (uint32_t)P.dimy * (uint32_t)P.dimz : 0u;
+    const uint32_t vox = ((uint32_t)x0 * (uint32_t)P.dimy + (uint32_t)y0) * (uint32_t)P.dimz + (uint32_t)z0;
+    const float *c[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        c[k] = data + (uint64_t)(vox + ((k & 4) ? dxv : 0u) + ((k & 2) ? dyv : 0u) + ((k & 1) ? dzv : 0u)) *
+                          (uint32_t)P.t32;
+    for (int t0 = 0; t0 < P.t32; t0 += 128) {
+        const int ta = t0 + 4 * l;
+        const int sa = min(ta, P.t32 - 4);  // past the row: re-read, dropped
+        float4 va[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) va[k] = *reinterpret_cast<const float4 *>(c[k] + sa);
+        float4 a = float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            a.x = __builtin_fmaf(w[k], va[k].x, a.x); a.y = __builtin_fmaf(w[k], va[k].y, a.y);
+            a.z = __builtin_fmaf(w[k], va[k].z, a.z); a.w = __builtin_fmaf(w[k], va[k].w, a.w);
+        }
+        if (ta < P.t32) *reinterpret_cast<float4 *>(out + ta) = a;
+    }
+    return true;
+}
+
 // -------------------------------------------------------------------------
 // Bootstrap getter (boot.cu:19-113, 115-193, 330-608)
 // -------------------------------------------------------------------------
@@ -914,7 +1013,7 @@ __device__ int get_direction_boot(const DevParams &P, const DevBufs &B, const fl
     const int l = lane32();
     const int hr = P.hr, dn = P.delta_nr, nv = P.nverts, T = P.dimt;
     for (int att = 0; att < nattempts; ++att) {
-        const int rv = trilinear(P, B.data, P.t32, T, px, py, pz, S.vox);
+        const int rv = bb_gather(P, B.data, px, py, pz, S.vox) ? 0 : -1;
         WAVE_SYNC();
         if (rv == 0) {
             for (int m = l; m < hr; m += 32) S.msk[m] = S.vox[B.dwi_idx[m]];
@@ -3854,9 +3953,9 @@ __global__ void __launch_bounds__(256) phase2_kernel(DevParams P, DevBufs B, con
 // the seeds in processing order; `work` holds QUEUES zeroed counters.  The
 // order changes no result: random streams and output slots follow the seed
 // index.
-// Plain PTT is held to 128 VGPRs (4 waves per SIMD): the few spills cost less
-// than the latency hiding gained (+8% at 200k seeds).  Bootstrap likewise
-// (4 waves per SIMD, which its 5 KB of LDS per slot allows: +13% CSA).  The
+// Bootstrap takes 256 VGPRs (2 waves per SIMD): at 128 it spills 140 of them and
+// its products' loads in flight too (CSA 3001 seeds 87 ms at 2, 95 at 3, 99 at
+// 4 waves; 20 000 seeds 217, 228 and 270 ms).  The
 // flat loop of the learned proposal (V == 5) needs about 170 VGPRs and at 128
 // spills inside its loop, so it runs at 3 waves per SIMD (168 VGPRs), in
 // 768-thread workgroups (one staged copy of the network serves 24 slots).
@@ -3866,7 +3965,7 @@ __global__ void __launch_bounds__((MODEL == CUSLINES_PTT && V == 1)   ? 512
                                                                       : 256,
                                   (MODEL == CUSLINES_PTT && V == 5) ? 3
                                   : (MODEL == CUSLINES_PTT && V != 2)           ? 4
-                                                                                : (MODEL <= CUSLINES_PROB ? 4 : 1))
+                                                                                : (MODEL <= CUSLINES_CSA ? 2 : MODEL <= CUSLINES_PROB ? 4 : 1))
     phase2_queue_kernel(DevParams P, DevBufs B, const float *__restrict__ seeds,
                                                            int nseeds, int rng_chunk, const int *__restrict__ offsets,
                                                            const int *__restrict__ dirs, int *__restrict__ sline_seed,
@@ -4376,48 +4475,6 @@ __device__ void bb_end_pass(const DevParams &P, const DevBufs &B, BbSlot &st, Ph
     }
     bb_next_seed(P, B, st, rng, nseeds, seeds, rng_chunk, offsets, dirs, order, work, sline);
     if (!st.done) bb_start_pass(P, st, sline);
-}
-
-// trilinear on 16-byte loads: lane l owns channels 128 c + 4 l .. + 3, a
-// chunk's 8 corner loads in flight (two chunks' 64 registers spill at 4 waves
-// per SIMD: 25,000 seeds 101 instead of 91 ms).  False outside the volume.
-__device__ __forceinline__ bool bb_gather(const DevParams &P, const float *__restrict__ data, float px, float py,
-                                          float pz, float *out) {
-    if ((px < -0.5f) | (px + 0.5f >= (float)P.dimx) | (py < -0.5f) | (py + 0.5f >= (float)P.dimy) | (pz < -0.5f) |
-        (pz + 0.5f >= (float)P.dimz))
-        return false;
-    const int l = lane32();
-    const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
-    const float wx1 = px - fx, wy1 = py - fy, wz1 = pz - fz;
-    const float wx0 = 1.0f - wx1, wy0 = 1.0f - wy1, wz0 = 1.0f - wz1;
-    const int x0 = (int)((0.0f > fx) ? 0.0f : fx), y0 = (int)((0.0f > fy) ? 0.0f : fy),
-              z0 = (int)((0.0f > fz) ? 0.0f : fz);
-    const float w[8] = {(wx0 * wy0) * wz0, (wx0 * wy0) * wz1, (wx0 * wy1) * wz0, (wx0 * wy1) * wz1,
-                        (wx1 * wy0) * wz0, (wx1 * wy0) * wz1, (wx1 * wy1) * wz0, (wx1 * wy1) * wz1};
-    const uint32_t dzv = (z0 + 1 < P.dimz) ? 1u : 0u;
-    const uint32_t dyv = (y0 + 1 < P.dimy) ? (uint32_t)P.dimz : 0u;
-    const uint32_t dxv = (x0 + 1 < P.dimx) ? (uint32_t)P.dimy * (uint32_t)P.dimz : 0u;
-    const uint32_t vox = ((uint32_t)x0 * (uint32_t)P.dimy + (uint32_t)y0) * (uint32_t)P.dimz + (uint32_t)z0;
-    const float *c[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-        c[k] = data + (uint64_t)(vox + ((k & 4) ? dxv : 0u) + ((k & 2) ? dyv : 0u) + ((k & 1) ? dzv : 0u)) *
-                          (uint32_t)P.t32;
-    for (int t0 = 0; t0 < P.t32; t0 += 128) {
-        const int ta = t0 + 4 * l;
-        const int sa = min(ta, P.t32 - 4);  // past the row: re-read, dropped
-        float4 va[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) va[k] = *reinterpret_cast<const float4 *>(c[k] + sa);
-        float4 a = float4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            a.x = __builtin_fmaf(w[k], va[k].x, a.x); a.y = __builtin_fmaf(w[k], va[k].y, a.y);
-            a.z = __builtin_fmaf(w[k], va[k].z, a.z); a.w = __builtin_fmaf(w[k], va[k].w, a.w);
-        }
-        if (ta < P.t32) *reinterpret_cast<float4 *>(out + ta) = a;
-    }
-    return true;
 }
 
 // OCC: waves per SIMD the kernel is compiled for (2: 185 VGPRs and one
