@@ -4783,13 +4783,14 @@ __global__ void seed_scatter(const int *__restrict__ key, int n, const int *__re
 // gradients once; activations stay in LDS.  The products run on
 // v_mfma_f32_16x16x4_f32 (fp32 operands and sums); wave w owns hidden neurons
 // 16 w .. 16 w + 15 of both layers.
-// At the default 4096 pairs every workgroup has one tile, and what bounds it is
-// latency: reading the weights (10 us), seven short phases between barriers
-// (8 us), writing and re-reading MLP_GROUPS partials (27 MB, 7 + 5 us).  Loss and
-// gradient of 4096 pairs 360 -> 75 us with both copies to the host; the layer
-// by layer, element by element kernels before took 13 launches and re-read
-// the weights for every pair.  60 000 pairs: 94 us, 15 tiles a workgroup at 5 us,
-// where the matrix products alone are 3.6 us.
+// What bounds it at the default 4096 pairs is latency: reading the weights
+// (10 us), seven short phases between barriers a tile (5-8 us, three tiles a
+// workgroup), writing and re-reading the partials (11 MB).  Loss and gradient of
+// 4096 pairs 361 -> 58 us with the copy to the host; the layer by layer,
+// element by element kernels before took 13 launches and re-read the weights for
+// every pair.  With room in the workspace for 256 partials, one tile each, it
+// is 49 us.  60 000 pairs: 94 us, 15 tiles a workgroup at 5 us, where the matrix
+// products alone are 3.6 us.
 // -------------------------------------------------------------------------
 __device__ __forceinline__ float bf16_round(float x) {  // to the nearest bf16, ties to even
     uint32_t b = __float_as_uint(x);
@@ -4810,6 +4811,21 @@ static_assert(MLP_H == 16 * MLP_THREADS / 64 && MLP_IN % 4 == 0 && MLP_OUT <= 32
 // of 16 consecutive floats overlap little (reads across the rows).
 constexpr int MLP_LDX = 84, MLP_LDH = 148, MLP_LDO = 36;
 
+// The parameter that float `col` (before the loss) of a partial belongs to, -1
+// for a tile's rows and columns past the layer's.
+__device__ __forceinline__ int mlp_part_param(int col) {
+    if (col >= MLP_PART_B) {
+        const int j = col - MLP_PART_B;
+        return (j < MLP_H) ? MLP_B1 + j : (j < 2 * MLP_H) ? MLP_B2 + j - MLP_H : MLP_B3 + j - 2 * MLP_H;
+    }
+    // tile k, thread (wave w, lane (i, q)), float r: row 4 q + r and column i of the tile
+    const int k = col / (4 * MLP_THREADS), th = (col >> 2) & (MLP_THREADS - 1);
+    const int w = th >> 6, i = th & 15, row = 4 * ((th >> 4) & 3) + (col & 3);
+    if (k < 3) return (16 * k + i < MLP_IN) ? MLP_W1 + (16 * w + row) * MLP_IN + 16 * k + i : -1;
+    if (k < 11) return MLP_W2 + (16 * w + row) * MLP_H + 16 * (k - 3) + i;
+    return (16 * (k - 11) + row < MLP_OUT) ? MLP_W3 + (16 * (k - 11) + row) * MLP_H + 16 * w + i : -1;
+}
+
 struct __attribute__((packed, aligned(4))) FloatQuad {  // 16 bytes at any float's address
     float v[4];
 };
@@ -4823,7 +4839,8 @@ __device__ __forceinline__ float row_sum16(float v) {  // sum over the 16 lanes 
 }
 
 __global__ void __launch_bounds__(MLP_THREADS, 2)
-    mlp_train_kernel(const float *__restrict__ prm, const float *__restrict__ pairs, int n, float *__restrict__ part) {
+    mlp_train_kernel(const float *__restrict__ prm, const float *__restrict__ pairs, int n, float *__restrict__ part,
+                     float *__restrict__ grad, float *__restrict__ mean_loss) {
     __shared__ __align__(16) float sx[2][MLP_TILE * MLP_LDX];  // pairs: 40 inputs, 24 targets
     __shared__ __align__(16) float sh1[MLP_TILE * MLP_LDH], sh2[MLP_TILE * MLP_LDH];
     __shared__ __align__(16) float sd1[MLP_TILE * MLP_LDH], sd2[MLP_TILE * MLP_LDH];  // gradients at the hidden layers
@@ -4996,9 +5013,24 @@ __global__ void __launch_bounds__(MLP_THREADS, 2)
         // the next tile's pairs go to the other buffer; sh1 is written after its barrier
     }
 
+    // the lanes' tiles as they are; a lone workgroup's, and its sums, to their places
+    const bool lone = gridDim.x == 1;
     float *P = part + (size_t)blockIdx.x * MLP_PART;
-    FloatQuad *P4 = reinterpret_cast<FloatQuad *>(P) + tid;
-    auto put = [&](int k, const v4 &g) { P4[k * MLP_THREADS] = FloatQuad{{g[0], g[1], g[2], g[3]}}; };
+    auto put = [&](int k, const v4 &g) {
+        if (!lone) {
+            reinterpret_cast<FloatQuad *>(P)[k * MLP_THREADS + tid] = FloatQuad{{g[0], g[1], g[2], g[3]}};
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int at = mlp_part_param(4 * (k * MLP_THREADS + tid) + r);
+                if (at >= 0) grad[at] = g[r];
+            }
+        }
+    };
+    auto put1 = [&](int at, float v) {
+        if (lone) grad[mlp_part_param(at)] = v;
+        else P[at] = v;
+    };
 #pragma unroll
     for (int k = 0; k < 3; ++k) put(k, g1[k]);
 #pragma unroll
@@ -5010,21 +5042,22 @@ __global__ void __launch_bounds__(MLP_THREADS, 2)
         const int j = 16 * w + 4 * q + r;
         const float s1 = row_sum16(gb1[r]), s2 = row_sum16(gb2[r]);
         if (i == 0) {
-            P[MLP_PART_B + j] = s1;
-            P[MLP_PART_B + H + j] = s2;
+            put1(MLP_PART_B + j, s1);
+            put1(MLP_PART_B + H + j, s2);
         }
     }
     gb3 = row_sum16(gb3);
     loss = row_sum16(loss);
     if (i == 0) {
-        if (oj < NO) P[MLP_PART_B + 2 * H + oj] = gb3;
+        if (oj < NO) put1(MLP_PART_B + 2 * H + oj, gb3);
         sred[oj] = loss;
     }
     __syncthreads();
     if (tid == 0) {
         float l = 0.0f;
         for (int k = 0; k < MLP_THREADS / 16; ++k) l += sred[k];
-        P[MLP_PART_LOSS] = l;
+        if (lone) mean_loss[0] = l / (float)NO / (float)n;
+        else P[MLP_PART_LOSS] = l;
     }
 }
 
@@ -5049,20 +5082,9 @@ __global__ void __launch_bounds__(256)
     const float v = (sp[0][c] + sp[1][c]) + (sp[2][c] + sp[3][c]);
     if (col == MLP_PART_LOSS) {
         loss[0] = v / (float)MLP_OUT / (float)n;
-    } else if (col >= MLP_PART_B) {
-        const int j = col - MLP_PART_B;
-        grad[(j < MLP_H) ? MLP_B1 + j : (j < 2 * MLP_H) ? MLP_B2 + j - MLP_H : MLP_B3 + j - 2 * MLP_H] = v;
     } else {
-        // tile k, thread (wave w, lane (i, q)), float r: row 4 q + r and column i of the tile
-        const int k = col / (4 * MLP_THREADS), th = (col >> 2) & (MLP_THREADS - 1);
-        const int w = th >> 6, i = th & 15, row = 4 * ((th >> 4) & 3) + (col & 3);
-        if (k < 3) {
-            if (16 * k + i < MLP_IN) grad[MLP_W1 + (16 * w + row) * MLP_IN + 16 * k + i] = v;
-        } else if (k < 11) {
-            grad[MLP_W2 + (16 * w + row) * MLP_H + 16 * (k - 3) + i] = v;
-        } else if (16 * (k - 11) + row < MLP_OUT) {
-            grad[MLP_W3 + (16 * (k - 11) + row) * MLP_H + 16 * w + i] = v;
-        }
+        const int at = mlp_part_param(col);
+        if (at >= 0) grad[at] = v;
     }
 }
 
@@ -6804,15 +6826,25 @@ int cuslines_tap_count(cuslines_tracker *t, int64_t *out2, int reset) {
     return CUSLINES_OK;
 }
 
-// Workgroups of the training kernel: one per tile of pairs up to one per CU.
-static int mlp_groups(int n) { return std::min((n + MLP_TILE - 1) / MLP_TILE, MLP_GROUPS); }
+// Floats of the caller's workspace: 561 a pair and 16,512 for every 128 pairs.
+static size_t mlp_ws_floats(int n) {
+    return (size_t)n * (4 * MLP_H + 2 * MLP_OUT + 1) + ((size_t)n + 127) / 128 * MLP_H * (MLP_H + 1);
+}
+
+// Workgroups of the training kernel: one per tile of pairs, up to one per CU
+// and as many as the workspace has room for (105 at 4096 pairs); a lone one
+// writes the gradient itself.
+static int mlp_groups(int n) {
+    const size_t room = std::max<size_t>(1, mlp_ws_floats(n) / MLP_PART);
+    return (int)std::min<size_t>(room, (size_t)std::min((n + MLP_TILE - 1) / MLP_TILE, MLP_GROUPS));
+}
 
 constexpr int MLP_MAX_PAIRS = 65535 * 128;
 
 int cuslines_mlp_workspace_bytes(int32_t n, size_t *bytes) {
     if (!bytes || n <= 0) return fail(CUSLINES_EINVAL, "n > 0 and bytes required");
     if (n > MLP_MAX_PAIRS) return fail(CUSLINES_EINVAL, "at most 8,388,480 pairs per training call");
-    *bytes = (size_t)mlp_groups(n) * MLP_PART * sizeof(float);
+    *bytes = mlp_ws_floats(n) * sizeof(float);
     return CUSLINES_OK;
 }
 
@@ -6825,9 +6857,10 @@ int cuslines_mlp_loss_grad_async(cuslines_tracker *t, const float *params_d, con
     float *part = static_cast<float *>(work_d);
     const int groups = mlp_groups(n);
     hipLaunchKernelGGL(mlp_train_kernel, dim3((unsigned)groups), dim3(MLP_THREADS), 0, t->stream, params_d, pairs_d, n,
-                       part);
-    hipLaunchKernelGGL(mlp_sum_kernel, dim3(MLP_PART_LOSS / MLP_SUM_COLS + 1), dim3(256), 0, t->stream, part,
-                       groups, n, grad_d, loss_d);
+                       part, grad_d, loss_d);
+    if (groups > 1)
+        hipLaunchKernelGGL(mlp_sum_kernel, dim3(MLP_PART_LOSS / MLP_SUM_COLS + 1), dim3(256), 0, t->stream, part,
+                           groups, n, grad_d, loss_d);
     HIPC(hipGetLastError());
     return CUSLINES_OK;
 }
