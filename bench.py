@@ -271,6 +271,10 @@ def kernel_name(args, lowrank=False):
     if args.getter == "ptt" and args.ptt_lanes:
         kind = "phase2_ptt_flat_kernel" if args.stepping == "flat" else "phase2_ptt_queue_kernel"
         return f"{kind}<{args.ptt_lanes}>"
+    if args.stepping == "flat" and args.getter == "ptt":
+        return "phase2_ptt_kernel"
+    if args.stepping == "flat" and args.getter == "prob":
+        return "phase2_prob_kernel<3>"  # 724 channels: three register chunks of 256
     v = 4 if args.stepping == "flat" else 0
     return f"phase2_queue_kernel<{MODEL_IDS[args.getter]}, {v}>"
 
