@@ -687,19 +687,75 @@ __device__ __forceinline__ float gemv_xf(float x) {
 // the 16-byte row loads of one instruction are 512 contiguous bytes; else
 // row-major.  x comes from LDS as broadcast reads and must be 16-byte
 // aligned, already transformed (gemv_xf).
-// Four of these products are three quarters of an exact attempt's time (170 k
-// cycles for a lone slot), and each waits for its matrix's blocks from L2
-// (some 1200 cycles) rather than for its sums: a step reads 282 KB of matrices.
-// With a block in flight behind the one being summed, no branch per column,
-// the gather on 16-byte loads and 2 waves per SIMD: CSA 200 seeds 79 -> 65 ms,
-// 3001 (46x55x41) 99 -> 82 ms, 20 000 (81x106x76) 258 -> 212 ms, OPDT 5000
-// 153 -> 127 ms.  Out of line, the products are faster for few seeds (3001: 77
-// ms) but take the kernel to one wave per SIMD (20 000: 260 ms).
 __host__ __device__ inline size_t mat_offset(int M, int i, int j) {
     return (((size_t)(i >> 5) * (size_t)(M >> 2) + (size_t)(j >> 2)) << 7) + (size_t)((i & 31) << 2) + (size_t)(j & 3);
 }
 
-__device__ __forceinline__ void gemv_lanerow(int N, int M, const float *x, const float *__restrict__ mat, float *out) {
+__device__ void gemv_lanerow(int N, int M, const float *x, const float *__restrict__ mat, float *out) {
+    const int l = lane32();
+    const bool vec = (M & 3) == 0;
+    for (int i0 = 0; i0 < N; i0 += 32) {
+        const int i = i0 + l;
+        if (i < N) {
+            const float *row = vec ? mat + mat_offset(M, i, 0) : mat + (size_t)i * M;
+            float p[32];
+#pragma unroll
+            for (int q = 0; q < 32; ++q) p[q] = 0.0f;
+            for (int j0 = 0; j0 < M; j0 += 32) {
+                // All loads of the block are issued before the first use: a
+                // column past M re-reads the block's last valid one, and its
+                // product is dropped by the select, so no load sits behind a
+                // branch (and none leaves the matrix).
+                const int nj = min(32, M - j0);
+                if (vec) {  // M % 4 == 0: a vector is all in or all out
+                    const int nq = nj >> 2;
+                    float4 m[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q)
+                        m[q] = *reinterpret_cast<const float4 *>(row + ((size_t)(j0 + 4 * min(q, nq - 1)) << 5));
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        const float4 v = *reinterpret_cast<const float4 *>(x + j0 + 4 * q);
+                        const bool in = q < nq;
+                        const float a0 = __builtin_fmaf(v.x, m[q].x, p[4 * q]);
+                        const float a1 = __builtin_fmaf(v.y, m[q].y, p[4 * q + 1]);
+                        const float a2 = __builtin_fmaf(v.z, m[q].z, p[4 * q + 2]);
+                        const float a3 = __builtin_fmaf(v.w, m[q].w, p[4 * q + 3]);
+                        p[4 * q] = in ? a0 : p[4 * q];
+                        p[4 * q + 1] = in ? a1 : p[4 * q + 1];
+                        p[4 * q + 2] = in ? a2 : p[4 * q + 2];
+                        p[4 * q + 3] = in ? a3 : p[4 * q + 3];
+                    }
+                } else {
+                    float m[32];
+#pragma unroll
+                    for (int q = 0; q < 32; ++q) m[q] = row[j0 + min(q, nj - 1)];
+#pragma unroll
+                    for (int q = 0; q < 32; ++q) {
+                        const float a = __builtin_fmaf(x[j0 + q], m[q], p[q]);
+                        p[q] = (q < nj) ? a : p[q];
+                    }
+                }
+            }
+#pragma unroll
+            for (int d = 16; d >= 1; d >>= 1)
+#pragma unroll
+                for (int q = 0; q < d; ++q) p[q] = p[q] + p[q + d];
+            out[i] = p[0];
+        }
+    }
+    WAVE_SYNC();
+}
+
+// The same sums for the kernel of 2 waves per SIMD.  Four of these products are
+// three quarters of an exact attempt's time (170 k cycles for a lone slot), and
+// each waits for its matrix's blocks from L2 (some 1200 cycles) rather than for
+// its sums: a step reads 282 KB of matrices.  Here the next block's loads are in
+// flight behind the sums, without a branch per column, and with the 256
+// registers they take; launch_phase2 has the rule and its figures.  Out of line,
+// 3001 seeds are faster still (77 ms), but the kernel has one wave per SIMD left
+// (20 000 seeds: 260 ms); two or three blocks ahead spill (213, 233 ms).
+__device__ __forceinline__ void gemv_lanerow_wide(int N, int M, const float *x, const float *__restrict__ mat, float *out) {
     const int l = lane32();
     if ((M & 3) == 0) {
         // 32 rows by 32 columns a block; the next block's loads, of the same
@@ -769,39 +825,7 @@ __device__ __forceinline__ void gemv_lanerow(int N, int M, const float *x, const
         WAVE_SYNC();
         return;
     }
-    for (int i0 = 0; i0 < N; i0 += 32) {
-        const int i = i0 + l;
-        if (i < N) {
-            const float *row = mat + (size_t)i * M;
-            float p[32];
-#pragma unroll
-            for (int q = 0; q < 32; ++q) p[q] = 0.0f;
-            for (int j0 = 0; j0 < M; j0 += 32) {
-                // All loads of the block are issued before the first use: a
-                // column past M re-reads the block's last valid one, and its
-                // product is dropped by the select, so no load sits behind a
-                // branch (and none leaves the matrix).
-                int nj = min(32, M - j0);
-                float m[32], v[32];
-#pragma unroll
-                for (int q = 0; q < 32; ++q) m[q] = row[j0 + min(q, nj - 1)];
-#pragma unroll
-                for (int q = 0; q < 32; ++q) v[q] = x[j0 + min(q, nj - 1)];
-                asm volatile("" : "+v"(nj));  // selects: a branch each would wait for each product
-#pragma unroll
-                for (int q = 0; q < 32; ++q) {
-                    const float a = __builtin_fmaf(v[q], m[q], p[q]);
-                    p[q] = (q < nj) ? a : p[q];
-                }
-            }
-#pragma unroll
-            for (int d = 16; d >= 1; d >>= 1)
-#pragma unroll
-                for (int q = 0; q < d; ++q) p[q] = p[q] + p[q + d];
-            out[i] = p[0];
-        }
-    }
-    WAVE_SYNC();
+    gemv_lanerow(N, M, x, mat, out);
 }
 
 // -------------------------------------------------------------------------
@@ -1006,20 +1030,27 @@ __device__ int closest_peak(const DevParams &P, const float *sv, float dx, float
     return 0;
 }
 
-template <int MODEL>
+// WIDE: the kernel of 2 waves per SIMD.
+template <int MODEL, bool WIDE = false>
 __device__ int get_direction_boot(const DevParams &P, const DevBufs &B, const float *sv, BootLds &S,
                                   Philox &rng, int nattempts, float dx, float dy, float dz, float px,
                                   float py, float pz, float *ndx, float *ndy, float *ndz) {
     const int l = lane32();
+    const auto gemv = [](int N, int M, const float *x, const float *__restrict__ mat, float *out) {
+        if constexpr (WIDE) gemv_lanerow_wide(N, M, x, mat, out);
+        else gemv_lanerow(N, M, x, mat, out);
+    };
     const int hr = P.hr, dn = P.delta_nr, nv = P.nverts, T = P.dimt;
     for (int att = 0; att < nattempts; ++att) {
-        const int rv = bb_gather(P, B.data, px, py, pz, S.vox) ? 0 : -1;
+        int rv;
+        if constexpr (WIDE) rv = bb_gather(P, B.data, px, py, pz, S.vox) ? 0 : -1;
+        else rv = trilinear(P, B.data, P.t32, T, px, py, pz, S.vox);
         WAVE_SYNC();
         if (rv == 0) {
             for (int m = l; m < hr; m += 32) S.msk[m] = S.vox[B.dwi_idx[m]];
             WAVE_SYNC();
-            gemv_lanerow(hr, hr, S.msk, B.R, S.r);
-            gemv_lanerow(hr, hr, S.msk, B.H, S.h);
+            gemv(hr, hr, S.msk, B.R, S.r);
+            gemv(hr, hr, S.msk, B.H, S.h);
             for (int j = l; j < hr; j += 32) {
                 const int src = (int)(rng.next() % (uint32_t)hr);
                 S.h[j] = S.h[j] + S.r[src];
@@ -1045,15 +1076,15 @@ __device__ int get_direction_boot(const DevParams &P, const DevBufs &B, const fl
             // the model's transform of the signal, staged in h (free here)
             for (int j = l; j < hr; j += 32) S.h[j] = gemv_xf<(MODEL == CUSLINES_OPDT) ? 1 : 2>(S.msk[j]);
             WAVE_SYNC();
-            gemv_lanerow(dn, hr, S.h, B.dq, S.r);
+            gemv(dn, hr, S.h, B.dq, S.r);
             if (MODEL == CUSLINES_OPDT) {
-                gemv_lanerow(dn, hr, S.msk, B.db, S.h);
+                gemv(dn, hr, S.msk, B.db, S.h);
                 for (int j = l; j < dn; j += 32) S.r[j] = S.r[j] - S.h[j];
             } else {
                 if (l == 0) S.r[0] = CSA_C0;
             }
             WAVE_SYNC();
-            gemv_lanerow(nv, dn, S.r, B.smat, S.h);
+            gemv(nv, dn, S.r, B.smat, S.h);
         } else {
             for (int j = l; j < nv; j += 32) S.h[j] = 0.0f;
             WAVE_SYNC();
@@ -2697,7 +2728,8 @@ __device__ __forceinline__ int stage_network(const DevBufs &B, float *lds, DevBu
 
 // Phase 2 of one 32-lane slot with the stepping loop flattened (the queue
 // kernel's V == 4: the exact bootstrap getters and spheres too large for the
-// probabilistic getter's own kernel; V == 5: the learned proposal).  In track_seed a slot whose streamline pass, direction
+// probabilistic getter's own kernel; V == 5: the learned proposal; V == 6: the exact bootstrap getters at 2 waves
+// per SIMD).  In track_seed a slot whose streamline pass, direction
 // or seed ends leaves its loops and waits at their exit until the wave's
 // other slot leaves them too; here one iteration of a single loop is one
 // step (PTT: sub-step) of whichever pass the slot holds, and a slot whose
@@ -2711,7 +2743,7 @@ __device__ __forceinline__ int stage_network(const DevBufs &B, float *lds, DevBu
 // length (ints), its seed point and the direction (floats).
 constexpr int FLAT_STATE_FLOATS = 16;
 
-template <int MODEL, bool LEARNED = false>
+template <int MODEL, bool LEARNED = false, bool WIDE = false>
 __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv, SlotLds &S, float *st,
                           const float *__restrict__ seeds, int nseeds, int rng_chunk, const int *__restrict__ offsets,
                           const int *__restrict__ dirs, int *__restrict__ sline_seed, int *__restrict__ sline_len,
@@ -2815,7 +2847,7 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
                     ++nplain;
                 }
             } else
-                nd = get_direction_boot<MODEL>(P, B, sv, S.boot, rng, 5, dx, dy, dz, px, py, pz, &nx, &ny, &nz);
+                nd = get_direction_boot<MODEL, WIDE>(P, B, sv, S.boot, rng, 5, dx, dy, dz, px, py, pz, &nx, &ny, &nz);
             if (nd == 0) {
                 end = true;
             } else {
@@ -3953,9 +3985,9 @@ __global__ void __launch_bounds__(256) phase2_kernel(DevParams P, DevBufs B, con
 // the seeds in processing order; `work` holds QUEUES zeroed counters.  The
 // order changes no result: random streams and output slots follow the seed
 // index.
-// Bootstrap takes 256 VGPRs (2 waves per SIMD): at 128 it spills 140 of them and
-// its products' loads in flight too (CSA 3001 seeds 87 ms at 2, 95 at 3, 99 at
-// 4 waves; 20 000 seeds 217, 228 and 270 ms).  The
+// Bootstrap likewise (4 waves per SIMD, which its 5 KB of LDS per slot allows:
+// +13% CSA), but for small runs (V == 6: 2 waves and 256 VGPRs, the products'
+// loads in flight).  The
 // flat loop of the learned proposal (V == 5) needs about 170 VGPRs and at 128
 // spills inside its loop, so it runs at 3 waves per SIMD (168 VGPRs), in
 // 768-thread workgroups (one staged copy of the network serves 24 slots).
@@ -3965,7 +3997,9 @@ __global__ void __launch_bounds__((MODEL == CUSLINES_PTT && V == 1)   ? 512
                                                                       : 256,
                                   (MODEL == CUSLINES_PTT && V == 5) ? 3
                                   : (MODEL == CUSLINES_PTT && V != 2)           ? 4
-                                                                                : (MODEL <= CUSLINES_CSA ? 2 : MODEL <= CUSLINES_PROB ? 4 : 1))
+                                                                                : (V == 6                       ? 2
+                                                                                 : MODEL <= CUSLINES_PROB ? 4
+                                                                                                          : 1))
     phase2_queue_kernel(DevParams P, DevBufs B, const float *__restrict__ seeds,
                                                            int nseeds, int rng_chunk, const int *__restrict__ offsets,
                                                            const int *__restrict__ dirs, int *__restrict__ sline_seed,
@@ -3986,10 +4020,10 @@ __global__ void __launch_bounds__((MODEL == CUSLINES_PTT && V == 1)   ? 512
     const int l = lane32();
     SlotLds S;
     const int stride =
-        slot_floats(MODEL, false, P.nv32, P.t32, P.hr32) + ((V == 4 || V == 5) ? FLAT_STATE_FLOATS : 0);
+        slot_floats(MODEL, false, P.nv32, P.t32, P.hr32) + ((V >= 4) ? FLAT_STATE_FLOATS : 0);
     bind_slot<MODEL>(P, false, smem + svf + slot * stride, S);
-    if constexpr (V == 4 || V == 5) {
-        flat_slot<MODEL, V == 5>(P, BL, sv, S, smem + svf + slot * stride + stride - FLAT_STATE_FLOATS, seeds,
+    if constexpr (V >= 4) {
+        flat_slot<MODEL, V == 5, V == 6>(P, BL, sv, S, smem + svf + slot * stride + stride - FLAT_STATE_FLOATS, seeds,
                                  nseeds, rng_chunk, offsets, dirs, sline_seed, sline_len, sline, order, work);
         return;
     }
@@ -5646,7 +5680,7 @@ static int launch_phase2_v(cuslines_tracker *t, const float *seeds, int n, int c
     const size_t vf = ((MODEL == CUSLINES_PROB) ? (size_t)((3 * d.nverts + 3) & ~3) : 0) +
                       ((V == 1 || V == 5) ? (size_t)MLP_LDS_FLOATS : 0);
     const size_t lds = sizeof(float) * (vf + (size_t)nslots * (slot_floats(MODEL, false, d.nv32, d.t32, d.hr32) +
-                                                             ((V == 4 || V == 5) ? FLAT_STATE_FLOATS : 0)));
+                                                             ((V >= 4) ? FLAT_STATE_FLOATS : 0)));
     if (lds > 160 * 1024) return fail(CUSLINES_EINVAL, "sphere too large for LDS");
     if (t->schedule == CUSLINES_SCHED_STATIC) {
         HIPC(hipFuncSetAttribute((const void *)phase2_kernel<MODEL, V>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -5815,6 +5849,15 @@ static int launch_phase2(cuslines_tracker *t, const float *seeds, int n, int chu
         }
     }
     if constexpr (MODEL != CUSLINES_PTT) {
+        if constexpr (MODEL != CUSLINES_PROB) {
+            // Up to 8 seeds for each slot of 2 waves per SIMD the run lasts as
+            // long as its longest seeds, whose attempts the registers shorten;
+            // beyond, twice the slots hide more (CSA, ms at 2 | 4 waves: 200
+            // seeds 66 | 80, 3001 83 | 100, 20 000 211 | 256, 32 000 278 | 313,
+            // 40 000 333 | 304, 200 000 1432 | 1069; OPDT 5000 121 | 154).
+            if (t->flat && t->schedule != CUSLINES_SCHED_STATIC && n <= 8 * 16 * t->num_cu)
+                return launch_phase2_v<MODEL, 6>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
+        }
         if (t->flat && t->schedule != CUSLINES_SCHED_STATIC)
             return launch_phase2_v<MODEL, 4>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
     }

@@ -19,3 +19,18 @@ def test_sizes(kind, dirs, order, verts):
     g, o = _run_both(w, _seeds(w, 9))
     assert len(o["sline_len"]) > 0
     _assert_same(g, o)
+
+
+def test_large_run_has_the_small_runs_prefix():
+    """More than 8 seeds a slot (32,768 on 256 CUs) take the variant of 4 waves per SIMD."""
+    import numpy as np
+    from test_gpu_boot_mfma import _track
+
+    w = _workload("csa", 33, 4, 64)
+    seeds = _seeds(w, 33000)
+    full = _track(w, seeds, 0)
+    part = _track(w, seeds[:500], 0)
+    k, pts = len(part["sline_len"]), int(part["point_offsets"][-1])
+    assert k > 0 and np.array_equal(part["counts"], full["counts"][:500])
+    assert np.array_equal(part["sline_len"], full["sline_len"][:k])
+    assert np.array_equal(part["points"], full["points"][:pts])
