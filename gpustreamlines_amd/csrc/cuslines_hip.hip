@@ -4770,7 +4770,8 @@ __device__ __forceinline__ uint32_t spread3(uint32_t v) {  // bits 0..9 to every
     return v;
 }
 
-// Class of a seed with n directions: the more, the earlier.
+// Class of a seed with n directions: the more, the earlier.  Without offsets
+// every seed is in the first class: the order is then the spatial one alone.
 __device__ __forceinline__ int seed_class(int n) {
     if (n >= 8) return 0;
     return (n >= 6) ? 1 : (n >= 1) ? 7 - n : SEED_CLASSES - 1;
@@ -4787,7 +4788,7 @@ __global__ void seed_keys(DevParams P, const float *__restrict__ seeds, const in
         const int i = (f != f || f < 0.0f) ? 0 : (f > (float)(dims[a] - 1) ? dims[a] - 1 : (int)f);
         c[a] = (uint32_t)i >> brick_log2;
     }
-    const int k = seed_class(offsets[s + 1] - offsets[s]) * nbrick +
+    const int k = (offsets ? seed_class(offsets[s + 1] - offsets[s]) : 0) * nbrick +
                   (int)(spread3(c[0]) | (spread3(c[1]) << 1) | (spread3(c[2]) << 2));
     key[s] = k;
     atomicAdd(count + k, 1);
@@ -5618,7 +5619,7 @@ static size_t order_ws_ints(int n, int nb) {
 
 // Seeds by class and, in a class, in Morton order of their brick, by a counting
 // sort on the tracker's stream; the queue's counters and class starts in
-// t->d_work.  With `ws` (order_ws_ints(n, nb) ints of device memory) every
+// t->d_work.  Without offsets the seeds are one class.  With `ws` (order_ws_ints(n, nb) ints of device memory) every
 // buffer is carved from it and *order points into it; without, they are
 // stream-ordered allocations and the caller frees *order with hipFreeAsync.
 static int spatial_order(cuslines_tracker *t, const float *seeds, const int *offsets, int n, int **order, int *ws) {
@@ -5702,7 +5703,10 @@ static int launch_phase2_v(cuslines_tracker *t, const float *seeds, int n, int c
     if (grid > need) grid = need;
     if (grid < 1) grid = 1;
     int *order = nullptr;
-    if (int rc = spatial_order(t, seeds, offsets, n, &order, ws)) return rc;
+    // A recording run keeps the spatial order: its pairs are stored as they come
+    // until the buffer is full, and by class a buffer smaller than the run would
+    // hold those of the seeds with the most directions only.
+    if (int rc = spatial_order(t, seeds, V == 2 ? nullptr : offsets, n, &order, ws)) return rc;
     hipLaunchKernelGGL((phase2_queue_kernel<MODEL, V>), dim3((unsigned)grid), dim3(threads), lds, t->stream, d,
                        bufs_of(t), seeds, n, chunk, offsets, dirs, sseed, slen, sl, order, t->d_work);
     hipError_t e = hipGetLastError();
