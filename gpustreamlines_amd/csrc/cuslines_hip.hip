@@ -5381,11 +5381,9 @@ __global__ void chunk_totals(const int *__restrict__ offsets, int n, int cap, co
 }  // namespace
 
 // Workspace of cuslines_phase2_noalloc_async: the spatial seed order of at
-// most CUSLINES_NOALLOC_MAX_SEEDS seeds (order and keys), its bucket counts
-// and starts (at most 2^21 buckets) and the scan's block sums.  One copy per
+// most CUSLINES_NOALLOC_MAX_SEEDS seeds (order and keys).  One copy per
 // device for the life of the process, shared by every call on that device.
-constexpr size_t SCRATCH_INTS = 2 * (size_t)CUSLINES_NOALLOC_MAX_SEEDS + 2 * ((size_t)1 << 21) + 1 + 2048;
-constexpr size_t SCRATCH_BYTES = SCRATCH_INTS * sizeof(int);
+constexpr size_t SCRATCH_INTS = 2 * (size_t)CUSLINES_NOALLOC_MAX_SEEDS;
 static __device__ __align__(256) int scratch[SCRATCH_INTS];
 
 // =========================================================================
@@ -5430,6 +5428,7 @@ struct cuslines_tracker {
     uint32_t *d_lut = nullptr;
     std::vector<uint16_t> rank_vertex;  // PTT: vertex of each direction rank (corner-block order)
     int *d_work = nullptr;      // work-queue counters and class starts of the persistent phase-2 kernels (WORK_INTS)
+    int *d_sort = nullptr;      // seed order: bucket counts, starts and block sums (sort_ints)
     void *scratch = nullptr;    // device address of this device's `scratch` array
     float *d_blocks = nullptr;  // PTT corner blocks
     int use_blocks = 1;
@@ -5611,37 +5610,37 @@ static int order_buckets(const DevParams &d, int *brick_log2_out) {
     return SEED_CLASSES << (3 * bits);
 }
 
-// ints of the seed-order workspace: order and keys (n each), bucket counts
-// (nb), bucket starts (nb + 1) and the scan's block sums.
-static size_t order_ws_ints(int n, int nb) {
-    return 2 * (size_t)n + 2 * (size_t)nb + 1 + (size_t)((nb + 1023) / 1024);
-}
+// ints of the counting sort's own arrays: bucket counts (nb), bucket starts
+// (nb + 1) and the scan's block sums.  They are the handle's (2 MiB at
+// 81x106x76, 16 MiB at the most), not part of a caller's workspace: their size
+// follows how this library orders seeds, and a workspace that was large
+// enough once stays so.
+static size_t sort_ints(int nb) { return 2 * (size_t)nb + 1 + (size_t)((nb + 1023) / 1024); }
+
+// ints of the seed-order workspace: order and keys.
+static size_t order_ws_ints(int n) { return 2 * (size_t)n; }
 
 // Seeds by class and, in a class, in Morton order of their brick, by a counting
 // sort on the tracker's stream; the queue's counters and class starts in
-// t->d_work.  Without offsets the seeds are one class.  With `ws` (order_ws_ints(n, nb) ints of device memory) every
-// buffer is carved from it and *order points into it; without, they are
-// stream-ordered allocations and the caller frees *order with hipFreeAsync.
+// t->d_work.  Without offsets the seeds are one class.  With `ws`
+// (order_ws_ints(n) ints of device memory) order and keys are carved from it
+// and *order points into it; without, they are stream-ordered allocations and
+// the caller frees *order with hipFreeAsync.
 static int spatial_order(cuslines_tracker *t, const float *seeds, const int *offsets, int n, int **order, int *ws) {
     const DevParams &d = t->dp;
     int brick_log2 = 0;
     const int nb = order_buckets(d, &brick_log2);
-    int *key = nullptr, *count = nullptr, *start = nullptr, *bsum = nullptr;
+    int *count = t->d_sort, *start = count + nb, *bsum = start + nb + 1;
+    int *key = nullptr;
     if (ws) {
         *order = ws;
         key = ws + n;
-        count = key + n;
-        start = count + nb;
-        bsum = start + nb + 1;
     } else {
         *order = nullptr;
         hipError_t e = hipMallocAsync((void **)order, (size_t)n * sizeof(int), t->stream);
         if (e == hipSuccess) e = hipMallocAsync((void **)&key, (size_t)n * sizeof(int), t->stream);
-        if (e == hipSuccess) e = hipMallocAsync((void **)&count, (size_t)nb * sizeof(int), t->stream);
-        if (e == hipSuccess) e = hipMallocAsync((void **)&start, ((size_t)nb + 1) * sizeof(int), t->stream);
         if (e != hipSuccess) {
-            for (int *p : {*order, key, count, start})
-                if (p) (void)hipFreeAsync(p, t->stream);
+            if (*order) (void)hipFreeAsync(*order, t->stream);
             *order = nullptr;
             return fail(CUSLINES_ENOMEM, std::string("seed order: ") + hipGetErrorString(e));
         }
@@ -5657,11 +5656,7 @@ static int spatial_order(cuslines_tracker *t, const float *seeds, const int *off
         hipLaunchKernelGGL(queue_init, dim3(1), dim3(64), 0, t->stream, t->d_work, start, nb / SEED_CLASSES);
     }
     hipError_t e = hipGetLastError();
-    if (!ws) {
-        (void)hipFreeAsync(key, t->stream);
-        (void)hipFreeAsync(count, t->stream);
-        (void)hipFreeAsync(start, t->stream);
-    }
+    if (!ws) (void)hipFreeAsync(key, t->stream);
     if (rc) return rc;
     if (e != hipSuccess) return fail(CUSLINES_EHIP, std::string("seed order: ") + hipGetErrorString(e));
     return CUSLINES_OK;
@@ -5916,9 +5911,8 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Workspace of a bounded chunk: the seed order's (order_ws_ints), then the
 // block sums of the streamline-count scan (int) and of the point scan (int64).
-static size_t chunk_ws_bytes(const DevParams &d, int n, int cap) {
-    int bl = 0;
-    return align256(order_ws_ints(n, order_buckets(d, &bl)) * sizeof(int)) +
+static size_t chunk_ws_bytes(int n, int cap) {
+    return align256(order_ws_ints(n) * sizeof(int)) +
            align256((size_t)((n + 1023) / 1024) * sizeof(int)) + (size_t)((cap + 1023) / 1024) * sizeof(long long);
 }
 
@@ -5929,9 +5923,8 @@ static size_t chunk_ws_bytes(const DevParams &d, int n, int cap) {
 static int chunk_enqueue(cuslines_tracker *t, const float *seeds, int n, int chunk, int *counts, int *dirs,
                          int *offsets, int cap, int *sseed, int *slen, float *sl, long long *poff, float *pts,
                          long long *totals, char *ws) {
-    int bl = 0;
     int *order_ws = reinterpret_cast<int *>(ws);
-    char *p = ws + align256(order_ws_ints(n, order_buckets(t->dp, &bl)) * sizeof(int));
+    char *p = ws + align256(order_ws_ints(n) * sizeof(int));
     int *scan_ws = reinterpret_cast<int *>(p);
     long long *pscan_ws = reinterpret_cast<long long *>(p + align256((size_t)((n + 1023) / 1024) * sizeof(int)));
     if (n > 0)
@@ -5978,7 +5971,7 @@ static int chunk_check(cuslines_tracker *t, const float *seeds_d, int32_t nseeds
         !sline_d || !point_off_d || !points_d || !totals_d || !ws_d)
         return fail(CUSLINES_EINVAL, "null buffer");
     if (int rc = check_ready(t)) return rc;
-    const size_t need = chunk_ws_bytes(t->dp, nseeds, slot_cap);
+    const size_t need = chunk_ws_bytes(nseeds, slot_cap);
     if (ws_bytes < need)
         return fail(CUSLINES_EINVAL, "workspace of " + std::to_string(ws_bytes) + " bytes, " + std::to_string(need) +
                                          " needed (cuslines_chunk_workspace_bytes)");
@@ -6013,13 +6006,7 @@ static int phase2_entry(cuslines_tracker *t, const float *seeds_d, int32_t nseed
         return fail(CUSLINES_EINVAL, "null buffer");
     int rc = check_ready(t);
     if (rc) return rc;
-    int *ws = nullptr;
-    if (noalloc) {
-        int brick_log2 = 0;
-        if (order_ws_ints(nseeds, order_buckets(t->dp, &brick_log2)) * sizeof(int) > SCRATCH_BYTES)
-            return fail(CUSLINES_EINVAL, "seed-order workspace exceeds the scratch array");
-        ws = static_cast<int *>(t->scratch);
-    }
+    int *ws = noalloc ? static_cast<int *>(t->scratch) : nullptr;
     HIPC(hipSetDevice(t->device));
     const int chunk = rng_chunk > 0 ? rng_chunk : nseeds;
     return phase2_models(t, seeds_d, nseeds, chunk, offsets_d, dirs_d, sline_seed_d, sline_len_d, sline_d, ws);
@@ -6121,6 +6108,14 @@ int cuslines_tracker_create(const cuslines_params *p, int device, cuslines_track
     d.min_support_f = smallest_float_at_least((double)p->probe_quality * PMF_THRESHOLD_P);
     d.ptt_seed_thr_f = smallest_float_at_least(PMF_THRESHOLD_P);
     d.ptt_sub_step = (float)(d.step_d / (double)d.step_frac);
+    int brick_log2 = 0;
+    e = hipMalloc(&t->d_sort, sort_ints(order_buckets(d, &brick_log2)) * sizeof(int));
+    if (e != hipSuccess) {
+        dfree(t->d_work);
+        (void)hipStreamDestroy(t->stream);
+        delete t;
+        return fail(CUSLINES_ENOMEM, std::string("seed order: ") + hipGetErrorString(e));
+    }
     *out = t;
     return CUSLINES_OK;
 }
@@ -6131,9 +6126,10 @@ int cuslines_tracker_destroy(cuslines_tracker *t) {
     if (t->ngraphs) return fail(CUSLINES_ESTATE, "destroy the tracker's chunk graphs first");
     (void)hipSetDevice(t->device);
     if (t->stream) (void)hipStreamSynchronize(t->stream);
-    if (t->parent) {  // a fork owns only its stream and counters
+    if (t->parent) {  // a fork owns only its stream, its queue and its counters
         --t->parent->nforks;
         dfree(t->d_work);
+        dfree(t->d_sort);
         dfree(t->d_stats);
         if (t->stream) (void)hipStreamDestroy(t->stream);
         delete t;
@@ -6143,7 +6139,8 @@ int cuslines_tracker_destroy(cuslines_tracker *t) {
     dfree(t->d_H); dfree(t->d_R); dfree(t->d_db); dfree(t->d_dq); dfree(t->d_smat);
     dfree(t->d_hrm); dfree(t->d_fitm); dfree(t->d_odfm);
     dfree(t->d_ut); dfree(t->d_u); dfree(t->d_invlev);
-    dfree(t->d_b0); dfree(t->d_dwi); dfree(t->d_lut); dfree(t->d_work); dfree(t->d_blocks);
+    dfree(t->d_b0); dfree(t->d_dwi); dfree(t->d_lut); dfree(t->d_work); dfree(t->d_sort);
+    dfree(t->d_blocks);
     dfree(t->d_fprop); dfree(t->d_vprop); dfree(t->d_mlp); dfree(t->d_stats);
     if (t->stream) (void)hipStreamDestroy(t->stream);
     delete t;
@@ -6161,14 +6158,18 @@ int cuslines_tracker_fork(cuslines_tracker *t, cuslines_tracker **out) {
     f->ngraphs = 0;
     f->stream = nullptr;
     f->d_work = nullptr;
+    f->d_sort = nullptr;
     f->d_stats = nullptr;  // learned statistics and tap counts stay with the parent
     f->rec = nullptr;
     f->rec_count = nullptr;
     f->count_taps = 0;
     hipError_t e = hipStreamCreateWithFlags(&f->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&f->d_work, WORK_INTS * sizeof(int));
+    int brick_log2 = 0;
+    if (e == hipSuccess) e = hipMalloc(&f->d_sort, sort_ints(order_buckets(f->dp, &brick_log2)) * sizeof(int));
     if (e != hipSuccess) {
         dfree(f->d_work);
+        dfree(f->d_sort);
         if (f->stream) (void)hipStreamDestroy(f->stream);
         delete f;
         return fail(CUSLINES_EHIP, std::string("tracker fork: ") + hipGetErrorString(e));
@@ -6984,7 +6985,7 @@ int cuslines_compact_async(cuslines_tracker *t, const int32_t *sline_len_d, int3
 int cuslines_chunk_workspace_bytes(cuslines_tracker *t, int32_t nseeds, int32_t slot_cap, size_t *bytes) {
     if (!t || !bytes) return fail(CUSLINES_EINVAL, "null argument");
     if (nseeds < 0 || slot_cap < 1) return fail(CUSLINES_EINVAL, "negative size or slot_cap < 1");
-    *bytes = chunk_ws_bytes(t->dp, nseeds, slot_cap);
+    *bytes = chunk_ws_bytes(nseeds, slot_cap);
     return CUSLINES_OK;
 }
 
