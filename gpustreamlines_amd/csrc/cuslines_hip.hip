@@ -201,7 +201,11 @@ __device__ __forceinline__ uint32_t peak_mark(const uint32_t *marks, int j) {
 }
 
 __device__ int sort_dedup_peaks(const DevParams &P, const float *odf, uint16_t *cand, const float *sv, int n);
+__device__ __noinline__ int bb_tail(int symm, float cos_min_sep, const float *odf, uint16_t *cand, const float *verts,
+                                    int n);
 
+// CALL: the tail out of line.
+template <bool CALL = false>
 __device__ int peak_directions(const DevParams &P, const DevBufs &B, const float *odf, uint32_t *marks,
                                uint16_t *cand, const float *sv) {
     const int l = lane32();
@@ -256,7 +260,7 @@ __device__ int peak_directions(const DevParams &P, const DevBufs &B, const float
             n += __popc(msk);
         }
         WAVE_SYNC();
-        return sort_dedup_peaks(P, odf, cand, sv, n);
+        return CALL ? bb_tail(P.sphere_symm, P.cos_min_sep, odf, cand, sv, n) : sort_dedup_peaks(P, odf, cand, sv, n);
     }
     for (int w = l; w < (nv + 15) >> 4; w += 32) marks[w] = 0u;
     WAVE_SYNC();
@@ -287,7 +291,7 @@ __device__ int peak_directions(const DevParams &P, const DevBufs &B, const float
         n += __popc(msk);
     }
     WAVE_SYNC();
-    return sort_dedup_peaks(P, odf, cand, sv, n);
+    return CALL ? bb_tail(P.sphere_symm, P.cos_min_sep, odf, cand, sv, n) : sort_dedup_peaks(P, odf, cand, sv, n);
 }
 
 // The tail of peak_directions_d (tracking_helpers.cu:182-245) on the n
@@ -752,9 +756,11 @@ __device__ void gemv_lanerow(int N, int M, const float *x, const float *__restri
 // each waits for its matrix's blocks from L2 (some 1200 cycles) rather than for
 // its sums: a step reads 282 KB of matrices.  Here the next block's loads are in
 // flight behind the sums, without a branch per column, and with the 256
-// registers they take; launch_phase2 has the rule and its figures.  Out of line,
-// 3001 seeds are faster still (77 ms), but the kernel has one wave per SIMD left
-// (20 000 seeds: 260 ms); two or three blocks ahead spill (213, 233 ms).
+// registers they take; launch_phase2 has the rule and its figures.  The kernel
+// still spills 80 (CSA) and 92 (OPDT) vector registers around the products.
+// Out of line, 3001 seeds are faster still (77 ms), but the kernel has one wave
+// per SIMD left (20 000 seeds: 260 ms); two or three blocks ahead spill more
+// (20 000 seeds: 213, 233 ms).
 __device__ __forceinline__ void gemv_lanerow_wide(int N, int M, const float *x, const float *__restrict__ mat, float *out) {
     const int l = lane32();
     if ((M & 3) == 0) {
@@ -949,6 +955,18 @@ template <>
 struct SlotRng<CUSLINES_PROB> {
     typedef ProbStream<32> type;
 };
+// The exact bootstrap kernels' registers are full: with PAIR, and with the peak
+// tail inline, the one of 4 waves per SIMD spills 140 (CSA) and 143 (OPDT)
+// vector registers instead of 74 and 76.  100,000 seeds on 81x106x76, ms: CSA
+// 464 -> 418, OPDT 365 -> 335; 25,000 on this variant: 243 -> 230, 299 -> 286.
+template <>
+struct SlotRng<CUSLINES_OPDT> {
+    typedef PhiloxStream<false> type;
+};
+template <>
+struct SlotRng<CUSLINES_CSA> {
+    typedef PhiloxStream<false> type;
+};
 
 // trilinear on 16-byte loads: lane l owns channels 128 c + 4 l .. + 3, a
 // chunk's 8 corner loads in flight (two chunks' 64 registers spill at 4 waves
@@ -1033,7 +1051,7 @@ __device__ int closest_peak(const DevParams &P, const float *sv, float dx, float
 // WIDE: the kernel of 2 waves per SIMD.
 template <int MODEL, bool WIDE = false>
 __device__ int get_direction_boot(const DevParams &P, const DevBufs &B, const float *sv, BootLds &S,
-                                  Philox &rng, int nattempts, float dx, float dy, float dz, float px,
+                                  typename SlotRng<MODEL>::type &rng, int nattempts, float dx, float dy, float dz, float px,
                                   float py, float pz, float *ndx, float *ndy, float *ndz) {
     const int l = lane32();
     const auto gemv = [](int N, int M, const float *x, const float *__restrict__ mat, float *out) {
@@ -1096,7 +1114,7 @@ __device__ int get_direction_boot(const DevParams &P, const DevBufs &B, const fl
         for (int j = l; j < nv; j += 32)
             if (S.h[j] < thr) S.h[j] = 0.0f;
         WAVE_SYNC();
-        const int ndir = peak_directions(P, B, S.h, S.marks, S.cand, sv);
+        const int ndir = peak_directions<!WIDE>(P, B, S.h, S.marks, S.cand, sv);
         if (nattempts == 1) return ndir;
         if (ndir > 0 && closest_peak(P, sv, dx, dy, dz, ndir, S.cand, ndx, ndy, ndz)) {
             WAVE_SYNC();

@@ -137,8 +137,11 @@ __device__ __forceinline__ void usincos(float x, float *sn, float *cs) {
 // Philox4x32-10 (Salmon et al., SC'11) with the cuRAND-API stream layout
 // (key = seed; subsequence in counter words z:w; draw k in x:y = k/4, word
 // k%4).  One stream per lane of a seed slot, like the reference's
-// curand_init(RNG_SEED, 32*slot + lane [+1], 0).
-struct Philox {
+// curand_init(RNG_SEED, 32*slot + lane [+1], 0).  PAIR: both halves of a
+// round's products from one quarter-rate 64-bit multiply each; its register
+// pairs are what the exact bootstrap kernels have no room for (SlotRng).
+template <bool PAIR>
+struct PhiloxStream {
     uint32_t k0, k1, s0, s1, c0, c1;
     uint32_t r0, r1, r2, r3;
     int idx;
@@ -150,10 +153,15 @@ struct Philox {
         uint32_t key0 = k0, key1 = k1;
 #pragma unroll
         for (int r = 0; r < 10; ++r) {
-            // one quarter-rate multiply each for both halves of the product
-            const uint64_t m0 = (uint64_t)0xD2511F53u * x0, m1 = (uint64_t)0xCD9E8D57u * x2;
-            const uint32_t lo0 = (uint32_t)m0, hi0 = (uint32_t)(m0 >> 32);
-            const uint32_t lo1 = (uint32_t)m1, hi1 = (uint32_t)(m1 >> 32);
+            uint32_t lo0, hi0, lo1, hi1;
+            if constexpr (PAIR) {
+                const uint64_t m0 = (uint64_t)0xD2511F53u * x0, m1 = (uint64_t)0xCD9E8D57u * x2;
+                lo0 = (uint32_t)m0; hi0 = (uint32_t)(m0 >> 32);
+                lo1 = (uint32_t)m1; hi1 = (uint32_t)(m1 >> 32);
+            } else {
+                lo0 = 0xD2511F53u * x0; hi0 = __umulhi(0xD2511F53u, x0);
+                lo1 = 0xCD9E8D57u * x2; hi1 = __umulhi(0xCD9E8D57u, x2);
+            }
             const uint32_t n0 = hi1 ^ x1 ^ key0, n2 = hi0 ^ x3 ^ key1;
             x0 = n0; x1 = lo1; x2 = n2; x3 = lo0;
             key0 += 0x9E3779B9u;
@@ -193,5 +201,6 @@ struct Philox {
         return sn * s;
     }
 };
+using Philox = PhiloxStream<true>;
 
 }  // namespace cusl
