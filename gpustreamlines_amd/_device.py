@@ -185,12 +185,21 @@ class DeviceTracker:
         """Bootstrap phase-2 kernel: BOOT_EXACT (bit-identical to the CPU
         oracle) or BOOT_MFMA (16 seeds in lockstep, matrix products on the
         matrix cores; equal within float rounding).  waves_per_simd (2 or 4,
-        0 = by the number of seeds) picks the MFMA kernel's occupancy variant;
+        0 = by the number of seeds in flight, ``boot_waves``) picks the
+        kernel's occupancy variant;
         full_products keeps the full [H; R] product where the low-rank form
         (H = U U^T, R its leveraged centred residual matrix) would apply."""
         m = int(mode) | (int(waves_per_simd) << 8) | (self.BOOT_FULL_PRODUCTS if full_products else 0)
         _lib.check(self.L.cuslines_set_boot_mode(self.h, m), "set_boot_mode")
         self.boot_mode = int(mode)
+
+    def boot_waves(self, nseeds: int) -> int:
+        """Waves per SIMD (2 or 4) of the kernel variant that a launch of
+        ``nseeds`` seeds on this handle takes; with live forks each handle
+        counts as having as many in flight."""
+        w = C.c_int32()
+        _lib.check(self.L.cuslines_boot_waves(self.h, int(nseeds), C.byref(w)), "boot_waves")
+        return int(w.value)
 
     def boot_lowrank(self) -> int:
         """Rank of H used by the MFMA kernel's low-rank form (0: full products)."""

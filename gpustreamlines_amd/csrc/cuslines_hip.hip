@@ -5441,7 +5441,7 @@ struct cuslines_tracker {
     int rk16 = 0, hrank = 0;                                      // rank of H and rounded to 16 (0: not that form)
     int boot_full = 0;                                            // batched bootstrap: always the [H; R] product
     int boot_mode = CUSLINES_BOOT_EXACT;
-    int boot_occ = 0;  // batched bootstrap: waves per SIMD of the kernel variant (0: by the number of seeds)
+    int boot_occ = 0;  // bootstrap: waves per SIMD of the kernel variant (0: by the seeds in flight, boot_waves)
     int *d_b0 = nullptr, *d_dwi = nullptr;
     uint32_t *d_lut = nullptr;
     std::vector<uint16_t> rank_vertex;  // PTT: vertex of each direction rank (corner-block order)
@@ -5779,6 +5779,25 @@ static bool boot_batch_fits(const DevParams &d) {
     return d.hr16 <= 320 && d.dn16 <= 128 && d.nv16 <= 768 && d.dn16 <= d.t32;
 }
 
+// Waves per SIMD of the bootstrap kernels' variant for a launch of n seeds:
+// up to 8 seeds in flight for each slot of the 2-waves variant (16 a CU) the
+// run lasts as long as its longest seeds, whose steps the larger register
+// budget shortens; beyond, the other variant's second set of slots hides more.
+// In ms at 2 | 4 waves (81x106x76, 160 directions):
+//   batched CSA: 20 000 seeds 53 | 57, 32 000 80 | 88, 40 000 91 | 81, 60 000 111 | 93
+//   exact CSA: 200 seeds 132 | 160, 3001 158 | 195, 20 000 170 | 206, 32 000 250 | 308, 40 000 281 | 275,
+//   60 000 346 | 308, 200 000 996 | 745; exact OPDT: 20 000 190 | 238, 32 000 265 | 324, 40 000 300 | 355
+// A handle with forks is one of a pipeline's: each of them is taken to have as
+// many seeds in flight.  200,000 CSA seeds as chunks of 25,000 on 8 handles, end
+// to end, by the launch's seeds | by all handles': exact 1,880 | 1,645 ms, batched
+// 1,050 | 1,005 ms (OPDT exact 1,500 | 1,510, batched 782 | 769).
+static int boot_waves(const cuslines_tracker *t, int n) {
+    if (t->boot_occ) return t->boot_occ;
+    const cuslines_tracker *root = t->parent ? t->parent : t;
+    const long long handles = 1 + (long long)__atomic_load_n(&root->nforks, __ATOMIC_RELAXED);
+    return (n * handles <= 8LL * BB_SLOTS * t->num_cu) ? 2 : 4;
+}
+
 template <int MODEL>
 static int launch_boot_batch(cuslines_tracker *t, const float *seeds, int n, int chunk, const int *offsets,
                              const int *dirs, int *sseed, int *slen, float *sl, int *ws) {
@@ -5790,12 +5809,7 @@ static int launch_boot_batch(cuslines_tracker *t, const float *seeds, int n, int
                                         2 * (size_t)BB_WAVES * 16 + BB_SLOTS);
     if (lds > 160 * 1024) return fail(CUSLINES_EINVAL, "batched bootstrap slots too large for LDS");
     const bool lr = d.rk16 > 0;
-    // Up to 8 seeds for each slot of one workgroup per CU, the run lasts as
-    // long as its longest seeds, whose rounds are shorter with 256 registers;
-    // beyond that the two workgroups of the other variant fill each other's
-    // waits (CSA, 160 directions, ms at 2 | 4 waves: 6000 seeds 62 | 68,
-    // 25 000 74 | 80, 60 000 141 | 119, 150 000 327 | 230).
-    const int occ = t->boot_occ ? t->boot_occ : (n <= 8 * BB_SLOTS * t->num_cu) ? 2 : 4;
+    const int occ = boot_waves(t, n);
     const void *kfn = (occ == 4)
                           ? (lr ? (const void *)phase2_boot_batch_kernel<MODEL, 4, true>
                                 : (const void *)phase2_boot_batch_kernel<MODEL, 4, false>)
@@ -5867,12 +5881,7 @@ static int launch_phase2(cuslines_tracker *t, const float *seeds, int n, int chu
     }
     if constexpr (MODEL != CUSLINES_PTT) {
         if constexpr (MODEL != CUSLINES_PROB) {
-            // Up to 8 seeds for each slot of 2 waves per SIMD the run lasts as
-            // long as its longest seeds, whose attempts the registers shorten;
-            // beyond, twice the slots hide more (CSA, ms at 2 | 4 waves: 200
-            // seeds 66 | 80, 3001 83 | 100, 20 000 211 | 256, 32 000 278 | 313,
-            // 40 000 333 | 304, 200 000 1432 | 1069; OPDT 5000 121 | 154).
-            if (t->flat && t->schedule != CUSLINES_SCHED_STATIC && n <= 8 * 16 * t->num_cu)
+            if (t->flat && t->schedule != CUSLINES_SCHED_STATIC && boot_waves(t, n) == 2)
                 return launch_phase2_v<MODEL, 6>(t, seeds, n, chunk, offsets, dirs, sseed, slen, sl, ws);
         }
         if (t->flat && t->schedule != CUSLINES_SCHED_STATIC)
@@ -6145,7 +6154,7 @@ int cuslines_tracker_destroy(cuslines_tracker *t) {
     (void)hipSetDevice(t->device);
     if (t->stream) (void)hipStreamSynchronize(t->stream);
     if (t->parent) {  // a fork owns only its stream, its queue and its counters
-        --t->parent->nforks;
+        __atomic_fetch_sub(&t->parent->nforks, 1, __ATOMIC_RELAXED);
         dfree(t->d_work);
         dfree(t->d_sort);
         dfree(t->d_stats);
@@ -6192,7 +6201,7 @@ int cuslines_tracker_fork(cuslines_tracker *t, cuslines_tracker **out) {
         delete f;
         return fail(CUSLINES_EHIP, std::string("tracker fork: ") + hipGetErrorString(e));
     }
-    ++t->nforks;
+    __atomic_fetch_add(&t->nforks, 1, __ATOMIC_RELAXED);
     *out = f;
     return CUSLINES_OK;
 }
@@ -6669,6 +6678,15 @@ int cuslines_hat_lowrank(const float *H, const float *R, int32_t hr, int32_t *ra
 int cuslines_boot_lowrank(cuslines_tracker *t, int32_t *rank) {
     if (!t || !rank) return fail(CUSLINES_EINVAL, "null argument");
     *rank = (t->has_boot && !t->boot_full) ? t->hrank : 0;
+    return CUSLINES_OK;
+}
+
+int cuslines_boot_waves(cuslines_tracker *t, int32_t nseeds, int32_t *waves) {
+    if (!t || !waves) return fail(CUSLINES_EINVAL, "null argument");
+    if (nseeds < 0) return fail(CUSLINES_EINVAL, "negative size");
+    if (t->p.model_type != CUSLINES_OPDT && t->p.model_type != CUSLINES_CSA)
+        return fail(CUSLINES_EINVAL, "bootstrap variants are for OPDT and CSA trackers");
+    *waves = boot_waves(t, nseeds);
     return CUSLINES_OK;
 }
 

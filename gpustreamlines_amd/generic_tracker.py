@@ -78,7 +78,7 @@ class GenericTracker:
                 from .propagate_seeds import ChunkPipeline
 
                 step = per * gsz
-                pipe = ChunkPipeline(self.device_trackers[0], depth=depth if per == 1 else 2,
+                pipe = ChunkPipeline(self.device_trackers[0], depth=min(depth, nchunks) if per == 1 else 2,
                                      graphs=bool(getattr(self, "chunk_graphs", True)),
                                      rng_chunk=gsz if per > 1 else None)
                 try:

@@ -213,8 +213,9 @@ enum {
  * layout are the same.  MFMA mode needs hr <= 320 DWI volumes, delta_nr <= 128
  * and nverts <= 768 (phase 2 returns CUSLINES_EINVAL otherwise) and the
  * queue schedule (CUSLINES_SCHED_STATIC keeps the exact kernel).  Bits 8..15
- * of `mode` choose the MFMA kernel's occupancy, 2 or 4 waves per SIMD (the
- * autotuner's knob); 0 leaves it to the number of seeds of each launch.
+ * of `mode` choose the occupancy variant of the kernel (MFMA, or exact with
+ * flat stepping), 2 or 4 waves per SIMD, with the same results; 0 leaves it to
+ * the number of seeds in flight (cuslines_boot_waves).
  * When H is a projection H = U U^T of rank r <= 64 and R its leveraged centred
  * residual matrix (boot_utils.py:86-94: R = L (I - H) - column means, L =
  * diag(1 / sqrt(1 - H_ii))), as cuslines_set_boot_matrices checks to 1e-5, the
@@ -228,7 +229,13 @@ int cuslines_set_boot_mode(cuslines_tracker *t, int mode);
  * No counterpart in the reference. */
 int cuslines_boot_lowrank(cuslines_tracker *t, int32_t *rank);
 
-/* The same check on host arrays, without a tracker or a GPU: *rank = r when
+/* The occupancy variant, 2 or 4 waves per SIMD, that a bootstrap launch of
+ * nseeds seeds on this handle takes: as set, or by the seeds in flight, which
+ * are nseeds on each handle of the family (the parent and its live forks).  No
+ * counterpart in the reference. */
+int cuslines_boot_waves(cuslines_tracker *t, int32_t nseeds, int32_t *waves);
+
+/* The low-rank check on host arrays, without a tracker or a GPU: *rank = r when
  * H (hr x hr, row-major) is U U^T of rank r <= 64 < hr and R its leveraged
  * centred residual matrix, to 1e-5; else 0.  No counterpart in the
  * reference. */
