@@ -191,7 +191,7 @@ class DeviceTracker:
         (H = U U^T, R its leveraged centred residual matrix) would apply."""
         m = int(mode) | (int(waves_per_simd) << 8) | (self.BOOT_FULL_PRODUCTS if full_products else 0)
         _lib.check(self.L.cuslines_set_boot_mode(self.h, m), "set_boot_mode")
-        self.boot_mode = int(mode)
+        self.boot_mode, self.boot_full = int(mode), bool(full_products)
 
     def boot_waves(self, nseeds: int) -> int:
         """Waves per SIMD (2 or 4) of the kernel variant that a launch of

@@ -3,7 +3,10 @@
 Every launch shape gives bit-identical streamlines (the random streams are
 keyed by seed and virtual lane, never by hardware slot), so the tuner only
 measures: it runs phase 2 of a seed sample under each candidate shape on the
-tracker's stream, times it with HIP events, and applies the fastest.
+tracker's stream, times it with HIP events, and applies the fastest.  The
+library's own choice is the first candidate and stays unless another shape is
+faster by more than ``MARGIN``: it follows each launch's seeds, a pinned shape
+is that of the sample.
 
 Tuned knobs: schedule (persistent queue or static), threads per block (seed
 slots per workgroup), resident blocks per CU (the occupancy maximum or
@@ -54,7 +57,19 @@ class _Events:
         return float(t.value)
 
 
+MARGIN = 0.05  # a candidate is timed once: runs of one shape differ by a few percent
+
+
+def default(model_type: int, boot_mode: int = 0):
+    """The library's own choice of every knob."""
+    cfg = dict(schedule=0, threads=0, blocks_per_cu=0, lanes=0, flat=True)
+    if model_type in (0, 1) and boot_mode == 1:
+        cfg["waves_per_simd"] = 0
+    return cfg
+
+
 def candidates(model_type: int, boot_mode: int = 0):
+    yield default(model_type, boot_mode)
     if model_type == 3:  # PTT
         for lanes, threads in itertools.product((0, 16, 8), (256, 128)):
             yield dict(schedule=0, threads=threads, blocks_per_cu=0, lanes=lanes, flat=True)
@@ -66,7 +81,7 @@ def candidates(model_type: int, boot_mode: int = 0):
             yield dict(schedule=0, threads=0, blocks_per_cu=bpc, lanes=0, waves_per_simd=occ, flat=True)
     else:
         threads = (128, 64) if model_type in (0, 1) else (256, 128, 64)
-        for t in threads:
+        for t in threads[model_type in (0, 1):]:  # 128 threads are the bootstrap kernels' default
             yield dict(schedule=0, threads=t, blocks_per_cu=0, lanes=0, flat=True)
         yield dict(schedule=0, threads=threads[0], blocks_per_cu=2, lanes=0, flat=True)
         yield dict(schedule=0, threads=threads[0], blocks_per_cu=0, lanes=0, flat=False)
@@ -79,12 +94,21 @@ def apply(dt, cfg):
     if dt.params["model_type"] == 3:
         dt.set_lanes_per_seed(cfg["lanes"])
     if "waves_per_simd" in cfg:
-        dt.set_boot_mode(dt.BOOT_MFMA, cfg["waves_per_simd"])
+        dt.set_boot_mode(dt.BOOT_MFMA, cfg["waves_per_simd"], getattr(dt, "boot_full", False))
 
 
-def tune(dt, seeds: np.ndarray, rng_chunk: int = 0, verbose: bool = False):
+def pick(times: dict, first):
+    """The fastest configuration of ``times``; ``first`` when it is within MARGIN of it."""
+    best = min(times, key=times.get)
+    return first if times[first] <= times[best] * (1 + MARGIN) else best
+
+
+def tune(dt, seeds: np.ndarray, rng_chunk: int = 0, verbose: bool = False, run_seeds: int = 0):
     """Time phase 2 of ``seeds`` under each candidate shape on device tracker
-    ``dt``; apply and return the fastest ``(config, {config: ms})``."""
+    ``dt``; apply and return the chosen ``(config, {config: ms})``.
+    ``run_seeds``: seeds in flight in the runs to tune for, when ``seeds`` is a
+    sample of them: the bootstrap kernel's variant stays the library's choice
+    and is timed as such a run takes it."""
     seeds = np.ascontiguousarray(seeds, dtype=np.float32)
     n = len(seeds)
     nv = dt.params["nverts"]
@@ -106,20 +130,34 @@ def tune(dt, seeds: np.ndarray, rng_chunk: int = 0, verbose: bool = False):
         a, b = ev.pair()
         stream = C.c_void_p(dt.stream())
         times = {}
+        model, mode = dt.params["model_type"], getattr(dt, "boot_mode", 0)
+        boot = model in (0, 1)
+        waves = 0
+        if boot and run_seeds > 0:
+            dt.set_boot_mode(mode, 0, getattr(dt, "boot_full", False))
+            waves = dt.boot_waves(run_seeds)
         try:
-            for cfg in candidates(dt.params["model_type"], getattr(dt, "boot_mode", 0)):
+            for k, cfg in enumerate([default(model, mode), *candidates(model, mode)]):
+                if run_seeds > 0 and cfg.get("waves_per_simd"):
+                    continue
                 apply(dt, cfg)
+                if boot and not cfg.get("waves_per_simd"):
+                    dt.set_boot_mode(mode, waves, getattr(dt, "boot_full", False))
                 ev.hip.hipEventRecord(a, stream)
                 dt.phase2_async(sd.ptr, n, rng_chunk, od.ptr, dd.ptr, ssd.ptr, sld.ptr, sl.ptr)
                 ev.hip.hipEventRecord(b, stream)
                 dt.synchronize()
+                if k == 0:
+                    continue  # the first run of a process is slower than its repeats
                 key = tuple(sorted(cfg.items()))
                 times[key] = ev.ms(a, b)
                 if verbose:
                     print(f"[autotune] {cfg} {times[key]:.1f} ms", flush=True)
         finally:
             ev.destroy(a, b)
-        best = dict(min(times, key=times.get))
+            if boot:
+                dt.set_boot_mode(mode, 0, getattr(dt, "boot_full", False))
+        best = dict(pick(times, tuple(sorted(default(model, mode).items()))))
         apply(dt, best)
         return best, times
     finally:
