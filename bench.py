@@ -263,11 +263,12 @@ def measure_end_to_end(args, w, seeds, kernel_steps):
             "same_steps_as_kernel_pass": steps == kernel_steps}
 
 
-def kernel_name(args, lowrank=False):
-    """The phase-2 kernel the plain pass launches (as rocprofv3 names it)."""
+def kernel_name(args, lowrank=False, waves=4):
+    """The phase-2 kernel the plain pass launches (as rocprofv3 names it);
+    ``waves``: the bootstrap variant of that launch (``DeviceTracker.boot_waves``)."""
     if args.getter in ("csa", "opdt") and args.boot_mode == "mfma":
         lr = "true" if lowrank else "false"
-        return f"phase2_boot_batch_kernel<{MODEL_IDS[args.getter]}, {args.boot_occ or 4}, {lr}>"
+        return f"phase2_boot_batch_kernel<{MODEL_IDS[args.getter]}, {args.boot_occ or waves}, {lr}>"
     if args.getter == "ptt" and args.ptt_lanes:
         kind = "phase2_ptt_flat_kernel" if args.stepping == "flat" else "phase2_ptt_queue_kernel"
         return f"{kind}<{args.ptt_lanes}>"
@@ -275,7 +276,7 @@ def kernel_name(args, lowrank=False):
         return "phase2_ptt_kernel"
     if args.stepping == "flat" and args.getter == "prob":
         return "phase2_prob_kernel<3>"  # 724 channels: three register chunks of 256
-    v = 4 if args.stepping == "flat" else 0
+    v = 0 if args.stepping != "flat" else 6 if (args.boot_occ or waves) == 2 else 4
     return f"phase2_queue_kernel<{MODEL_IDS[args.getter]}, {v}>"
 
 
@@ -494,7 +495,7 @@ def main():
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": None,
-            "kernel": kernel_name(args, boot and dt.boot_lowrank() > 0),
+            "kernel": kernel_name(args, boot and dt.boot_lowrank() > 0, dt.boot_waves(n) if boot else 4),
             "alg_bytes_per_step": alg_launch / max(steps_per_pass, 1),
             "alg_bytes_per_launch": alg_launch,
         },
