@@ -2386,7 +2386,7 @@ __device__ void flat_group_ptt(const DevParams &P, const DevBufs &B, const PttCo
                     if (p == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
                     q = G::shfl(q, 0);
                     if (lo + q >= hi) { ++qk; continue; }
-                    const int s = order ? order[lo + q] : lo + q;
+                    const int s = order[lo + q];
                     const int nd = (P.slot_cap > 0 && offsets[s + 1] > P.slot_cap) ? 0 : offsets[s + 1] - offsets[s];
                     WAVE_SYNC();
                     for (int v = p; v < 32; v += L) { S.rk[v] = 0u; S.rc[v] = -1; }
@@ -2800,7 +2800,7 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
                     if (l == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
                     q = shfl32(q, 0);
                     if (lo + q >= hi) { ++qk; continue; }
-                    const int s = order ? order[lo + q] : lo + q;
+                    const int s = order[lo + q];
                     const int nd = (P.slot_cap > 0 && offsets[s + 1] > P.slot_cap) ? 0 : offsets[s + 1] - offsets[s];
                     rng.init(((uint64_t)P.seed_hi << 32) | P.seed_lo,
                              (uint64_t)32 * (uint64_t)(s % rng_chunk) + (MODEL == CUSLINES_PROB ? 0 : l) + 1);
@@ -3999,16 +3999,20 @@ __global__ void __launch_bounds__(256) phase2_kernel(DevParams P, DevBufs B, con
 
 // Persistent work queue: a fixed grid of slots; each 32-lane slot takes the
 // next seed from a counter as soon as its previous seed is done, so seeds of
-// very uneven length keep every slot busy.  `order` (or the identity) lists
-// the seeds in processing order; `work` holds QUEUES zeroed counters.  The
-// order changes no result: random streams and output slots follow the seed
+// very uneven length keep every slot busy.  `order` lists the seeds in
+// processing order and `work` holds WORK_INTS ints, the zeroed counters and
+// where each class starts in that order (queue_range): both as spatial_order
+// left them in the same call, since the class starts fit no other order.  The
+// order changes no streamline: random streams and output slots follow the seed
 // index.
-// Bootstrap likewise (4 waves per SIMD, which its 5 KB of LDS per slot allows:
-// +13% CSA), but for small runs (V == 6: 2 waves and 256 VGPRs, the products'
-// loads in flight).  The
-// flat loop of the learned proposal (V == 5) needs about 170 VGPRs and at 128
-// spills inside its loop, so it runs at 3 waves per SIMD (168 VGPRs), in
-// 768-thread workgroups (one staged copy of the network serves 24 slots).
+// The per-seed nesting of plain PTT and of its tap count is held to 128 VGPRs
+// (4 waves per SIMD): the few spills cost less than the latency hiding gained.
+// The bootstrap getters likewise (4 waves per SIMD, which their 5 KB of LDS per
+// slot allow), but for few seeds in flight (V == 6: 2 waves and 256 VGPRs, the
+// products' loads in flight).  The flat loop of the learned proposal (V == 5)
+// needs about 170 VGPRs and at 128 spills inside its loop, so it runs at 3 waves
+// per SIMD (168 VGPRs, 17 spilled), in 768-thread workgroups (one staged copy of
+// the network serves 24 slots).
 template <int MODEL, int V = 0>
 __global__ void __launch_bounds__((MODEL == CUSLINES_PTT && V == 1)   ? 512
                                   : (MODEL == CUSLINES_PTT && V == 5) ? 768
@@ -4056,7 +4060,7 @@ __global__ void __launch_bounds__((MODEL == CUSLINES_PTT && V == 1)   ? 512
             if (l == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
             q = shfl32(q, 0);
             if (lo + q >= hi) break;
-            const int s = order ? order[lo + q] : lo + q;
+            const int s = order[lo + q];
             track_seed<MODEL, V>(P, BL, sv, S, s, seeds, rng_chunk, offsets, dirs, sline_seed, sline_len, sline);
         }
     }
@@ -4469,7 +4473,7 @@ __device__ void bb_next_seed(const DevParams &P, const DevBufs &B, BbSlot &st, P
         if (l == 0 && lo < hi) q = atomicAdd(work + qr.counter, 1);
         q = shfl32(q, 0);
         if (lo + q >= hi) { ++st.qk; continue; }
-        const int s = order ? order[lo + q] : lo + q;
+        const int s = order[lo + q];
         const int nd = (P.slot_cap > 0 && offsets[s + 1] > P.slot_cap) ? 0 : offsets[s + 1] - offsets[s];
         if (nd == 0) continue;
         st.s = s;
