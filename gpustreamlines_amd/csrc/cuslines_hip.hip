@@ -200,21 +200,38 @@ __device__ __forceinline__ uint32_t peak_mark(const uint32_t *marks, int j) {
     return (marks[j >> 4] >> (2 * (j & 15))) & 3u;
 }
 
-__device__ int sort_dedup_peaks(const DevParams &P, const float *odf, uint16_t *cand, const float *sv, int n);
-__device__ __noinline__ int bb_tail(int symm, float cos_min_sep, const float *odf, uint16_t *cand, const float *verts,
-                                    int n);
+// What the peak search reads of the parameters and buffers: few enough to be
+// passed to its out-of-line forms.
+struct SepParams {
+    int sphere_symm;
+    float cos_min_sep;
+};
+struct PeakParams {
+    int nverts, nedges;
+    float rel_peak;
+    SepParams sep;
+    const uint16_t *nbr;
+    const uint32_t *edges;
+};
+
+__device__ __forceinline__ SepParams sep_params(const DevParams &P) { return SepParams{P.sphere_symm, P.cos_min_sep}; }
+__device__ __forceinline__ PeakParams peak_params(const DevParams &P, const DevBufs &B) {
+    return PeakParams{P.nverts, P.nedges, P.rel_peak, sep_params(P), B.nbr, B.edges};
+}
+
+__device__ int sort_dedup_peaks(const SepParams &P, const float *odf, uint16_t *cand, const float *sv, int n);
+__device__ __noinline__ int bb_tail(SepParams P, const float *odf, uint16_t *cand, const float *verts, int n);
 
 // CALL: the tail out of line.
 template <bool CALL = false>
-__device__ int peak_directions(const DevParams &P, const DevBufs &B, const float *odf, uint32_t *marks,
-                               uint16_t *cand, const float *sv) {
+__device__ int peak_directions(const PeakParams &P, const float *odf, uint32_t *marks, uint16_t *cand, const float *sv) {
     const int l = lane32();
     const int nv = P.nverts;
     float mn = REAL_MAX;
     for (int j = l; j < nv; j += 32) mn = (mn < odf[j]) ? mn : odf[j];
     mn = min32(mn);
     mn = (0.0f > mn) ? 0.0f : mn;
-    if (B.nbr) {
+    if (P.nbr) {
         // Vertex-centred form of the edge marks below: a vertex is a peak when
         // some neighbour is strictly smaller and none strictly larger, i.e.
         // when the smallest neighbour is below it and the largest not above
@@ -228,7 +245,7 @@ __device__ int peak_directions(const DevParams &P, const DevBufs &B, const float
             uint4 qs[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                qs[u] = reinterpret_cast<const uint4 *>(B.nbr)[min(j0 + 32 * u, nv - 1)];  // past the end: dropped
+                qs[u] = reinterpret_cast<const uint4 *>(P.nbr)[min(j0 + 32 * u, nv - 1)];  // past the end: dropped
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int j = j0 + 32 * u;
@@ -260,12 +277,12 @@ __device__ int peak_directions(const DevParams &P, const DevBufs &B, const float
             n += __popc(msk);
         }
         WAVE_SYNC();
-        return CALL ? bb_tail(P.sphere_symm, P.cos_min_sep, odf, cand, sv, n) : sort_dedup_peaks(P, odf, cand, sv, n);
+        return CALL ? bb_tail(P.sep, odf, cand, sv, n) : sort_dedup_peaks(P.sep, odf, cand, sv, n);
     }
     for (int w = l; w < (nv + 15) >> 4; w += 32) marks[w] = 0u;
     WAVE_SYNC();
     for (int e = l; e < P.nedges; e += 32) {
-        const uint32_t uv = B.edges[e];
+        const uint32_t uv = P.edges[e];
         const int u = (int)(uv & 0xffffu), v = (int)(uv >> 16);
         const float a = odf[u], b = odf[v];
         if (a < b) {
@@ -291,13 +308,13 @@ __device__ int peak_directions(const DevParams &P, const DevBufs &B, const float
         n += __popc(msk);
     }
     WAVE_SYNC();
-    return CALL ? bb_tail(P.sphere_symm, P.cos_min_sep, odf, cand, sv, n) : sort_dedup_peaks(P, odf, cand, sv, n);
+    return CALL ? bb_tail(P.sep, odf, cand, sv, n) : sort_dedup_peaks(P.sep, odf, cand, sv, n);
 }
 
 // The tail of peak_directions_d (tracking_helpers.cu:182-245) on the n
 // candidates in cand: descending sort when n < 32, then the greedy
 // minimum-separation filter.
-__device__ int sort_dedup_peaks(const DevParams &P, const float *odf, uint16_t *cand, const float *sv, int n) {
+__device__ int sort_dedup_peaks(const SepParams &P, const float *odf, uint16_t *cand, const float *sv, int n) {
     const int l = lane32();
     if (n == 0) return 0;
     if (n <= 32) {
@@ -943,7 +960,7 @@ __device__ int get_direction_prob(const DevParams &P, const DevBufs &B, const fl
     for (int i = l; i < nv; i += 32)
         if (pmf[i] < thr) pmf[i] = 0.0f;
     WAVE_SYNC();
-    return peak_directions(P, B, pmf, S.marks, S.cand, sv);
+    return peak_directions(peak_params(P, B), pmf, S.marks, S.cand, sv);
 }
 
 // The random streams of a slot: the probabilistic getter's one, the others' 32.
@@ -1114,7 +1131,7 @@ __device__ int get_direction_boot(const DevParams &P, const DevBufs &B, const fl
         for (int j = l; j < nv; j += 32)
             if (S.h[j] < thr) S.h[j] = 0.0f;
         WAVE_SYNC();
-        const int ndir = peak_directions<!WIDE>(P, B, S.h, S.marks, S.cand, sv);
+        const int ndir = peak_directions<!WIDE>(peak_params(P, B), S.h, S.marks, S.cand, sv);
         if (nattempts == 1) return ndir;
         if (ndir > 0 && closest_peak(P, sv, dx, dy, dz, ndir, S.cand, ndx, ndy, ndz)) {
             WAVE_SYNC();
@@ -2654,7 +2671,7 @@ __global__ void __launch_bounds__(256) phase1_kernel(DevParams P, DevBufs B, con
             pmf[i] = (v < P.ptt_seed_thr_f) ? 0.0f : v;
         }
         WAVE_SYNC();
-        n = peak_directions(P, B, pmf, S.prob.marks, S.prob.cand, sv);
+        n = peak_directions(peak_params(P, B), pmf, S.prob.marks, S.prob.cand, sv);
         kept = S.prob.cand;
     } else {
         float a, b, c;
@@ -4231,9 +4248,8 @@ __device__ __forceinline__ float bb_xf(float x) {
 // peak_directions with the threshold applied to every value it reads.  A
 // peak is never below thr (its thresholded value would be 0 with no
 // strictly smaller neighbour), so the kept candidates' values, the sort
-// keys, are the raw ODF values.  Needs the adjacency table (B.nbr).
-__device__ int bb_peaks_all(const DevParams &P, const DevBufs &B, const float *odf, float thr, uint16_t *cand,
-                        const float *sv) {
+// keys, are the raw ODF values.  Needs the adjacency table (PeakParams::nbr).
+__device__ int bb_peaks_all(const PeakParams &P, const float *odf, float thr, uint16_t *cand, const float *sv) {
     const int l = lane32();
     const int nv = P.nverts;
     uint32_t pk = 0u;
@@ -4254,7 +4270,7 @@ __device__ int bb_peaks_all(const DevParams &P, const DevBufs &B, const float *o
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int j = min(j0 + 32 * u, nv - 1);  // past the end: re-read a valid row, result dropped
-                qs[u] = reinterpret_cast<const uint4 *>(B.nbr)[j];
+                qs[u] = reinterpret_cast<const uint4 *>(P.nbr)[j];
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -4287,7 +4303,7 @@ __device__ int bb_peaks_all(const DevParams &P, const DevBufs &B, const float *o
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int j = min(j0 + 32 * u, nv - 1);
-                qs[u] = reinterpret_cast<const uint4 *>(B.nbr)[j];
+                qs[u] = reinterpret_cast<const uint4 *>(P.nbr)[j];
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -4327,32 +4343,23 @@ __device__ int bb_peaks_all(const DevParams &P, const DevBufs &B, const float *o
         n += __popc(msk);
     }
     WAVE_SYNC();
-    return sort_dedup_peaks(P, odf, cand, sv, n);
+    return sort_dedup_peaks(P.sep, odf, cand, sv, n);
 }
 
 // bb_peaks_all, or the edge form without an adjacency table (out of line:
 // rare, or a sphere with a vertex of more than 8 neighbours).
-__device__ __noinline__ int bb_peaks_slow(int nv, int nedges, int symm, float cos_min_sep, float rel_peak,
-                                          const uint16_t *nbr, const uint32_t *edges, const float *verts, float *odf,
-                                          float thr, uint32_t *marks, uint16_t *cand) {
-    DevParams P;
-    DevBufs B;
-    P.nverts = nv; P.nedges = nedges; P.sphere_symm = symm; P.cos_min_sep = cos_min_sep; P.rel_peak = rel_peak;
-    B.nbr = nbr; B.edges = edges;
-    if (nbr) return bb_peaks_all(P, B, odf, thr, cand, verts);
-    for (int j = lane32(); j < nv; j += 32)
+__device__ __noinline__ int bb_peaks_slow(PeakParams P, const float *verts, float *odf, float thr, uint32_t *marks,
+                                          uint16_t *cand) {
+    if (P.nbr) return bb_peaks_all(P, odf, thr, cand, verts);
+    for (int j = lane32(); j < P.nverts; j += 32)
         if (odf[j] < thr) odf[j] = 0.0f;
     WAVE_SYNC();
-    return peak_directions(P, B, odf, marks, cand, verts);
+    return peak_directions(P, odf, marks, cand, verts);
 }
 
-// sort_dedup_peaks out of line, for the kernel of 4 waves per SIMD: inlined
-// there it costs 20 spilled vector registers.
-__device__ __noinline__ int bb_tail(int symm, float cos_min_sep, const float *odf, uint16_t *cand, const float *verts,
-                                    int n) {
-    DevParams P;
-    P.sphere_symm = symm;
-    P.cos_min_sep = cos_min_sep;
+// sort_dedup_peaks out of line, for the kernels of 4 waves per SIMD: inlined
+// in the batched one it costs 20 spilled vector registers, in the exact one 30.
+__device__ __noinline__ int bb_tail(SepParams P, const float *odf, uint16_t *cand, const float *verts, int n) {
     return sort_dedup_peaks(P, odf, cand, verts, n);
 }
 
@@ -4729,11 +4736,10 @@ __global__ void __launch_bounds__(BB_THREADS, OCC)
                 const float thr = (float)(PMF_THRESHOLD_P * (double)mx);
                 int npk = ((fast >> slot) & 1u) ? bb_peak_list(nv, S.h, mx, S.marks, S.cand) : -1;
                 if (npk >= 0)
-                    npk = (OCC == 4) ? bb_tail(P.sphere_symm, P.cos_min_sep, S.h, S.cand, B.verts, npk)
-                                     : sort_dedup_peaks(P, S.h, S.cand, B.verts, npk);
+                    npk = (OCC == 4) ? bb_tail(sep_params(P), S.h, S.cand, B.verts, npk)
+                                     : sort_dedup_peaks(sep_params(P), S.h, S.cand, B.verts, npk);
                 else
-                    npk = bb_peaks_slow(nv, P.nedges, P.sphere_symm, P.cos_min_sep, P.rel_peak, B.nbr, B.edges, B.verts,
-                                        S.h, thr, S.marks, S.cand);
+                    npk = bb_peaks_slow(peak_params(P, B), B.verts, S.h, thr, S.marks, S.cand);
                 float nx = 0.0f, ny = 0.0f, nz = 0.0f;
                 const bool ok = npk > 0 && closest_peak(P, B.verts, st.dx, st.dy, st.dz, npk, S.cand, &nx, &ny, &nz);
                 WAVE_SYNC();
@@ -5700,14 +5706,16 @@ static int launch_phase2_v(cuslines_tracker *t, const float *seeds, int n, int c
     const size_t lds = sizeof(float) * (vf + (size_t)nslots * (slot_floats(MODEL, false, d.nv32, d.t32, d.hr32) +
                                                              ((V >= 4) ? FLAT_STATE_FLOATS : 0)));
     if (lds > 160 * 1024) return fail(CUSLINES_EINVAL, "sphere too large for LDS");
-    if (t->schedule == CUSLINES_SCHED_STATIC) {
-        HIPC(hipFuncSetAttribute((const void *)phase2_kernel<MODEL, V>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)lds));
-        const unsigned grid = (unsigned)((n + nslots - 1) / nslots);
-        hipLaunchKernelGGL((phase2_kernel<MODEL, V>), dim3(grid), dim3(threads), lds, t->stream, d, bufs_of(t), seeds,
-                           n, chunk, offsets, dirs, sseed, slen, sl);
-        HIPC(hipGetLastError());
-        return CUSLINES_OK;
+    if constexpr (V < 4) {  // the flat loops are the queue's
+        if (t->schedule == CUSLINES_SCHED_STATIC) {
+            HIPC(hipFuncSetAttribute((const void *)phase2_kernel<MODEL, V>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            const unsigned grid = (unsigned)((n + nslots - 1) / nslots);
+            hipLaunchKernelGGL((phase2_kernel<MODEL, V>), dim3(grid), dim3(threads), lds, t->stream, d, bufs_of(t),
+                               seeds, n, chunk, offsets, dirs, sseed, slen, sl);
+            HIPC(hipGetLastError());
+            return CUSLINES_OK;
+        }
     }
     const void *kfn = (const void *)phase2_queue_kernel<MODEL, V>;
     HIPC(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
