@@ -63,7 +63,8 @@ LEARNED_PASSES = 3
 
 
 def measured_traffic(workload: str, kernel: str):
-    """HBM bytes per launch of `kernel` on `workload` from the committed
+    """Bytes per launch of `kernel` on `workload` between L2 and the fabric (HBM and
+    Infinity Cache), from the committed
     rocprofv3 FETCH_SIZE/WRITE_SIZE summaries (profiles/*_traffic.json), or
     None when no summary covers this workload."""
     import glob
@@ -516,7 +517,7 @@ def main():
             res["config"]["proposal"] = "learned"
     traffic = measured_traffic(res["config"]["workload"], res["roofline"]["kernel"])
     if traffic is not None:
-        # the counters as read (FETCH_SIZE + WRITE_SIZE, no calibration factor)
+        # FETCH_SIZE (at the read requests' 128 bytes where they were counted) + WRITE_SIZE
         res["roofline"]["traffic"] = traffic.get("traffic_bytes_unscaled", traffic["traffic_bytes"])
         res["roofline"]["traffic_source"] = traffic["source"]
     for b in (sd, cd, dd, od, ssd, sld, sl):

@@ -769,11 +769,11 @@ __device__ void gemv_lanerow(int N, int M, const float *x, const float *__restri
 }
 
 // The same sums for the kernel of 2 waves per SIMD.  Four of these products are
-// three quarters of an exact attempt's time (170 k cycles for a lone slot), and
+// three quarters of an exact attempt's time (148 k cycles for a lone slot), and
 // each waits for its matrix's blocks from L2 (some 1200 cycles) rather than for
 // its sums: a step reads 282 KB of matrices.  Here the next block's loads are in
 // flight behind the sums, without a branch per column, and with the 256
-// registers they take; launch_phase2 has the rule and its figures.  The kernel
+// registers they take; boot_waves has the rule and its figures.  The kernel
 // still spills 80 (CSA) and 92 (OPDT) vector registers around the products.
 // Out of line, 3001 seeds are faster still (77 ms), but the kernel has one wave
 // per SIMD left (20 000 seeds: 260 ms); two or three blocks ahead spill more
@@ -2979,8 +2979,9 @@ __device__ void flat_slot(const DevParams &P, const DevBufs &B, const float *sv,
 // formed where it is read: the 31 midpoints that the 5 levels of the binary
 // search can visit (one per lane), the last element and the final window.
 //
-// What bounds it: VALU issue (737 instructions a step, 0.5 a cycle and CU at
-// 25,000 seeds) and, for the last seeds, the chain of one step (about 3 us).
+// What bounds it: VALU issue (745 instructions a step; 0.5 a cycle and CU at
+// 25,000 seeds, 0.79 at 250,000) and, for the last seeds, the chain of one step
+// (2.8 us alone).
 // Measured against flat_slot<PROB> (81x106x76, 724 vertices, step 1/4 voxel):
 // 64 seeds 9.8 -> 2.6 ms, 25,000 seeds 120 -> 41 ms, 100,000 255 -> 126 ms;
 // fetched from memory at 25,000 seeds: 17 GB for 9.6 M steps.  The same
@@ -3492,11 +3493,14 @@ __global__ void __launch_bounds__(256, PROB_WAVES)
 //    the face scan from row shifts; the frame stays in registers.
 // Same additions, products and draws in the same order: bit-identical.
 //
-// What bounds it: VALU instructions (1,498 a sub-step and slot; data_support's
-// loop took 1,881), a third of them the 24 x 8 frames; a dependent one takes
-// 8.4 cycles, so a lone wave needs about 21,000 cycles a sub-step.  Against
-// flat_slot<PTT>: 40 seeds 193 -> 148 ms, 4,001 361 -> 267 ms, 25,000 760 ->
-// 640 ms, 250,000 4.67 -> 4.39 s.
+// What bounds it: a wave's own chain.  A dependent instruction takes 8.4
+// cycles, and a lone seed 8 us (19,000 cycles) a sub-step.  At 250,000 seeds
+// (1,365 VALU instructions a sub-step, a third of them the 24 x 8 frames;
+// data_support's loop took 1,881) the CUs issue 0.66 a cycle, and reads, 6.5 TB/s
+// of them past L2, are open for 765 cycles: neither issue nor the fabric is at its
+// limit, two waves per SIMD wait.  Against flat_slot<PTT> with the seeds in
+// spatial order: 40 seeds 195 -> 151 ms (runs differ by as much), 4,001 352 ->
+// 255 ms, 25,000 696 -> 480 ms, 250,000 3.95 -> 3.66 s.
 // -------------------------------------------------------------------------
 // 2 waves per SIMD and all of a group's taps in flight: at 3 waves (168
 // registers, 29 spilled) with 3 taps 25,000 seeds take 714 ms instead of 618
@@ -4542,7 +4546,7 @@ __device__ void bb_end_pass(const DevParams &P, const DevBufs &B, BbSlot &st, Ph
 
 // OCC: waves per SIMD the kernel is compiled for (2: 185 VGPRs and one
 // workgroup per CU; 4: 128 VGPRs, 40 spilled, and two workgroups per CU, whose
-// lockstep phases overlap).  launch_boot_batch has the rule and its figures.
+// lockstep phases overlap).  boot_waves has the rule and its figures.
 // LR: the low-rank form of the [H; R] product (P.rk16 > 0), a separate
 // instantiation so that each form's kernel carries only its own registers.
 template <int MODEL, int OCC, bool LR>
