@@ -974,7 +974,7 @@ struct SlotRng<CUSLINES_PROB> {
 };
 // The exact bootstrap kernels' registers are full: with PAIR, and with the peak
 // tail inline, the one of 4 waves per SIMD spills 140 (CSA) and 143 (OPDT)
-// vector registers instead of 74 and 76.  100,000 seeds on 81x106x76, ms: CSA
+// vector registers instead of 76.  100,000 seeds on 81x106x76, ms: CSA
 // 464 -> 418, OPDT 365 -> 335; 25,000 on this variant: 243 -> 230, 299 -> 286.
 template <>
 struct SlotRng<CUSLINES_OPDT> {
